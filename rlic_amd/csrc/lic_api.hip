@@ -555,11 +555,12 @@ int run_on_device(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
   auto* c = reinterpret_cast<rlic::Cell<T>*>(base + off_cells);
   T* tmp = need_tmp ? reinterpret_cast<T*>(base + off_tmp) : nullptr;
   uint4* code_ptr = replay ? reinterpret_cast<uint4*>(base + off_codes) : nullptr;
+  const uint32_t epoch = rlic::next_epoch();
   {
     // the cells and the padded weight copy in one launch
     LaunchTimer timer("lic_pack", stream);
-    RLIC_HIP_TRY(rlic::launch_pack<T>(tex, tsy, tsx, u, usy, usx, v, vsy, vsx, g, c, stream,
-                                      kernel, klen, kpad),
+    RLIC_HIP_TRY(rlic::launch_pack<T>(tex, tsy, tsx, u, usy, usx, v, vsy, vsx, g, c, epoch,
+                                      stream, kernel, klen, kpad),
                  "pack");
   }
   kernel = kpad + pad;
@@ -573,9 +574,9 @@ int run_on_device(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
   auto trace = [&](T* dst, uint4* codes) {
     LaunchTimer timer(pair ? "lic_trace_pair" : "lic_trace", stream);
     return pair ? rlic::launch_trace_pair<T>(c, kernel, klen, g, m, uv_mode, profile, dst, codes,
-                                             stream)
+                                             epoch, stream)
                 : rlic::launch_trace<T>(c, kernel, klen, g, m, uv_mode, profile, dst, codes,
-                                        stream);
+                                        epoch, stream);
   };
   if (iterations == 1 && !stats) {
     RLIC_HIP_TRY(trace(out, nullptr), "trace");

@@ -45,6 +45,7 @@ struct BatchField {
   uint4* codes;         // move record, or nullptr
   FieldGeom g;
   int32_t klen, uv_mode;
+  uint32_t epoch;       // of the packing of `cells` (wide_mark)
   int32_t iterations;   // pack step only (0: copy the texture to out)
   int32_t regions_x, regions;  // set by launch_queue
   int64_t pack_block0;         // set by launch_queue

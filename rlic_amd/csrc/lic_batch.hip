@@ -75,8 +75,10 @@ __global__ __launch_bounds__(256) void lic_pack_batch(const BatchField<T>* field
       f.out[static_cast<int64_t>(i) * f.g.nx + j] = f.tex[i * f.tsy + j * f.tsx];
     return;
   }
-  f.cells[static_cast<int64_t>(gi) * (f.g.nx + 2) + gj] =
-      guarded_cell(f.tex, f.tsy, f.tsx, f.u, f.usy, f.usx, f.v, f.vsy, f.vsx, f.g, gi, gj);
+  store_guarded_cell(
+      f.cells, gi, gj, f.g,
+      guarded_cell(f.tex, f.tsy, f.tsx, f.u, f.usy, f.usx, f.v, f.vsy, f.vsx, f.g, gi, gj),
+      f.epoch);
 }
 
 __global__ void lic_zero_u32(uint32_t* p, int64_t n) {
@@ -96,12 +98,13 @@ __device__ __forceinline__ void batch_trace_pixel(const BatchField<T>& f,
   const uint32_t row0 =
       static_cast<uint32_t>(i0 + 1) * sg.grow + static_cast<uint32_t>(j0 + 1) * cell.unit;
   const CellVal<T> c0 = cell(row0);
+  const bool short_path = !wide_mark(f.cells, f.epoch);
   T acc = macc<FMA>(kernel[kmid], c0.x, T(0));  // src/lib.rs:375-383
   acc = trace_direction<T, FMA, BRANCHLESS, POL, true, REC, BUF>(
-      acc, c0.u, c0.v, row0, cell, kernel, kmid, n_fwd, sg, f.codes, np, p, 0);
+      acc, c0.u, c0.v, row0, cell, kernel, kmid, n_fwd, sg, f.codes, np, p, 0, short_path);
   acc = trace_direction<T, FMA, BRANCHLESS, POL, false, REC, BUF>(
-      acc, c0.u, c0.v, row0, cell, kernel, kmid, n_bwd, sg, f.codes, np, p,
-      chunks_of(n_fwd));
+      acc, c0.u, c0.v, row0, cell, kernel, kmid, n_bwd, sg, f.codes, np, p, chunks_of(n_fwd),
+      short_path);
   dst[p] = acc;
 }
 
@@ -568,6 +571,7 @@ int batch_run(const FieldSpec* specs, int64_t nfields, int profile, hipStream_t 
                     s.y_left, s.y_right};
     f.klen = static_cast<int32_t>(s.kernel_len);
     f.uv_mode = s.uv_mode;
+    f.epoch = next_epoch();
     f.iterations = static_cast<int32_t>(s.iterations);
     ksrc[k] = s.kernel;
     tmp[k] = s.iterations > 1 ? reinterpret_cast<T*>(base + off_tmp[k]) : nullptr;

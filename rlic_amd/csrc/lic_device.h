@@ -91,29 +91,38 @@ __device__ __forceinline__ double buf_load(const __amdgpu_buffer_rsrc_t r, uint3
 
 // The b64/b128 builtins return GCC vector_size vectors of unsigned int;
 // they are bit-cast whole (bit-casting a subscripted lane miscompiles).
+// Structured buffer load of 16 bytes at `offset` of element `index` (an LLVM
+// intrinsic that has no builtin of its own).
+typedef uint32_t Quad __attribute__((ext_vector_type(4)));
+__device__ Quad struct_buffer_load(__amdgpu_buffer_rsrc_t r, int32_t index, int32_t offset,
+                                   int32_t soffset,
+                                   int32_t aux) __asm("llvm.amdgcn.struct.ptr.buffer.load.v4i32");
 __device__ __forceinline__ CellVal<float> buf_load_cell(const __amdgpu_buffer_rsrc_t r,
-                                                        uint32_t off, float*) {
-  const float4 c = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+                                                        uint32_t index, float*) {
+  const float4 c = __builtin_bit_cast(float4, struct_buffer_load(r, index, 0, 0, 0));
   return {c.x, c.y, c.z, c.w};
 }
 __device__ __forceinline__ CellVal<double> buf_load_cell(const __amdgpu_buffer_rsrc_t r,
-                                                         uint32_t off, double*) {
-  const double2 uv =
-      __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-  const double2 xp =
-      __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, off + 16u, 0, 0));
+                                                         uint32_t index, double*) {
+  const double2 uv = __builtin_bit_cast(double2, struct_buffer_load(r, index, 0, 0, 0));
+  const double2 xp = __builtin_bit_cast(double2, struct_buffer_load(r, index, 16, 0, 0));
   return {uv.x, uv.y, xp.x, xp.y};
 }
 
-// Cell gather at `pos`: a byte offset (BUF) or an element index (global).
+// Cell gather at the cell index `pos`.  With BUF the buffer is a structured
+// one (its stride the cell size, its range counted in cells), so the address
+// unit multiplies the index: positions, row steps and jumps are plain cell
+// counts, and a jump is one 2-cycle add instead of a 4-cycle shift-add.
 template <typename T, bool BUF>
 struct CellGather {
   const Cell<T>* base;
   __amdgpu_buffer_rsrc_t rsrc;
   __device__ __forceinline__ CellGather(const Cell<T>* p, int64_t n) : base(p) {
-    if constexpr (BUF) rsrc = make_rsrc(p, static_cast<uint32_t>(n * sizeof(Cell<T>)));
+    if constexpr (BUF)
+      rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<Cell<T>*>(p), (short)sizeof(Cell<T>),
+                                               static_cast<int>(n), kBufferWord3);
   }
-  static constexpr uint32_t unit = BUF ? static_cast<uint32_t>(sizeof(Cell<T>)) : 1u;
+  static constexpr uint32_t unit = 1u;
   __device__ __forceinline__ CellVal<T> operator()(uint32_t pos) const {
     if constexpr (BUF) {
       return buf_load_cell(rsrc, pos, static_cast<T*>(nullptr));
@@ -149,6 +158,15 @@ __device__ __forceinline__ uint32_t lane_copy(uint32_t x) {
   uint32_t r;
   asm("v_mov_b32 %0, %1" : "=v"(r) : "v"(x));
   return r;
+}
+
+// Keeps the computation of x where it is written: without it the compiler
+// moves a group's sums past the group's closing branch, and with them (global
+// loads) a second load of each cell for its texture value, or (masks of the
+// move codes) the registers that hold what they are made from.
+template <typename T>
+__device__ __forceinline__ void keep_in_step(T& x) {
+  asm volatile("" : "+v"(x));
 }
 
 // x with its sign bit xor-ed with `sign` (0 or 0x80000000; for double it
@@ -235,6 +253,165 @@ __device__ __forceinline__ T time_to_next_pixel(T velocity, T frac) {
   return time_to_next_pixel<T, FMA, BRANCHLESS>(velocity, frac, __builtin_signbit(velocity));
 }
 
+// Ranges of the step's short path (fast_group).  A field is "wide" when a
+// velocity component is infinite or nonzero below kMin / above kMax in
+// magnitude; the packing kernels look at every component and mark such a
+// field (wide_mark), whose lines then take the full rule throughout.
+// Within these ranges and with numerators of at least numerator_min (or
+// zero) the products n |w|, the quotient and its remainder are normal
+// numbers or exact, so no scaling is needed.
+template <typename T>
+struct VelocityRange;
+template <>
+struct VelocityRange<float> {
+  static constexpr float kMin = 0x1p-40f, kMax = 0x1p40f;
+};
+template <>
+struct VelocityRange<double> {
+  static constexpr double kMin = 0x1p-300, kMax = 0x1p300;
+};
+
+template <typename T>
+__device__ __forceinline__ bool velocity_wide(T w) {
+  const T a = abs_t(w);
+  return a > VelocityRange<T>::kMax || (a < VelocityRange<T>::kMin && a != T(0));
+}
+
+// The mark of a wide field: the first word of its guarded array's corner
+// cell (0, 0), which no step reaches.  Each packing of a field has its own
+// `epoch`; a packing thread that sees a wide component stores the epoch
+// there, so the word needs no clearing before (a stale word that happens to
+// equal the epoch only costs the short path).
+template <typename T>
+__device__ __forceinline__ bool wide_mark(const Cell<T>* cells, uint32_t epoch) {
+  return *reinterpret_cast<const uint32_t*>(cells) == epoch;
+}
+
+__device__ __forceinline__ float near_tie(float*) { return 0x1p-18f; }
+__device__ __forceinline__ double near_tie(double*) { return 0x1p-40; }
+
+// Key of a numerator n >= 0 that puts zero last: below numerator_key_min
+// for 0 < n < 2^-60 (float), 2^-300 (double).  A double key reads the top
+// word only: fractions, and with them numerators, that start at zero or at
+// least 2^-300 (fraction_usable) stay multiples of 2^-1004, for products of a
+// quotient of at least 2^-600 and a component of at least 2^-300 are.
+__device__ __forceinline__ uint32_t numerator_key(float n) {
+  return __builtin_bit_cast(uint32_t, n) - 1u;
+}
+__device__ __forceinline__ uint32_t numerator_key(double n) {
+  return static_cast<uint32_t>(__builtin_bit_cast(uint64_t, n) >> 32) - 1u;
+}
+__device__ __forceinline__ uint32_t numerator_key_min(float*) { return ((127u - 60u) << 23) - 1u; }
+__device__ __forceinline__ uint32_t numerator_key_min(double*) {
+  return ((1023u - 300u) << 20) - 1u;
+}
+
+// Fractions the short path starts from: in [0, 1], zero or at least 2^-300.
+// It keeps them in [0, 1]: away from ties the step ends before the other
+// axis' edge, and rounding is monotone.
+__device__ __forceinline__ bool fraction_usable(float f) { return f >= 0.0f && f <= 1.0f; }
+__device__ __forceinline__ bool fraction_usable(double f) {
+  return f == 0.0 || (f >= 0x1p-300 && f <= 1.0);
+}
+
+// Lane masks (0 or all ones) in VGPRs, and selections by them: v_bitop3
+// issues in half the cycles of v_cndmask and v_bfi, and written as builtins
+// they are not turned back into compares and selects.
+__device__ __forceinline__ uint32_t sign_mask(float x) {
+  return static_cast<uint32_t>(__builtin_bit_cast(int32_t, x) >> 31);
+}
+__device__ __forceinline__ uint32_t sign_mask(double x) {
+  return static_cast<uint32_t>(static_cast<int32_t>(__builtin_bit_cast(uint64_t, x) >> 32) >> 31);
+}
+template <uint32_t TABLE>
+__device__ __forceinline__ uint32_t bitop3(uint32_t a, uint32_t b, uint32_t c) {
+  return static_cast<uint32_t>(__builtin_amdgcn_bitop3_b32(a, b, c, TABLE));
+}
+// where the mask is set a, else b
+__device__ __forceinline__ uint32_t pick(uint32_t m, uint32_t a, uint32_t b) {
+  return bitop3<0xCA>(m, a, b);
+}
+struct Words {
+  uint32_t lo, hi;
+};
+__device__ __forceinline__ float pick(uint32_t m, float a, float b) {
+  return __builtin_bit_cast(float, pick(m, __builtin_bit_cast(uint32_t, a),
+                                        __builtin_bit_cast(uint32_t, b)));
+}
+__device__ __forceinline__ double pick(uint32_t m, double a, double b) {
+  const Words x = __builtin_bit_cast(Words, a), y = __builtin_bit_cast(Words, b);
+  return __builtin_bit_cast(double, Words{pick(m, x.lo, y.lo), pick(m, x.hi, y.hi)});
+}
+// x where the mask is clear (FLIP: set), else +0
+template <bool FLIP>
+__device__ __forceinline__ uint32_t keep_bits(uint32_t x, uint32_t m) {
+  return bitop3<FLIP ? 0xC0 : 0x30>(x, m, m);
+}
+template <bool FLIP>
+__device__ __forceinline__ float keep_where(float x, uint32_t m) {
+  return __builtin_bit_cast(float, keep_bits<FLIP>(__builtin_bit_cast(uint32_t, x), m));
+}
+template <bool FLIP>
+__device__ __forceinline__ double keep_where(double x, uint32_t m) {
+  const Words w = __builtin_bit_cast(Words, x);
+  return __builtin_bit_cast(double, Words{keep_bits<FLIP>(w.lo, m), keep_bits<FLIP>(w.hi, m)});
+}
+// where m is set the fraction on the edge just crossed (1 where the step was
+// toward lower indices: the mask `neg`, or with FLIP its complement; else 0),
+// else f
+template <bool FLIP>
+__device__ __forceinline__ float pick_edge(uint32_t m, uint32_t neg, float f) {
+  const uint32_t one = 0x3F800000u;
+  const uint32_t edge = bitop3<FLIP ? 0x0C : 0xC0>(neg, one, one);
+  return pick(m, __builtin_bit_cast(float, edge), f);
+}
+template <bool FLIP>
+__device__ __forceinline__ double pick_edge(uint32_t m, uint32_t neg, double f) {
+  const uint32_t one = 0x3FF00000u;
+  const uint32_t edge = bitop3<FLIP ? 0x0C : 0xC0>(neg, one, one);
+  const Words w = __builtin_bit_cast(Words, f);
+  return __builtin_bit_cast(double,
+                            Words{keep_bits<false>(w.lo, m), pick(m, edge, w.hi)});
+}
+// x with its sign bit xor-ed with that of s
+__device__ __forceinline__ float copy_sign_of(float x, float s) {
+  return __builtin_bit_cast(float, bitop3<0x78>(__builtin_bit_cast(uint32_t, x),
+                                                __builtin_bit_cast(uint32_t, s), 0x80000000u));
+}
+__device__ __forceinline__ double copy_sign_of(double x, double s) {
+  const Words a = __builtin_bit_cast(Words, x), b = __builtin_bit_cast(Words, s);
+  return __builtin_bit_cast(double, Words{a.lo, bitop3<0x78>(a.hi, b.hi, 0x80000000u)});
+}
+// word * 16 + the code bits of a step in its two low bits (y axis where `mx`
+// is clear, toward lower indices where `neg` is set, with FLIP clear); the
+// two bits above are left over from the masks.
+template <bool FLIP>
+__device__ __forceinline__ uint32_t push_code(uint32_t word, uint32_t neg, uint32_t mx) {
+  const uint32_t bits = bitop3<FLIP ? 0x1B : 0xB1>(neg, mx, 1u << 28);
+  return __builtin_amdgcn_alignbit(word, bits, 28);
+}
+
+// n / d correctly rounded, for n, d >= 0 within the ranges above and d > 0:
+// the refinement steps of the IEEE division (reciprocal, Newton, quotient,
+// exact remainder, correction: Markstein 1990) without its scaling and
+// special cases.  In float one Newton step and one correction do: every pair
+// of 23-bit mantissas was tried on gfx950 against the remainder test (2^46
+// pairs, none wrong); scaling by powers of two is exact in between.  In
+// double these are the steps of hipcc's own division.
+__device__ __forceinline__ float quotient_rn(float n, float d) {
+  const float y0 = __builtin_amdgcn_rcpf(d);
+  const float y = fma_t(fma_t(-d, y0, 1.0f), y0, y0);
+  const float q = n * y;
+  return fma_t(fma_t(-d, q, n), y, q);
+}
+__device__ __forceinline__ double quotient_rn(double n, double d) {
+  double y = __builtin_amdgcn_rcp(d);
+  y = fma_t(fma_t(-d, y, 1.0), y, y);
+  y = fma_t(fma_t(-d, y, 1.0), y, y);
+  const double q = n * y;
+  return fma_t(fma_t(-d, q, n), y, q);
+}
+
 struct FieldGeom {
   int32_t ny, nx;
   int32_t x_left, x_right, y_left, y_right;  // 1 = periodic, 0 = closed
@@ -293,6 +470,16 @@ __device__ __forceinline__ Cell<T> guarded_cell(const T* __restrict__ tex, int64
     c.pad = T(0);
   }
   return c;
+}
+
+// Stores guarded cell (gi, gj) and marks a wide field (wide_mark); corner
+// (0, 0) itself, the mark's place, is not written.
+template <typename T>
+__device__ __forceinline__ void store_guarded_cell(Cell<T>* __restrict__ cells, int32_t gi,
+                                                   int32_t gj, const FieldGeom& g,
+                                                   const Cell<T>& c, uint32_t epoch) {
+  if (gi != 0 || gj != 0) cells[static_cast<int64_t>(gi) * (g.nx + 2) + gj] = c;
+  if (velocity_wide(c.u) || velocity_wide(c.v)) *reinterpret_cast<uint32_t*>(cells) = epoch;
 }
 
 // Move codes recorded by the tracing pass (4 bits per step, 8 per word), a

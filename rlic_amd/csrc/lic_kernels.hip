@@ -11,6 +11,7 @@
 //   lic_copy2d  strided 2-D copy (iterations == 0)
 //   lic_repack_texture  texture slot refresh when passes are re-traced
 #include <algorithm>
+#include <atomic>
 #include <type_traits>
 
 #include "lic_device.h"
@@ -36,7 +37,7 @@ __global__ __launch_bounds__(256) void lic_pack(const T* __restrict__ tex, int64
                                                 int64_t vsx, FieldGeom g,
                                                 Cell<T>* __restrict__ cells,
                                                 const T* __restrict__ kernel, int32_t klen,
-                                                T* __restrict__ kpad) {
+                                                T* __restrict__ kpad, uint32_t epoch) {
   if (kpad) {
     const int64_t threads = static_cast<int64_t>(gridDim.x) * gridDim.y * 256;
     const int64_t total = int64_t{klen} + 2 * kKernelPad;
@@ -50,8 +51,8 @@ __global__ __launch_bounds__(256) void lic_pack(const T* __restrict__ tex, int64
   const int32_t gj = blockIdx.x * 64 + (threadIdx.x & 63);
   const int32_t gi = blockIdx.y * 4 + (threadIdx.x >> 6);
   if (gi >= g.ny + 2 || gj >= g.nx + 2) return;
-  cells[static_cast<int64_t>(gi) * (g.nx + 2) + gj] =
-      guarded_cell(tex, tsy, tsx, u, usy, usx, v, vsy, vsx, g, gi, gj);
+  store_guarded_cell(cells, gi, gj, g,
+                     guarded_cell(tex, tsy, tsx, u, usy, usx, v, vsy, vsx, g, gi, gj), epoch);
 }
 
 // The texture slot of every cell of the guarded array from the C-order
@@ -84,7 +85,7 @@ template <typename T, bool FMA, bool BRANCHLESS, bool POL, bool REC, bool BUF>
 __global__ __launch_bounds__(256) void lic_trace(const Cell<T>* __restrict__ cells,
                                                  const T* __restrict__ kernel, int32_t klen,
                                                  FieldGeom g, TileMap m, T* __restrict__ out,
-                                                 uint4* __restrict__ codes) {
+                                                 uint4* __restrict__ codes, uint32_t epoch) {
   int32_t ty, tx, py, px;
   tile_of_block(blockIdx.x, m, ty, tx);
   pixel_of_thread(threadIdx.x, m, py, px);
@@ -99,12 +100,13 @@ __global__ __launch_bounds__(256) void lic_trace(const Cell<T>* __restrict__ cel
   const uint32_t row0 =
       static_cast<uint32_t>(i0 + 1) * sg.grow + static_cast<uint32_t>(j0 + 1) * cell.unit;
   const CellVal<T> c0 = cell(row0);
+  const bool short_path = !wide_mark(cells, epoch);
   T acc = macc<FMA>(kernel[kmid], c0.x, T(0));  // src/lib.rs:375-383
   acc = trace_direction<T, FMA, BRANCHLESS, POL, true, REC, BUF>(
-      acc, c0.u, c0.v, row0, cell, kernel, kmid, n_fwd, sg, codes, np, p, 0);
+      acc, c0.u, c0.v, row0, cell, kernel, kmid, n_fwd, sg, codes, np, p, 0, short_path);
   acc = trace_direction<T, FMA, BRANCHLESS, POL, false, REC, BUF>(
-      acc, c0.u, c0.v, row0, cell, kernel, kmid, n_bwd, sg, codes, np, p,
-      chunks_of(n_fwd));
+      acc, c0.u, c0.v, row0, cell, kernel, kmid, n_bwd, sg, codes, np, p, chunks_of(n_fwd),
+      short_path);
   out[static_cast<int64_t>(i0) * g.nx + j0] = acc;
 }
 
@@ -125,7 +127,7 @@ __global__ __launch_bounds__(256) void lic_trace(const Cell<T>* __restrict__ cel
 template <typename T, bool FMA, bool BRANCHLESS, bool POL, bool REC>
 __global__ __launch_bounds__(64) void lic_trace_pair(
     const Cell<T>* __restrict__ cells, const T* __restrict__ kernel, int32_t klen, FieldGeom g,
-    TileMap m, T* __restrict__ out, uint4* __restrict__ codes) {
+    TileMap m, T* __restrict__ out, uint4* __restrict__ codes, uint32_t epoch) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int32_t lane = threadIdx.x;
   const bool fwd = lane < 32;
@@ -154,13 +156,10 @@ __global__ __launch_bounds__(64) void lic_trace_pair(
     acc = macc<FMA>(kernel[kmid], c0.x, T(0));  // src/lib.rs:375-383
     // every lane stores (no branch in the step): forward lanes into the
     // spare row kmid
-    auto keep = [&](int32_t s, T x, bool live) {
-      vals[32 * (fwd ? kmid : s)] = x;
-      live_steps = live ? s + 1 : live_steps;
-    };
+    auto keep = [&](int32_t s, T x) { vals[32 * (fwd ? kmid : s)] = x; };
     acc = trace_direction<T, FMA, BRANCHLESS, POL, true, REC, true, true>(
         acc, c0.u, c0.v, row0, cell, kernel, kmid, kmid, sg, codes, np, p,
-        fwd ? 0 : chunks_of(kmid), false, false, fwd, keep);
+        fwd ? 0 : chunks_of(kmid), !wide_mark(cells, epoch), fwd, keep, &live_steps);
   }
   __syncthreads();
   const int32_t nb = __shfl(live_steps, k + 32);  // the backward partner's
@@ -691,8 +690,8 @@ int32_t code_chunks(int32_t klen) {
 template <typename T>
 hipError_t launch_pack(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t usy,
                        int64_t usx, const T* v, int64_t vsy, int64_t vsx, const FieldGeom& g,
-                       Cell<T>* cells, hipStream_t stream, const T* kernel, int32_t klen,
-                       T* kpad) {
+                       Cell<T>* cells, uint32_t epoch, hipStream_t stream, const T* kernel,
+                       int32_t klen, T* kpad) {
   dim3 grid((g.nx + 2 + 63) / 64, (g.ny + 2 + 3) / 4);
   if (kpad) {  // enough threads for the weights of a long kernel on a small image
     const int64_t need = (int64_t{klen} + 2 * kKernelPad + 255) / 256;
@@ -701,12 +700,16 @@ hipError_t launch_pack(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64
                          (need + grid.y - 1) / grid.y, std::max<int64_t>(grid.x, 1024)));
   }
   hipLaunchKernelGGL(lic_pack<T>, grid, dim3(256), 0, stream, tex, tsy, tsx, u, usy, usx, v, vsy,
-                     vsx, g, cells, kernel, klen, kpad);
+                     vsx, g, cells, kernel, klen, kpad, epoch);
   return hipGetLastError();
 }
 
 int32_t kernel_pad() { return kKernelPad; }
 
+uint32_t next_epoch() {
+  static std::atomic<uint32_t> epoch{0};
+  return epoch.fetch_add(1, std::memory_order_relaxed) + 1;
+}
 
 template <typename T>
 hipError_t launch_repack_texture(const T* x, const FieldGeom& g, Cell<T>* cells,
@@ -731,14 +734,14 @@ inline bool fits_buffer(int64_t bytes) { return bytes > 0 && bytes <= 0xFFFFFFFF
 
 template <typename T, bool FMA, bool BL, bool POL, bool REC>
 static hipError_t trace_one(const Cell<T>* cells, const T* kernel, int32_t klen,
-                            const FieldGeom& g, const TileMap& m, T* out, uint4* codes,
+                            const FieldGeom& g, const TileMap& m, T* out, uint4* codes, uint32_t epoch,
                             hipStream_t stream) {
   if (fits_buffer(guarded_cells(g.ny, g.nx) * static_cast<int64_t>(sizeof(Cell<T>)))) {
     hipLaunchKernelGGL((lic_trace<T, FMA, BL, POL, REC, true>), dim3(m.n_tiles), dim3(kBlock),
-                       0, stream, cells, kernel, klen, g, m, out, codes);
+                       0, stream, cells, kernel, klen, g, m, out, codes, epoch);
   } else {
     hipLaunchKernelGGL((lic_trace<T, FMA, BL, POL, REC, false>), dim3(m.n_tiles), dim3(kBlock),
-                       0, stream, cells, kernel, klen, g, m, out, codes);
+                       0, stream, cells, kernel, klen, g, m, out, codes, epoch);
   }
   return hipGetLastError();
 }
@@ -746,30 +749,31 @@ static hipError_t trace_one(const Cell<T>* cells, const T* kernel, int32_t klen,
 template <typename T, bool FMA, bool BL>
 static hipError_t trace_mode(const Cell<T>* cells, const T* kernel, int32_t klen,
                              const FieldGeom& g, const TileMap& m, int uv_mode, T* out,
-                             uint4* codes, hipStream_t stream) {
+                             uint4* codes, uint32_t epoch,
+                            hipStream_t stream) {
   const bool rec = codes != nullptr;
   if (uv_mode == 1) {
-    return rec ? trace_one<T, FMA, BL, true, true>(cells, kernel, klen, g, m, out, codes, stream)
-               : trace_one<T, FMA, BL, true, false>(cells, kernel, klen, g, m, out, codes,
+    return rec ? trace_one<T, FMA, BL, true, true>(cells, kernel, klen, g, m, out, codes, epoch, stream)
+               : trace_one<T, FMA, BL, true, false>(cells, kernel, klen, g, m, out, codes, epoch,
                                                     stream);
   }
-  return rec ? trace_one<T, FMA, BL, false, true>(cells, kernel, klen, g, m, out, codes, stream)
-             : trace_one<T, FMA, BL, false, false>(cells, kernel, klen, g, m, out, codes, stream);
+  return rec ? trace_one<T, FMA, BL, false, true>(cells, kernel, klen, g, m, out, codes, epoch, stream)
+             : trace_one<T, FMA, BL, false, false>(cells, kernel, klen, g, m, out, codes, epoch, stream);
 }
 
 template <typename T>
 hipError_t launch_trace(const Cell<T>* cells, const T* kernel, int32_t klen, const FieldGeom& g,
-                        const TileMap& m, int uv_mode, int profile, T* out, uint4* codes,
-                        hipStream_t stream) {
+                        const TileMap& m, int uv_mode, int profile, T* out, uint4* codes, uint32_t epoch,
+                            hipStream_t stream) {
   switch (profile & 3) {
     case 0:
-      return trace_mode<T, false, false>(cells, kernel, klen, g, m, uv_mode, out, codes, stream);
+      return trace_mode<T, false, false>(cells, kernel, klen, g, m, uv_mode, out, codes, epoch, stream);
     case 1:
-      return trace_mode<T, true, false>(cells, kernel, klen, g, m, uv_mode, out, codes, stream);
+      return trace_mode<T, true, false>(cells, kernel, klen, g, m, uv_mode, out, codes, epoch, stream);
     case 2:
-      return trace_mode<T, false, true>(cells, kernel, klen, g, m, uv_mode, out, codes, stream);
+      return trace_mode<T, false, true>(cells, kernel, klen, g, m, uv_mode, out, codes, epoch, stream);
     default:
-      return trace_mode<T, true, true>(cells, kernel, klen, g, m, uv_mode, out, codes, stream);
+      return trace_mode<T, true, true>(cells, kernel, klen, g, m, uv_mode, out, codes, epoch, stream);
   }
 }
 
@@ -779,31 +783,32 @@ size_t trace_pair_lds_bytes(int32_t klen, size_t elem) {
 
 template <typename T, bool FMA, bool BL, bool POL, bool REC>
 static hipError_t trace_pair_one(const Cell<T>* cells, const T* kernel, int32_t klen,
-                                 const FieldGeom& g, const TileMap& m, T* out, uint4* codes,
-                                 hipStream_t stream) {
+                                 const FieldGeom& g, const TileMap& m, T* out, uint4* codes, uint32_t epoch,
+                            hipStream_t stream) {
   const size_t lds = trace_pair_lds_bytes(klen, sizeof(T));
   auto* fn = &lic_trace_pair<T, FMA, BL, POL, REC>;
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
   hipLaunchKernelGGL(fn, dim3(m.n_tiles * 8), dim3(64), lds, stream, cells, kernel, klen, g, m,
-                     out, codes);
+                     out, codes, epoch);
   return hipGetLastError();
 }
 
 template <typename T, bool FMA, bool BL>
 static hipError_t trace_pair_mode(const Cell<T>* cells, const T* kernel, int32_t klen,
                                   const FieldGeom& g, const TileMap& m, int uv_mode, T* out,
-                                  uint4* codes, hipStream_t stream) {
+                                  uint4* codes, uint32_t epoch,
+                            hipStream_t stream) {
   const bool rec = codes != nullptr;
   if (uv_mode == 1) {
-    return rec ? trace_pair_one<T, FMA, BL, true, true>(cells, kernel, klen, g, m, out, codes,
+    return rec ? trace_pair_one<T, FMA, BL, true, true>(cells, kernel, klen, g, m, out, codes, epoch,
                                                          stream)
-               : trace_pair_one<T, FMA, BL, true, false>(cells, kernel, klen, g, m, out, codes,
+               : trace_pair_one<T, FMA, BL, true, false>(cells, kernel, klen, g, m, out, codes, epoch,
                                                           stream);
   }
-  return rec ? trace_pair_one<T, FMA, BL, false, true>(cells, kernel, klen, g, m, out, codes,
+  return rec ? trace_pair_one<T, FMA, BL, false, true>(cells, kernel, klen, g, m, out, codes, epoch,
                                                         stream)
-             : trace_pair_one<T, FMA, BL, false, false>(cells, kernel, klen, g, m, out, codes,
+             : trace_pair_one<T, FMA, BL, false, false>(cells, kernel, klen, g, m, out, codes, epoch,
                                                          stream);
 }
 
@@ -872,20 +877,21 @@ bool trace_pair_fits(int32_t klen, int64_t ny, int64_t nx) {
 template <typename T>
 hipError_t launch_trace_pair(const Cell<T>* cells, const T* kernel, int32_t klen,
                              const FieldGeom& g, const TileMap& m, int uv_mode, int profile,
-                             T* out, uint4* codes, hipStream_t stream) {
+                             T* out, uint4* codes, uint32_t epoch,
+                             hipStream_t stream) {
   if (!trace_pair_fits<T>(klen, g.ny, g.nx)) return hipErrorInvalidValue;
   switch (profile & 3) {
     case 0:
-      return trace_pair_mode<T, false, false>(cells, kernel, klen, g, m, uv_mode, out, codes,
+      return trace_pair_mode<T, false, false>(cells, kernel, klen, g, m, uv_mode, out, codes, epoch,
                                               stream);
     case 1:
-      return trace_pair_mode<T, true, false>(cells, kernel, klen, g, m, uv_mode, out, codes,
+      return trace_pair_mode<T, true, false>(cells, kernel, klen, g, m, uv_mode, out, codes, epoch,
                                              stream);
     case 2:
-      return trace_pair_mode<T, false, true>(cells, kernel, klen, g, m, uv_mode, out, codes,
+      return trace_pair_mode<T, false, true>(cells, kernel, klen, g, m, uv_mode, out, codes, epoch,
                                              stream);
     default:
-      return trace_pair_mode<T, true, true>(cells, kernel, klen, g, m, uv_mode, out, codes,
+      return trace_pair_mode<T, true, true>(cells, kernel, klen, g, m, uv_mode, out, codes, epoch,
                                             stream);
   }
 }
@@ -1004,19 +1010,21 @@ hipError_t launch_replay_lds_hybrid(const T* x, const T* kernel, int32_t klen, c
 #define RLIC_INSTANTIATE(T)                                                                     \
   template hipError_t launch_pack<T>(const T*, int64_t, int64_t, const T*, int64_t, int64_t,   \
                                      const T*, int64_t, int64_t, const FieldGeom&, Cell<T>*,   \
-                                     hipStream_t, const T*, int32_t, T*);                      \
+                                     uint32_t, hipStream_t, const T*, int32_t, T*);                      \
   template hipError_t launch_repack_texture<T>(const T*, const FieldGeom&, Cell<T>*,           \
                                                hipStream_t);                                    \
   template hipError_t launch_copy2d<T>(const T*, int64_t, int64_t, int32_t, int32_t, T*,       \
                                        hipStream_t);                                           \
   template hipError_t launch_trace<T>(const Cell<T>*, const T*, int32_t, const FieldGeom&,     \
-                                      const TileMap&, int, int, T*, uint4*, hipStream_t);   \
+                                      const TileMap&, int, int, T*, uint4*, uint32_t,        \
+                                      hipStream_t);                                             \
   template hipError_t launch_replay<T>(const T*, const T*, int32_t, const FieldGeom&,          \
                                        const TileMap&, int, T*, const uint4*, hipStream_t);    \
   template bool lds_replay_fits<T>(int32_t);                                                   \
   template bool trace_pair_fits<T>(int32_t, int64_t, int64_t);                               \
   template hipError_t launch_trace_pair<T>(const Cell<T>*, const T*, int32_t, const FieldGeom&, \
-                                           const TileMap&, int, int, T*, uint4*, hipStream_t);  \
+                                           const TileMap&, int, int, T*, uint4*, uint32_t,      \
+                                           hipStream_t);                                        \
   template LdsTile lds_replay_tile<T>(int32_t);                                                \
   template hipError_t launch_replay_lds<T>(const T*, const T*, int32_t, const FieldGeom&, int, \
                                            T*, const uint4*, hipStream_t);                      \

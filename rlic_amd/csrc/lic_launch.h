@@ -22,8 +22,12 @@ int32_t code_chunks(int32_t klen);
 template <typename T>
 hipError_t launch_pack(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t usy,
                        int64_t usx, const T* v, int64_t vsy, int64_t vsx, const FieldGeom& g,
-                       Cell<T>* cells, hipStream_t stream, const T* kernel = nullptr,
-                       int32_t klen = 0, T* kpad = nullptr);
+                       Cell<T>* cells, uint32_t epoch, hipStream_t stream,
+                       const T* kernel = nullptr, int32_t klen = 0, T* kpad = nullptr);
+
+// A value for one packing of a field's cells (wide_mark): the packing and
+// the traces of its cells are given the same.
+uint32_t next_epoch();
 
 // Zeros on each side of the padded kernel-weight copy the streamline
 // kernels read (they load taps in groups of 8 without bounds checks).
@@ -43,7 +47,7 @@ hipError_t launch_copy2d(const T* src, int64_t sy, int64_t sx, int32_t ny, int32
 template <typename T>
 hipError_t launch_trace(const Cell<T>* cells, const T* kernel, int32_t klen, const FieldGeom& g,
                         const TileMap& m, int uv_mode, int profile, T* out, uint4* codes,
-                        hipStream_t stream);
+                        uint32_t epoch, hipStream_t stream);
 
 // Paired trace (both directions of a pixel on two lanes) for fields too
 // small to fill the GPU: trace_pair_fits tells whether it applies (odd
@@ -56,7 +60,7 @@ bool trace_pair_fits(int32_t klen, int64_t ny, int64_t nx);
 template <typename T>
 hipError_t launch_trace_pair(const Cell<T>* cells, const T* kernel, int32_t klen,
                              const FieldGeom& g, const TileMap& m, int uv_mode, int profile,
-                             T* out, uint4* codes, hipStream_t stream);
+                             T* out, uint4* codes, uint32_t epoch, hipStream_t stream);
 
 template <typename T>
 hipError_t launch_replay(const T* x, const T* kernel, int32_t klen, const FieldGeom& g,

@@ -34,6 +34,7 @@ template <typename T>
 struct Resident {
   FieldGeom g{};
   int32_t klen = 0, uv_mode = 0;
+  uint32_t epoch = 0;      // of the packing of `cells` (wide_mark)
   void* block = nullptr;
   size_t bytes = 0;        // budget charge (field_bytes)
   size_t block_bytes = 0;  // allocated: bytes rounded up to a size class

@@ -113,6 +113,7 @@ int Server::admit(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
   r.g = FieldGeom{static_cast<int32_t>(ny), static_cast<int32_t>(nx), xl, xr, yl, yr};
   r.klen = static_cast<int32_t>(klen);
   r.uv_mode = uv_mode;
+  r.epoch = next_epoch();
   r.bytes = bytes;
   r.block_bytes = size_class(bytes);
   if (hipError_t e = take_block(bytes, r.block_bytes, &r.block); e != hipSuccess) {
@@ -142,7 +143,8 @@ int Server::admit(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
     e = hipMemcpyAsync(r.weights, kernel, sizeof(T) * static_cast<size_t>(klen),
                        hipMemcpyDefault, stream_);
   if (e == hipSuccess && n > 0)
-    e = launch_pack<T>(tex, tsy, tsx, u, usy, usx, v, vsy, vsx, r.g, r.cells, stream_);
+    e = launch_pack<T>(tex, tsy, tsx, u, usy, usx, v, vsy, vsx, r.g, r.cells, r.epoch,
+                       stream_);
   if (e != hipSuccess) {
     (void)hipFreeAsync(r.block, stream_);  // not cached: the failed copy may have left it in use
     err = std::string("admitting field: ") + hipGetErrorString(e);
@@ -188,6 +190,7 @@ void Server::plan_dtype(StepWork<T>& w, std::vector<int64_t>& finished) {
     f.g = r.g;
     f.klen = r.klen;
     f.uv_mode = r.uv_mode;
+    f.epoch = r.epoch;
     f.iterations = static_cast<int32_t>(std::min<int64_t>(r.target - r.done, INT32_MAX));
     Segment sg{};
     sg.field = static_cast<int32_t>(w.fields.size());

@@ -31,8 +31,8 @@ __host__ __device__ inline int32_t chunks_of(int32_t nsteps) {
 // accumulator untouched, and a lane with a zero vector keeps its position
 // (src/lib.rs:242-244); steps run in groups of 8 (one code word, one batch
 // of 8 weights) and a wave leaves the loop once all its lines have ended.
-// POL and REC: 0 = off, 1 = on, kRuntime = decided by the wave-uniform
-// arguments pol_on / rec_on (one kernel body for fields of mixed modes).
+// With `short_path` (the field's velocities are not wide, velocity_wide),
+// whole groups of the branchless rule run as fast_group.
 //
 // The cells form a guarded array (guarded_cells: (ny + 2) x (nx + 2)
 // with a ring of guard cells around the image) and `row` is the position.
@@ -45,13 +45,122 @@ __host__ __device__ inline int32_t chunks_of(int32_t nsteps) {
 // LANE_DIR: the direction is the lane's own (forward where fwd_lane), one
 // body for both (the paired trace, lic_trace_pair); FORWARD then names the
 // weights the accumulator takes (the backward lanes' sum is not used).
-// `sink(s, x, live)` sees each step's texture value.
-constexpr int kRuntime = 2;
-
+// `sink(s, x)` sees each step's texture value (possibly more than once: the
+// last call for a step counts), and `*live_steps`, if not null, receives the
+// number of steps taken before the line ended.
 struct NoSink {
   template <typename T>
-  __device__ __forceinline__ void operator()(int32_t, T, bool) const {}
+  __device__ __forceinline__ void operator()(int32_t, T) const {}
 };
+
+// Eight steps of the default step rule on the short path: what trace_direction
+// does in its full group, with the two divisions of a step replaced by one.
+//
+// The full rule divides twice (tx = n_x / |u|, ty = n_y / |v|, with n the
+// remaining fraction of the cell along the axis), compares, and then uses
+// only the smaller quotient.  Here the axis is picked by the sign of
+// e = n_x |v| - n_y |u| (one product and one fused multiply-add), and only the
+// picked quotient is formed.  Besides the division saved, the next cell's
+// address no longer waits for a quotient: the gather is issued first and the
+// division runs while it is in flight.
+//
+// Exactness.  The caller guarantees that every nonzero finite velocity of
+// the field lies within VelocityRange (velocity_wide), so the products
+// neither overflow nor lose bits to underflow.  With |e| > near_tie n_y |u|
+// the two exact quotients differ by more than near_tie / 2 relatively, so
+// their roundings compare as the exact ones do; otherwise (an exact or a near tie, both components zero, a NaN component:
+// every one of them fails the comparison) the lane is reported.  The
+// quotient is quotient_rn's, which needs a numerator that is zero or not tiny
+// (numerator_key_min): smaller ones are reported too.  A chunk in which a moving
+// lane is reported is thrown away and done again by the full rule, so the
+// results are the full rule's bit for bit.  A reported lane may pick a wrong
+// axis until the chunk ends, but a step always leads from an image cell to
+// an image cell or a guard cell and from there to an image cell, so its
+// gathers stay inside the guarded array.
+//
+// Lanes that do not move (line ended, or a zero vector) take part with a
+// zero step; the caller restores their sums and codes.  Returns the lane
+// mask of reported lanes.
+//
+// What bounds it: VALU issue.  On gfx950 a wave instruction occupies its SIMD
+// for 2 cycles (float add, multiply, fma; 32-bit add, subtract, and/or/xor,
+// bitop3, arithmetic shift right) or 4 (compares, v_cndmask, min/max,
+// shift-or, bfi, add with carry, every double operation), 8 for v_rcp_f32 and
+// 16 for v_rcp_f64 (measured with streams of one instruction).  So choices are
+// made with lane masks in VGPRs (sign words and v_bitop3) rather than with
+// compares and v_cndmask.  Trace launches, full rule alone -> with this:
+// 4096^2 float L=129 with the record 2.47 -> 1.94 ms, 16384^2 float
+// polarization L=257 72.2 -> 55.3 ms, 8192^2 double polarization L=257
+// 30.1 -> 26.5 ms, 256^2 double L=65 (paired) 22.6 -> 19.3 us.
+template <typename T, bool FMA, int POL, bool FORWARD, int REC, bool BUF, bool LANE_DIR,
+          typename Sink>
+__device__ __forceinline__ uint64_t fast_group(
+    T& acc, T& fx, T& fy, T& pu, T& pv, T& last_u, T& last_v, uint32_t& row, uint32_t& word,
+    const T (&kw)[8], const CellGather<T, BUF>& cell, uint32_t step_x, uint32_t step_y,
+    uint32_t lane_sign, int32_t s0, Sink& sink) {
+  // masks of the sign of (pu, pv): a backward step's signs are the opposite
+  constexpr bool kFlip = !FORWARD && !LANE_DIR;
+  uint64_t reported = 0;
+  uint32_t low = 0xFFFFFFFFu;  // smallest numerator seen (numerator_key)
+  uint32_t jump[8], jumped = 0;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    if constexpr (POL != 0) {  // src/lib.rs:339-347, unfused dot product
+      const T d1 = pu * last_u;
+      const T d2 = pv * last_v;
+      const T dot = (d1 + d2) + T(0);  // + 0: a sum of -0 does not flip
+      pu = copy_sign_of(pu, dot);
+      pv = copy_sign_of(pv, dot);
+      last_u = pu;
+      last_v = pv;
+    }
+    const T mu = LANE_DIR ? xor_sign(pu, lane_sign) : (FORWARD ? pu : -pu);
+    const T mv = LANE_DIR ? xor_sign(pv, lane_sign) : (FORWARD ? pv : -pv);
+    const uint32_t sx = sign_mask(LANE_DIR ? mu : pu), sy = sign_mask(LANE_DIR ? mv : pv);
+    // the numerators of time_to_next_pixel (branchless rule): with the
+    // sign bit set 0 * (0.5 - f) + f, else 2 * (0.5 - f) + f
+    const T nx = macc<FMA>(T(2), keep_where<kFlip>(T(0.5) - fx, sx), fx);
+    const T ny = macc<FMA>(T(2), keep_where<kFlip>(T(0.5) - fy, sy), fy);
+    const T cy = ny * abs_t(mu);
+    const T e = fma_t(nx, abs_t(mv), -cy);
+    const uint32_t mx = sign_mask(e);  // step along x
+    reported |= __builtin_amdgcn_ballot_w64(!(abs_t(e) > cy * near_tie(static_cast<T*>(nullptr))));
+    // where the picked component is nonzero (or the lane is reported),
+    // pos_x and pos_y of the full rule are the sign tests already made
+    const uint32_t sp = pick(mx, sx, sy);
+    const uint32_t s = pick(mx, step_x, step_y);
+    const uint32_t at = kFlip ? row + sp - (s ^ sp) : row - sp + (s ^ sp);
+    const CellVal<T> cv = cell(at);
+    const T n = pick(mx, nx, ny);
+    const T t = quotient_rn(n, abs_t(pick(mx, mu, mv)));
+    low = min(low, numerator_key(n));
+    const T fy_after_x = macc<FMA>(t, mv, fy);
+    const T fx_after_y = macc<FMA>(t, mu, fx);
+    fx = pick_edge<kFlip>(mx, sp, fx_after_y);
+    fy = pick_edge<kFlip>(~mx, sp, fy_after_x);
+    jump[q] = pad_bits(cv.pad);
+    jumped |= jump[q];
+    row = at + jump[q] * cell.unit;
+    acc = macc<FMA>(kw[q], cv.x, acc);  // src/lib.rs:353-360
+    sink(s0 + q, cv.x);
+    pu = cv.u;
+    pv = cv.v;
+    if constexpr (REC != 0) {
+      word = push_code<kFlip>(word, sp, mx);
+      keep_in_step(word);
+    }
+    keep_in_step(acc);
+  }
+  if constexpr (REC != 0) {
+    word = (word & 0x33333333u) | 0x11111111u * kMoveMoved;
+    if (__builtin_amdgcn_ballot_w64(jumped != 0u) != 0) {  // uniform: some line left the image
+#pragma unroll
+      for (int q = 0; q < 8; ++q) word |= jump[q] != 0u ? kMoveEdge << (28 - 4 * q) : 0u;
+    }
+  }
+  return reported |
+         __builtin_amdgcn_ballot_w64(low < numerator_key_min(static_cast<T*>(nullptr)));
+}
 
 template <typename T, bool FMA, bool BRANCHLESS, int POL, bool FORWARD, int REC, bool BUF,
           bool LANE_DIR = false, typename Sink = NoSink>
@@ -60,11 +169,10 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
                                              const T* __restrict__ kernel, int32_t kmid,
                                              int32_t nsteps, const StepGeom& sg,
                                              uint4* __restrict__ codes, int64_t np, int64_t p,
-                                             int32_t c0, bool pol_on = false,
-                                             bool rec_on = false, bool fwd_lane = true,
-                                             Sink sink = Sink{}) {
-  const bool pol = POL == kRuntime ? pol_on : POL != 0;
-  const bool rec = REC == kRuntime ? rec_on : REC != 0;
+                                             int32_t c0, bool short_path,
+                                             bool fwd_lane = true, Sink sink = Sink{},
+                                             int32_t* live_steps = nullptr) {
+  constexpr bool pol = POL != 0, rec = REC != 0;
   const uint32_t lane_sign = fwd_lane ? 0u : 0x80000000u;  // LANE_DIR: negate on backward lanes
   T fx = T(0.5), fy = T(0.5);      // src/lib.rs:315-318
   T last_u = T(0), last_v = T(0);  // src/lib.rs:320-323
@@ -73,11 +181,85 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
   const uint32_t row_up = lane_copy(sg.grow);  // row step, held in VGPRs across the loop
   const uint32_t row_down = lane_copy(0u - sg.grow);
   const int32_t nchunks = chunks_of(nsteps);
+  // Short path: whole groups of a chunk by fast_group; when a moving lane is
+  // reported, the chunk is done again by the full rule.  Off for the rest of
+  // the direction after a chunk that reports many lanes (a field of ties,
+  // e.g. u = v everywhere) or a second chunk that reports any, so that such
+  // a line costs little more than the full rule alone.  (One saved state per
+  // chunk: saving it for every group cost 2 VALU instructions per step.)
+  bool fast = BRANCHLESS && short_path;
+  int32_t misses = 0;
+  bool live_now = false, moves_now = false;  // set before a chunk of the short path
+  bool status_known = false;
   for (int32_t ch = 0; ch < nchunks; ++ch) {
     uint32_t words[4] = {0u, 0u, 0u, 0u};
     bool any_alive = true;
+    int g0 = 0;
+    if (BRANCHLESS && fast) {  // uniform
+      if (!status_known) {  // lanes that do not move never move again
+        live_now = alive && !__builtin_isunordered(pu, pv);
+        moves_now = live_now && (pu != T(0) || pv != T(0));
+        status_known = true;
+      }
+      const uint64_t m_moves = __builtin_amdgcn_ballot_w64(moves_now);
+      const uint32_t step_x = moves_now ? unit : 0u, step_y = moves_now ? sg.grow : 0u;
+      // fractions outside what fast_group takes (the full rule can leave
+      // some after a tie): this chunk by the full rule
+      const bool usable = __builtin_amdgcn_ballot_w64(moves_now && !(fraction_usable(fx) &&
+                                                                      fraction_usable(fy))) == 0;
+      const int full = usable ? min(4, (nsteps - ch * kChunkSteps) >> 3) : 0;
+      const T acc_0 = acc, fx_0 = fx, fy_0 = fy, pu_0 = pu, pv_0 = pv, lu_0 = last_u,
+              lv_0 = last_v;
+      const uint32_t row_0 = row;
+      uint64_t reported = 0;
 #pragma unroll 1
-    for (int g = 0; g < 4; ++g) {
+      for (; g0 < full; ++g0) {
+        const int32_t s0 = ch * kChunkSteps + 8 * g0;
+        T kw[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+          kw[q] = kernel[FORWARD ? kmid + 1 + s0 + q : kmid - 1 - s0 - q];
+        uint32_t word = 0;
+        reported = fast_group<T, FMA, POL, FORWARD, REC, BUF, LANE_DIR>(
+                       acc, fx, fy, pu, pv, last_u, last_v, row, word, kw, cell, step_x, step_y,
+                       lane_sign, s0, sink) &
+                   m_moves;
+        if (reported != 0) break;  // uniform
+        words[g0] = word;
+      }
+      if (reported == 0) {
+        if (m_moves != __builtin_amdgcn_ballot_w64(true)) {  // uniform
+          // a zero vector stays (code 0) and has added its cell's value at
+          // every step; an ended line adds nothing and records stops
+          acc = live_now ? acc : acc_0;
+          const uint32_t still = live_now ? 0u : 0x11111111u * kMoveStop;
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            words[g] = moves_now ? words[g] : (g < full ? still : 0u);
+        }
+        if (full == 0) {
+          status_known = false;  // the full rule runs next
+        } else {
+          alive = live_now;
+          if (live_steps) *live_steps = live_now ? ch * kChunkSteps + 8 * full : *live_steps;
+          any_alive = __builtin_amdgcn_ballot_w64(alive) != 0;
+        }
+      } else {
+        fast = ++misses < 2 && __popcll(reported) < 8;
+        status_known = false;
+        acc = acc_0;
+        fx = fx_0;
+        fy = fy_0;
+        pu = pu_0;
+        pv = pv_0;
+        last_u = lu_0;
+        last_v = lv_0;
+        row = row_0;
+        g0 = 0;
+      }
+    }
+#pragma unroll 1
+    for (int g = g0; g < 4; ++g) {
       const int32_t s0 = ch * kChunkSteps + 8 * g;
       if (s0 >= nsteps || !any_alive) break;  // uniform
       T kw[8];
@@ -91,7 +273,7 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
         // a NaN component ends the line (src/lib.rs:336-338)
         const bool ordered = !__builtin_isunordered(pu, pv);
         const bool live = alive && ordered;
-        if (POL != 0 && pol) {  // src/lib.rs:339-347, unfused dot product
+        if constexpr (pol) {  // src/lib.rs:339-347, unfused dot product
           const T d1 = pu * last_u;
           const T d2 = pv * last_v;
           const bool flip = d1 + d2 < T(0);
@@ -146,10 +328,11 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
         row = at + jump * unit;
         const T next_acc = macc<FMA>(kw[q], cv.x, acc);  // src/lib.rs:353-360
         acc = live ? next_acc : acc;
-        sink(s0 + q, cv.x, live);
+        sink(s0 + q, cv.x);
+        if (live_steps) *live_steps = live ? s0 + q + 1 : *live_steps;
         pu = cv.u;
         pv = cv.v;
-        if (REC != 0 && rec) {
+        if constexpr (rec) {
           // The code's four bits (moved, edge, y axis, negative direction;
           // the three low bits alone for the stop code) are combined from
           // the step's comparisons as wave lane masks on the scalar unit,
@@ -174,11 +357,11 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
       }
       // a last group of fewer than 8 steps: its first step to the top
       // nibble, "stay" codes after its last
-      if (REC != 0 && rec && nsteps - s0 < 8) word <<= 4 * (8 - (nsteps - s0));
+      if (rec && nsteps - s0 < 8) word <<= 4 * (8 - (nsteps - s0));
       words[g] = word;
       any_alive = __builtin_amdgcn_ballot_w64(alive) != 0;
     }
-    if (REC != 0 && rec) codes[(c0 + ch) * np + p] = make_uint4(words[0], words[1], words[2], words[3]);
+    if (rec) codes[(c0 + ch) * np + p] = make_uint4(words[0], words[1], words[2], words[3]);
     if (!any_alive) break;  // every line of the wave ended
   }
   return acc;
