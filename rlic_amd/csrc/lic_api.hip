@@ -466,10 +466,10 @@ struct ScratchLayout {
 };
 
 template <typename T>
-ScratchLayout scratch_layout(int32_t ny, int32_t nx, int32_t klen, bool need_tmp) {
+ScratchLayout scratch_layout(const rlic::FieldGeom& g, int32_t klen, bool need_tmp) {
   auto up = [](size_t x) { return (x + 255) & ~size_t{255}; };
-  const size_t n = static_cast<size_t>(ny) * static_cast<size_t>(nx);
-  const size_t ncells = static_cast<size_t>(rlic::guarded_cells(ny, nx));
+  const size_t n = static_cast<size_t>(g.ny) * static_cast<size_t>(g.nx);
+  const size_t ncells = static_cast<size_t>(rlic::cell_slots(g));
   ScratchLayout l;
   l.cells = up(sizeof(T) * static_cast<size_t>(klen + 2 * rlic::kernel_pad()));
   l.tmp = l.cells + up(sizeof(rlic::Cell<T>) * ncells);
@@ -492,9 +492,9 @@ struct FixedScratch {
 constexpr int kTracePairMaxPixels = 1 << 17;
 
 template <typename T>
-bool use_trace_pair(int32_t klen, int32_t ny, int32_t nx) {
+bool use_trace_pair(int32_t klen, const rlic::FieldGeom& g) {
   const int64_t max_px = env_int("RLIC_TRACE_PAIR_MAX", kTracePairMaxPixels);
-  return static_cast<int64_t>(ny) * nx <= max_px && rlic::trace_pair_fits<T>(klen, ny, nx);
+  return static_cast<int64_t>(g.ny) * g.nx <= max_px && rlic::trace_pair_fits<T>(klen, g);
 }
 
 // `fixed`: take the call's scratch from that region and allocate nothing
@@ -504,7 +504,7 @@ bool use_trace_pair(int32_t klen, int32_t ny, int32_t nx) {
 template <typename T>
 int run_on_device(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t usy, int64_t usx,
                   const T* v, int64_t vsy, int64_t vsx, int32_t ny, int32_t nx,
-                  const T* kernel, int32_t klen, int uv_mode, const rlic::FieldGeom& g,
+                  const T* kernel, int32_t klen, int uv_mode, const rlic::FieldGeom& field,
                   int64_t iterations, T* out, int profile, hipStream_t stream,
                   const FixedScratch* fixed = nullptr) {
   if (iterations == 0) {
@@ -521,7 +521,21 @@ int run_on_device(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
   const int32_t pad = rlic::kernel_pad();
   const bool stats = !fixed && env_int("RLIC_TRACE_STATS", 0) != 0;
   const bool need_tmp = iterations > 1 || stats;
-  const ScratchLayout lay = scratch_layout<T>(ny, nx, klen, need_tmp);
+  rlic::FieldGeom g = field;
+  rlic::choose_row_order<T>(g);
+  ScratchLayout lay = scratch_layout<T>(g, klen, need_tmp);
+  if (fixed && !g.linear) {
+    // plain rows where their layout fits the region (with the record, or
+    // without) and that of row pairs, with its spare row, does not
+    g.linear = 1;
+    const ScratchLayout plain = scratch_layout<T>(g, klen, need_tmp);
+    const size_t record = need_tmp ? lay.code_bytes : 0;
+    auto only_plain = [&](size_t more) {
+      return plain.codes + more <= fixed->bytes && lay.codes + more > fixed->bytes;
+    };
+    if (only_plain(record) || only_plain(0)) lay = plain;
+    else g.linear = 0;
+  }
   const size_t code_bytes = lay.code_bytes;
   bool replay = need_tmp && env_int("RLIC_REPLAY", 1) != 0;
   if (!fixed && replay && code_bytes > (size_t{256} << 20)) {
@@ -570,7 +584,7 @@ int run_on_device(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
   const rlic::TileMap m = rlic::make_tile_map(ny, nx, env_int("RLIC_TILE_BAND", 64),
                                               env_int("RLIC_WAVE_W_LOG2", 4));
   // one tracing pass into dst, recording the moves into codes (or not)
-  const bool pair = !stats && use_trace_pair<T>(klen, ny, nx);
+  const bool pair = !stats && use_trace_pair<T>(klen, g);
   auto trace = [&](T* dst, uint4* codes) {
     LaunchTimer timer(pair ? "lic_trace_pair" : "lic_trace", stream);
     return pair ? rlic::launch_trace_pair<T>(c, kernel, klen, g, m, uv_mode, profile, dst, codes,
@@ -1084,9 +1098,11 @@ int convolve_noalloc_entry(const T* tex, int64_t tsy, int64_t tsx, const T* u, i
   if (ny == 0 || nx == 0) return RLIC_OK;  // nothing to compute
   if (iterations > 0) {
     // weights, cells and ping-pong buffer must fit; the move record may not
-    const size_t need = scratch_layout<T>(static_cast<int32_t>(ny), static_cast<int32_t>(nx),
-                                          static_cast<int32_t>(klen), iterations > 1)
-                            .codes;
+    // (with plain rows: run_on_device takes them where row pairs do not fit)
+    rlic::FieldGeom plain{static_cast<int32_t>(ny), static_cast<int32_t>(nx), xl, xr, yl, yr};
+    plain.linear = 1;
+    const size_t need =
+        scratch_layout<T>(plain, static_cast<int32_t>(klen), iterations > 1).codes;
     if (need > static_cast<size_t>(RLIC_NOALLOC_SCRATCH_BYTES))
       return set_error(RLIC_ERR_INVALID_ARGUMENT,
                        "an image of %lld x %lld pixels with a kernel of %lld weights needs %zu "

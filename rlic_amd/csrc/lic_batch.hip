@@ -66,8 +66,10 @@ __global__ __launch_bounds__(256) void lic_pack_batch(const BatchField<T>* field
   const BatchField<T>& f = fields[lo];
   const int64_t local = b - f.pack_block0;
   const int32_t bx = (f.g.nx + 2 + 63) / 64;
-  const int32_t gj = static_cast<int32_t>(local % bx) * 64 + (threadIdx.x & 63);
-  const int32_t gi = static_cast<int32_t>(local / bx) * 4 + (threadIdx.x >> 6);
+  int32_t gi, gj;
+  pack_cell_of_thread(threadIdx.x, gi, gj);
+  gi += static_cast<int32_t>(local / bx) * 4;
+  gj += static_cast<int32_t>(local % bx) * 64;
   if (gi >= f.g.ny + 2 || gj >= f.g.nx + 2) return;
   if (f.iterations == 0) {
     const int32_t i = gi - 1, j = gj - 1;
@@ -89,20 +91,19 @@ template <typename T, bool FMA, bool BRANCHLESS, int POL, int REC, bool BUF>
 __device__ __forceinline__ void batch_trace_pixel(const BatchField<T>& f,
                                                   const T* __restrict__ kernel, T* dst,
                                                   int32_t i0, int32_t j0) {
-  const CellGather<T, BUF> cell(f.cells, guarded_cells(f.g.ny, f.g.nx));
-  const StepGeom sg = make_step_geom(f.g, cell.unit);
+  const CellGather<T, BUF> cell(f.cells, cell_slots(f.g));
+  const StepGeom sg = make_step_geom(f.g);
   const int32_t kmid = f.klen / 2;
   const int32_t n_fwd = f.klen - 1 - kmid, n_bwd = kmid;
   const int64_t np = static_cast<int64_t>(f.g.ny) * f.g.nx;
   const int64_t p = static_cast<int64_t>(i0) * f.g.nx + j0;
-  const uint32_t row0 =
-      static_cast<uint32_t>(i0 + 1) * sg.grow + static_cast<uint32_t>(j0 + 1) * cell.unit;
+  const uint32_t row0 = static_cast<uint32_t>(cell_slot(f.g, i0 + 1, j0 + 1));
   const CellVal<T> c0 = cell(row0);
   const bool short_path = !wide_mark(f.cells, f.epoch);
   T acc = macc<FMA>(kernel[kmid], c0.x, T(0));  // src/lib.rs:375-383
-  acc = trace_direction<T, FMA, BRANCHLESS, POL, true, REC, BUF>(
+  acc = trace_direction<T, FMA, BRANCHLESS, POL, true, REC, BUF, true>(
       acc, c0.u, c0.v, row0, cell, kernel, kmid, n_fwd, sg, f.codes, np, p, 0, short_path);
-  acc = trace_direction<T, FMA, BRANCHLESS, POL, false, REC, BUF>(
+  acc = trace_direction<T, FMA, BRANCHLESS, POL, false, REC, BUF, true>(
       acc, c0.u, c0.v, row0, cell, kernel, kmid, n_bwd, sg, f.codes, np, p, chunks_of(n_fwd),
       short_path);
   dst[p] = acc;
@@ -185,7 +186,9 @@ __global__ __launch_bounds__(256) void lic_batch_persistent(const BatchField<T>*
   __shared__ uint32_t delta_s[4][16];
   const int32_t lane = threadIdx.x & 63;
   uint32_t* delta = delta_s[threadIdx.x >> 6];
-  const int32_t py = lane >> 3, px = lane & 7;
+  const int32_t py = lane >> 3, px = lane & 7;  // replays: rows of the 8 x 8 square
+  // traces: quads of lanes on 2 x 2 pixels of it (pixel_of_quads)
+  const int32_t ty = ((lane >> 4) << 1) | ((lane >> 1) & 1), tx = ((lane >> 1) & 6) | (lane & 1);
   // Completed items are published in batches: per-segment counts of up to
   // kPendSlots segments are held by the wave and published together behind
   // one release fence (the fence writes back L2, too costly per item) once
@@ -285,7 +288,8 @@ __global__ __launch_bounds__(256) void lic_batch_persistent(const BatchField<T>*
     const int64_t local = item - seg.item0;
     const int32_t ry = static_cast<int32_t>(local / f.regions_x);
     const int32_t rx = static_cast<int32_t>(local - static_cast<int64_t>(ry) * f.regions_x);
-    const int32_t i_base = (ry << (sq_log2 + 3)) + py, j_base = (rx << (sq_log2 + 3)) + px;
+    const int32_t i_base = (ry << (sq_log2 + 3)) + (seg.pass == 0 ? ty : py);
+    const int32_t j_base = (rx << (sq_log2 + 3)) + (seg.pass == 0 ? tx : px);
     const T* __restrict__ kern = kpool + f.kernel_off;  // uniform: weights via scalar loads
     T* dst = static_cast<T*>(seg.dst);
     if (seg.pass == 0) {
@@ -373,7 +377,7 @@ int launch_queue(std::vector<BatchField<T>>& fields, const std::vector<const T*>
       pack_blocks += static_cast<int64_t>((f.g.nx + 2 + 63) / 64) * ((f.g.ny + 2 + 3) / 4);
     f.kernel_off = pool_len + kKernelPad;
     pool_len += f.klen + 2 * kKernelPad;
-    if (guarded_cells(f.g.ny, f.g.nx) * static_cast<int64_t>(sizeof(Cell<T>)) > 0xFFFFFFFFll)
+    if (cell_slots(f.g) * static_cast<int64_t>(sizeof(Cell<T>)) > 0xFFFFFFFFll)
       buf = false;
   }
   int64_t items = 0;
@@ -535,13 +539,17 @@ int batch_run(const FieldSpec* specs, int64_t nfields, int profile, hipStream_t 
               BatchScratch& scratch, std::string& err) {
   // per-field working memory: cells, ping-pong partner, move record
   std::vector<size_t> off_cells(nfields), off_tmp(nfields), off_codes(nfields);
+  std::vector<FieldGeom> geom(nfields);
   size_t bytes = 0;
   for (int64_t k = 0; k < nfields; ++k) {
     const FieldSpec& s = specs[k];
     const size_t n = static_cast<size_t>(s.ny * s.nx);
+    geom[k] = FieldGeom{static_cast<int32_t>(s.ny), static_cast<int32_t>(s.nx), s.x_left,
+                        s.x_right, s.y_left, s.y_right};
+    choose_row_order<T>(geom[k]);
     off_cells[k] = bytes;
     if (s.iterations > 0)
-      bytes = align_up(bytes + sizeof(Cell<T>) * static_cast<size_t>(guarded_cells(s.ny, s.nx)));
+      bytes = align_up(bytes + sizeof(Cell<T>) * static_cast<size_t>(cell_slots(geom[k])));
     off_tmp[k] = bytes;
     if (s.iterations > 1) bytes = align_up(bytes + sizeof(T) * n);
     off_codes[k] = bytes;
@@ -567,8 +575,7 @@ int batch_run(const FieldSpec* specs, int64_t nfields, int profile, hipStream_t 
     f.out = s.out;
     f.cells = s.iterations > 0 ? reinterpret_cast<Cell<T>*>(base + off_cells[k]) : nullptr;
     f.codes = s.iterations > 1 ? reinterpret_cast<uint4*>(base + off_codes[k]) : nullptr;
-    f.g = FieldGeom{static_cast<int32_t>(s.ny), static_cast<int32_t>(s.nx), s.x_left, s.x_right,
-                    s.y_left, s.y_right};
+    f.g = geom[k];
     f.klen = static_cast<int32_t>(s.kernel_len);
     f.uv_mode = s.uv_mode;
     f.epoch = next_epoch();

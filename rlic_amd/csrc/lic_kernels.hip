@@ -48,8 +48,10 @@ __global__ __launch_bounds__(256) void lic_pack(const T* __restrict__ tex, int64
       kpad[t] = (k >= 0 && k < klen) ? kernel[k] : T(0);
     }
   }
-  const int32_t gj = blockIdx.x * 64 + (threadIdx.x & 63);
-  const int32_t gi = blockIdx.y * 4 + (threadIdx.x >> 6);
+  int32_t gi, gj;
+  pack_cell_of_thread(threadIdx.x, gi, gj);
+  gi += blockIdx.y * 4;
+  gj += blockIdx.x * 64;
   if (gi >= g.ny + 2 || gj >= g.nx + 2) return;
   store_guarded_cell(cells, gi, gj, g,
                      guarded_cell(tex, tsy, tsx, u, usy, usx, v, vsy, vsx, g, gi, gj), epoch);
@@ -60,12 +62,14 @@ __global__ __launch_bounds__(256) void lic_pack(const T* __restrict__ tex, int64
 template <typename T>
 __global__ __launch_bounds__(256) void lic_repack_texture(const T* __restrict__ x, FieldGeom g,
                                                           Cell<T>* __restrict__ cells) {
-  const int32_t gj = blockIdx.x * 64 + (threadIdx.x & 63);
-  const int32_t gi = blockIdx.y * 4 + (threadIdx.x >> 6);
+  int32_t gi, gj;
+  pack_cell_of_thread(threadIdx.x, gi, gj);
+  gi += blockIdx.y * 4;
+  gj += blockIdx.x * 64;
   if (gi >= g.ny + 2 || gj >= g.nx + 2) return;
   int32_t i, j;
   if (guard_source(gi, gj, g.ny, g.nx, g.x_left, g.x_right, g.y_left, g.y_right, i, j))
-    cells[static_cast<int64_t>(gi) * (g.nx + 2) + gj].x = x[static_cast<int64_t>(i) * g.nx + j];
+    cells[cell_slot(g, gi, gj)].x = x[static_cast<int64_t>(i) * g.nx + j];
 }
 
 template <typename T>
@@ -78,9 +82,9 @@ __global__ __launch_bounds__(256) void lic_copy2d(const T* __restrict__ src, int
   dst[static_cast<int64_t>(i) * nx + j] = src[i * sy + j * sx];
 }
 
-// The cells are the field's guarded array (lic_pack); a position is a
-// byte offset into it with BUF (buffer loads, arrays below 4 GiB), else a
-// cell index.
+// The cells are the field's guarded array (lic_pack), a position a slot of it:
+// with BUF (arrays below 4 GiB) read by structured buffer loads, else by
+// global loads from plain rows (choose_row_order).
 template <typename T, bool FMA, bool BRANCHLESS, bool POL, bool REC, bool BUF>
 __global__ __launch_bounds__(256) void lic_trace(const Cell<T>* __restrict__ cells,
                                                  const T* __restrict__ kernel, int32_t klen,
@@ -88,23 +92,23 @@ __global__ __launch_bounds__(256) void lic_trace(const Cell<T>* __restrict__ cel
                                                  uint4* __restrict__ codes, uint32_t epoch) {
   int32_t ty, tx, py, px;
   tile_of_block(blockIdx.x, m, ty, tx);
-  pixel_of_thread(threadIdx.x, m, py, px);
+  if constexpr (BUF) pixel_of_quads(threadIdx.x, m, py, px);
+  else pixel_of_thread(threadIdx.x, m, py, px);  // plain rows
   const int32_t i0 = ty * tile_h(m) + py, j0 = tx * tile_w(m) + px;
   if (i0 >= g.ny || j0 >= g.nx) return;
-  const CellGather<T, BUF> cell(cells, guarded_cells(g.ny, g.nx));
-  const StepGeom sg = make_step_geom(g, cell.unit);
+  const CellGather<T, BUF> cell(cells, cell_slots(g));
+  const StepGeom sg = make_step_geom(g);
   const int32_t kmid = klen / 2;
   const int32_t n_fwd = klen - 1 - kmid, n_bwd = kmid;
   const int64_t np = static_cast<int64_t>(g.ny) * g.nx;  // code slot = pixel index
   const int64_t p = static_cast<int64_t>(i0) * g.nx + j0;
-  const uint32_t row0 =
-      static_cast<uint32_t>(i0 + 1) * sg.grow + static_cast<uint32_t>(j0 + 1) * cell.unit;
+  const uint32_t row0 = static_cast<uint32_t>(cell_slot(g, i0 + 1, j0 + 1));
   const CellVal<T> c0 = cell(row0);
   const bool short_path = !wide_mark(cells, epoch);
   T acc = macc<FMA>(kernel[kmid], c0.x, T(0));  // src/lib.rs:375-383
-  acc = trace_direction<T, FMA, BRANCHLESS, POL, true, REC, BUF>(
+  acc = trace_direction<T, FMA, BRANCHLESS, POL, true, REC, BUF, BUF>(
       acc, c0.u, c0.v, row0, cell, kernel, kmid, n_fwd, sg, codes, np, p, 0, short_path);
-  acc = trace_direction<T, FMA, BRANCHLESS, POL, false, REC, BUF>(
+  acc = trace_direction<T, FMA, BRANCHLESS, POL, false, REC, BUF, BUF>(
       acc, c0.u, c0.v, row0, cell, kernel, kmid, n_bwd, sg, codes, np, p, chunks_of(n_fwd),
       short_path);
   out[static_cast<int64_t>(i0) * g.nx + j0] = acc;
@@ -135,7 +139,7 @@ __global__ __launch_bounds__(64) void lic_trace_pair(
   // a block is one wave: eight blocks take the 256 pixels of a tile
   int32_t ty, tx, py, px;
   tile_of_block(static_cast<int32_t>(blockIdx.x) >> 3, m, ty, tx);
-  pixel_of_thread((static_cast<int32_t>(blockIdx.x) & 7) * 32 + k, m, py, px);
+  pixel_of_quads((static_cast<int32_t>(blockIdx.x) & 7) * 32 + k, m, py, px);
   const int32_t i0 = ty * tile_h(m) + py, j0 = tx * tile_w(m) + px;
   const bool inside = i0 < g.ny && j0 < g.nx;
   const int32_t kmid = klen / 2;  // steps of either direction
@@ -147,17 +151,16 @@ __global__ __launch_bounds__(64) void lic_trace_pair(
   T acc = T(0);
   int32_t live_steps = 0;  // backward lanes: steps before the line ended
   if (inside) {
-    const CellGather<T, true> cell(cells, guarded_cells(g.ny, g.nx));
-    const StepGeom sg = make_step_geom(g, cell.unit);
+    const CellGather<T, true> cell(cells, cell_slots(g));
+    const StepGeom sg = make_step_geom(g);
     const int64_t np = static_cast<int64_t>(g.ny) * g.nx;
-    const uint32_t row0 =
-        static_cast<uint32_t>(i0 + 1) * sg.grow + static_cast<uint32_t>(j0 + 1) * cell.unit;
+    const uint32_t row0 = static_cast<uint32_t>(cell_slot(g, i0 + 1, j0 + 1));
     const CellVal<T> c0 = cell(row0);
     acc = macc<FMA>(kernel[kmid], c0.x, T(0));  // src/lib.rs:375-383
     // every lane stores (no branch in the step): forward lanes into the
     // spare row kmid
     auto keep = [&](int32_t s, T x) { vals[32 * (fwd ? kmid : s)] = x; };
-    acc = trace_direction<T, FMA, BRANCHLESS, POL, true, REC, true, true>(
+    acc = trace_direction<T, FMA, BRANCHLESS, POL, true, REC, true, true, true>(
         acc, c0.u, c0.v, row0, cell, kernel, kmid, kmid, sg, codes, np, p,
         fwd ? 0 : chunks_of(kmid), !wide_mark(cells, epoch), fwd, keep, &live_steps);
   }
@@ -668,6 +671,9 @@ __global__ __launch_bounds__(kLdsThreads) void lic_replay_lds(const T* __restric
 // Launchers
 // ---------------------------------------------------------------------------
 
+// Buffer addressing covers arrays of fewer than 2^32 bytes.
+inline bool fits_buffer(int64_t bytes) { return bytes > 0 && bytes <= 0xFFFFFFFFll; }
+
 TileMap make_tile_map(int32_t ny, int32_t nx, int32_t band, int32_t wave_w_log2) {
   TileMap m;
   m.wave_w_log2 = wave_w_log2 < 3 ? 3 : (wave_w_log2 > 5 ? 5 : wave_w_log2);
@@ -706,6 +712,12 @@ hipError_t launch_pack(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64
 
 int32_t kernel_pad() { return kKernelPad; }
 
+template <typename T>
+void choose_row_order(FieldGeom& g) {
+  g.linear = 0;
+  if (!fits_buffer(cell_slots(g) * static_cast<int64_t>(sizeof(Cell<T>)))) g.linear = 1;
+}
+
 uint32_t next_epoch() {
   static std::atomic<uint32_t> epoch{0};
   return epoch.fetch_add(1, std::memory_order_relaxed) + 1;
@@ -728,15 +740,12 @@ hipError_t launch_copy2d(const T* src, int64_t sy, int64_t sx, int32_t ny, int32
   return hipGetLastError();
 }
 
-// Buffer addressing covers arrays of fewer than 2^32 bytes.
-inline bool fits_buffer(int64_t bytes) { return bytes > 0 && bytes <= 0xFFFFFFFFll; }
-
 
 template <typename T, bool FMA, bool BL, bool POL, bool REC>
 static hipError_t trace_one(const Cell<T>* cells, const T* kernel, int32_t klen,
                             const FieldGeom& g, const TileMap& m, T* out, uint4* codes, uint32_t epoch,
                             hipStream_t stream) {
-  if (fits_buffer(guarded_cells(g.ny, g.nx) * static_cast<int64_t>(sizeof(Cell<T>)))) {
+  if (fits_buffer(cell_slots(g) * static_cast<int64_t>(sizeof(Cell<T>)))) {
     hipLaunchKernelGGL((lic_trace<T, FMA, BL, POL, REC, true>), dim3(m.n_tiles), dim3(kBlock),
                        0, stream, cells, kernel, klen, g, m, out, codes, epoch);
   } else {
@@ -868,10 +877,10 @@ int32_t lds_replay_limit_bytes() {
 }
 
 template <typename T>
-bool trace_pair_fits(int32_t klen, int64_t ny, int64_t nx) {
+bool trace_pair_fits(int32_t klen, const FieldGeom& g) {
   const size_t limit = static_cast<size_t>(lds_replay_limit_bytes());
   return klen % 2 == 1 && trace_pair_lds_bytes(klen, sizeof(T)) <= limit &&
-         fits_buffer(guarded_cells(ny, nx) * static_cast<int64_t>(sizeof(Cell<T>)));
+         fits_buffer(cell_slots(g) * static_cast<int64_t>(sizeof(Cell<T>)));
 }
 
 template <typename T>
@@ -879,7 +888,7 @@ hipError_t launch_trace_pair(const Cell<T>* cells, const T* kernel, int32_t klen
                              const FieldGeom& g, const TileMap& m, int uv_mode, int profile,
                              T* out, uint4* codes, uint32_t epoch,
                              hipStream_t stream) {
-  if (!trace_pair_fits<T>(klen, g.ny, g.nx)) return hipErrorInvalidValue;
+  if (!trace_pair_fits<T>(klen, g)) return hipErrorInvalidValue;
   switch (profile & 3) {
     case 0:
       return trace_pair_mode<T, false, false>(cells, kernel, klen, g, m, uv_mode, out, codes, epoch,
@@ -1020,8 +1029,9 @@ hipError_t launch_replay_lds_hybrid(const T* x, const T* kernel, int32_t klen, c
                                       hipStream_t);                                             \
   template hipError_t launch_replay<T>(const T*, const T*, int32_t, const FieldGeom&,          \
                                        const TileMap&, int, T*, const uint4*, hipStream_t);    \
+  template void choose_row_order<T>(FieldGeom&);                                               \
   template bool lds_replay_fits<T>(int32_t);                                                   \
-  template bool trace_pair_fits<T>(int32_t, int64_t, int64_t);                               \
+  template bool trace_pair_fits<T>(int32_t, const FieldGeom&);                                 \
   template hipError_t launch_trace_pair<T>(const Cell<T>*, const T*, int32_t, const FieldGeom&, \
                                            const TileMap&, int, int, T*, uint4*, uint32_t,      \
                                            hipStream_t);                                        \

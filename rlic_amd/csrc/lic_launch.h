@@ -15,8 +15,16 @@ TileMap make_tile_map(int32_t ny, int32_t nx, int32_t band, int32_t wave_w_log2)
 // slot for a kernel of length klen (forward chunks, then backward chunks).
 int32_t code_chunks(int32_t klen);
 
-// The field's guarded cell array (guarded_cells(ny, nx) cells) from its
-// strided texture, u and v; with `kpad`, in the same launch, the padded
+// Sets g.linear: row pairs where buffer loads address the array (4 GiB), else
+// plain rows.  (Beyond, the trace's global loads cost it a 64-bit add a step
+// and the choice of the row distance another 8 issue cycles of about 100,
+// more than the pairs gave there: 16384^2 float polarization 56.8 ms with
+// pairs, 54.8 without.)
+template <typename T>
+void choose_row_order(FieldGeom& g);
+
+// The field's guarded cell array (cell_slots(g) cells) from its strided
+// texture, u and v; with `kpad`, in the same launch, the padded
 // weight copy of `kernel`: kpad (klen + 2 * kernel_pad() elements) =
 // [zeros][kernel][zeros].
 template <typename T>
@@ -56,7 +64,7 @@ hipError_t launch_trace(const Cell<T>* cells, const T* kernel, int32_t klen, con
 // same record, and returns hipErrorInvalidValue where it does not apply.
 size_t trace_pair_lds_bytes(int32_t klen, size_t elem);
 template <typename T>
-bool trace_pair_fits(int32_t klen, int64_t ny, int64_t nx);
+bool trace_pair_fits(int32_t klen, const FieldGeom& g);
 template <typename T>
 hipError_t launch_trace_pair(const Cell<T>* cells, const T* kernel, int32_t klen,
                              const FieldGeom& g, const TileMap& m, int uv_mode, int profile,

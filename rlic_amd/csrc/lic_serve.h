@@ -90,6 +90,8 @@ class Server {
 
  private:
   template <typename T>
+  static size_t block_bytes(int64_t cells, int64_t ny, int64_t nx, int64_t klen, bool record);
+  template <typename T>
   std::map<int64_t, Resident<T>>& table();
   template <typename T>
   void plan_dtype(StepWork<T>& w, std::vector<int64_t>& finished);

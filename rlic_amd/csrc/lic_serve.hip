@@ -89,9 +89,14 @@ constexpr int64_t kSingleReplayMinPixels = int64_t{1} << 18;
 
 template <typename T>
 size_t Server::field_bytes(int64_t ny, int64_t nx, int64_t klen, bool record) {
+  return block_bytes<T>(guarded_cells(ny, nx), ny, nx, klen, record);
+}
+
+template <typename T>
+size_t Server::block_bytes(int64_t cells, int64_t ny, int64_t nx, int64_t klen, bool record) {
   const size_t n = static_cast<size_t>(ny * nx);
   size_t b = align256(sizeof(T) * static_cast<size_t>(std::max<int64_t>(klen, 0) + 2 * kernel_pad()));
-  b += align256(sizeof(Cell<T>) * static_cast<size_t>(guarded_cells(ny, nx)));
+  b += align256(sizeof(Cell<T>) * static_cast<size_t>(cells));
   b += 2 * align256(sizeof(T) * n);
   if (record) b += align256(sizeof(uint4) * static_cast<size_t>(code_chunks(static_cast<int32_t>(klen))) * n);
   return b;
@@ -115,7 +120,10 @@ int Server::admit(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
   r.uv_mode = uv_mode;
   r.epoch = next_epoch();
   r.bytes = bytes;
-  r.block_bytes = size_class(bytes);
+  choose_row_order<T>(r.g);
+  // the charge counts the cells themselves, the block their slots as well
+  // (half a row pair more when ny is odd)
+  r.block_bytes = size_class(block_bytes<T>(cell_slots(r.g), ny, nx, klen, record));
   if (hipError_t e = take_block(bytes, r.block_bytes, &r.block); e != hipSuccess) {
     (void)hipGetLastError();
     err = std::string("allocating resident field: ") + hipGetErrorString(e);
@@ -128,7 +136,7 @@ int Server::admit(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
   r.weights = padded + pad;
   p += align256(sizeof(T) * static_cast<size_t>(std::max<int64_t>(klen, 0) + 2 * pad));
   r.cells = reinterpret_cast<Cell<T>*>(p);
-  p += align256(sizeof(Cell<T>) * static_cast<size_t>(guarded_cells(ny, nx)));
+  p += align256(sizeof(Cell<T>) * static_cast<size_t>(cell_slots(r.g)));
   r.buf[0] = reinterpret_cast<T*>(p);
   p += align256(sizeof(T) * n);
   r.buf[1] = reinterpret_cast<T*>(p);

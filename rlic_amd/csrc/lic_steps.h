@@ -22,9 +22,8 @@ __host__ __device__ inline int32_t chunks_of(int32_t nsteps) {
 }
 
 // One streamline direction of one pixel (src/lib.rs:304-362), starting from
-// the vector (pu, pv) of the start cell, already loaded.  The position is
-// (row, j) with row = i * nx, both in the gather's units.  Returns the
-// updated accumulator.  With REC, writes the move code of every step.
+// the vector (pu, pv) of the start cell, already loaded.  The position `row`
+// is the cell's slot (cell_slot).  Returns the updated accumulator.  With REC, writes the move code of every step.
 //
 // The step is written without divergent branches: a lane whose line has
 // ended (NaN vector) keeps executing with its position frozen and its
@@ -35,12 +34,15 @@ __host__ __device__ inline int32_t chunks_of(int32_t nsteps) {
 // whole groups of the branchless rule run as fast_group.
 //
 // The cells form a guarded array (guarded_cells: (ny + 2) x (nx + 2)
-// with a ring of guard cells around the image) and `row` is the position.
+// with a ring of guard cells around the image).
 // A guard cell holds the values of the cell that a step onto it ends on by
 // the boundary rule (src/lib.rs:83-95: the edge cell itself for a closed
 // side, the opposite edge cell for a periodic one) and, in its pad slot,
 // the jump in cells to that cell (0 in image cells): a step is one add of
 // +-1 cell or +-1 row, the gather, and one shifted add of the jump.
+//
+// PAIRS: the array may be in row pairs (or plain rows, as `sg` says); without,
+// it is in plain rows.
 //
 // LANE_DIR: the direction is the lane's own (forward where fwd_lane), one
 // body for both (the paired trace, lic_trace_pair); FORWARD then names the
@@ -88,20 +90,25 @@ struct NoSink {
 // shift-or, bfi, add with carry, every double operation), 8 for v_rcp_f32 and
 // 16 for v_rcp_f64 (measured with streams of one instruction).  So choices are
 // made with lane masks in VGPRs (sign words and v_bitop3) rather than with
-// compares and v_cndmask.  Trace launches, full rule alone -> with this:
-// 4096^2 float L=129 with the record 2.47 -> 1.94 ms, 16384^2 float
-// polarization L=257 72.2 -> 55.3 ms, 8192^2 double polarization L=257
-// 30.1 -> 26.5 ms, 256^2 double L=65 (paired) 22.6 -> 19.3 us.
-template <typename T, bool FMA, int POL, bool FORWARD, int REC, bool BUF, bool LANE_DIR,
-          typename Sink>
+// compares and v_cndmask.  A step is about 36 VALU instructions, 90 issue
+// cycles per wave (the full rule's 57 took about 170); with that the L1 gather
+// path is as busy (TD 97%, 29-34 cycles per wave gather on the CU's one
+// path).  Trace launches, full rule in plain rows -> with this alone -> and
+// row pairs (cell_slot): 4096^2 float L=129 with the record 2.47 -> 1.92 ->
+// 1.86 ms, 2111x1500 float with holes L=201 775 -> 684 -> 603 us, 1021x1537
+// double L=151 499 -> 447 -> 430 us, 16384^2 float polarization L=257 (plain
+// rows) 72.2 -> 55.0 -> 54.5 ms, 8192^2 double polarization 30.1 -> 26.4 ->
+// 26.4 ms, 256^2 double L=65 (paired lanes) 22.6 -> 19.3 -> 19.9 us.
+template <typename T, bool FMA, int POL, bool FORWARD, int REC, bool BUF, bool PAIRS,
+          bool LANE_DIR, typename Sink>
 __device__ __forceinline__ uint64_t fast_group(
     T& acc, T& fx, T& fy, T& pu, T& pv, T& last_u, T& last_v, uint32_t& row, uint32_t& word,
-    const T (&kw)[8], const CellGather<T, BUF>& cell, uint32_t step_x, uint32_t step_y,
-    uint32_t lane_sign, int32_t s0, Sink& sink) {
+    const T (&kw)[8], const CellGather<T, BUF>& cell, const StepGeom& sg, uint32_t lane_sign,
+    int32_t s0, Sink& sink) {
   // masks of the sign of (pu, pv): a backward step's signs are the opposite
   constexpr bool kFlip = !FORWARD && !LANE_DIR;
-  uint64_t reported = 0;
-  uint32_t low = 0xFFFFFFFFu;  // smallest numerator seen (numerator_key)
+  uint32_t apart = 0xFFFFFFFFu;  // sign bit: no near tie so far
+  uint32_t low = 0xFFFFFFFFu;    // smallest numerator seen (numerator_key)
   uint32_t jump[8], jumped = 0;
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
@@ -124,23 +131,34 @@ __device__ __forceinline__ uint64_t fast_group(
     const T cy = ny * abs_t(mu);
     const T e = fma_t(nx, abs_t(mv), -cy);
     const uint32_t mx = sign_mask(e);  // step along x
-    reported |= __builtin_amdgcn_ballot_w64(!(abs_t(e) > cy * near_tie(static_cast<T*>(nullptr))));
+    apart &= top_word(fma_t(near_tie(static_cast<T*>(nullptr)), cy, -abs_t(e)));
     // where the picked component is nonzero (or the lane is reported),
     // pos_x and pos_y of the full rule are the sign tests already made
     const uint32_t sp = pick(mx, sx, sy);
-    const uint32_t s = pick(mx, step_x, step_y);
+    uint32_t dist_y = sg.far_y;
+    if constexpr (PAIRS) {
+      const uint32_t far = bitop3<kFlip ? 0xEB : 0xBE>(0u - (row & 1u), sp, sg.all_far);
+      dist_y = pick(far, sg.far_y, sg.near_y);
+    }
+    const uint32_t s = pick(mx, sg.step_x, dist_y);
     const uint32_t at = kFlip ? row + sp - (s ^ sp) : row - sp + (s ^ sp);
     const CellVal<T> cv = cell(at);
     const T n = pick(mx, nx, ny);
     const T t = quotient_rn(n, abs_t(pick(mx, mu, mv)));
     low = min(low, numerator_key(n));
+    if (q & 1) {
+      keep_in_step(apart);
+      keep_in_step(low);
+    }
     const T fy_after_x = macc<FMA>(t, mv, fy);
     const T fx_after_y = macc<FMA>(t, mu, fx);
-    fx = pick_edge<kFlip>(mx, sp, fx_after_y);
-    fy = pick_edge<kFlip>(~mx, sp, fy_after_x);
+    // on the edge just crossed: 1 after a step toward lower indices, else 0
+    const T edge = edge_fraction<kFlip>(sp, static_cast<T*>(nullptr));
+    fx = pick(mx, edge, fx_after_y);
+    fy = pick(mx, fy_after_x, edge);
     jump[q] = pad_bits(cv.pad);
     jumped |= jump[q];
-    row = at + jump[q] * cell.unit;
+    row = at + jump[q];
     acc = macc<FMA>(kw[q], cv.x, acc);  // src/lib.rs:353-360
     sink(s0 + q, cv.x);
     pu = cv.u;
@@ -155,15 +173,20 @@ __device__ __forceinline__ uint64_t fast_group(
     word = (word & 0x33333333u) | 0x11111111u * kMoveMoved;
     if (__builtin_amdgcn_ballot_w64(jumped != 0u) != 0) {  // uniform: some line left the image
 #pragma unroll
-      for (int q = 0; q < 8; ++q) word |= jump[q] != 0u ? kMoveEdge << (28 - 4 * q) : 0u;
+      for (int q = 0; q < 8; ++q) {
+        keep_in_step(jump[q]);  // compared here, not before the branch
+        word |= jump[q] != 0u ? kMoveEdge << (28 - 4 * q) : 0u;
+      }
+      keep_in_step(word);  // a branch, not selects
     }
   }
-  return reported |
-         __builtin_amdgcn_ballot_w64(low < numerator_key_min(static_cast<T*>(nullptr)));
+  return __builtin_amdgcn_ballot_w64(static_cast<int32_t>(apart) >= 0) |
+         __builtin_amdgcn_ballot_w64(low < numerator_key_min(static_cast<T*>(nullptr))) |
+         __builtin_amdgcn_ballot_w64(__builtin_isunordered(fx, fy));
 }
 
 template <typename T, bool FMA, bool BRANCHLESS, int POL, bool FORWARD, int REC, bool BUF,
-          bool LANE_DIR = false, typename Sink = NoSink>
+          bool PAIRS, bool LANE_DIR = false, typename Sink = NoSink>
 __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
                                              const CellGather<T, BUF>& cell,
                                              const T* __restrict__ kernel, int32_t kmid,
@@ -177,9 +200,7 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
   T fx = T(0.5), fy = T(0.5);      // src/lib.rs:315-318
   T last_u = T(0), last_v = T(0);  // src/lib.rs:320-323
   bool alive = true;
-  const uint32_t unit = cell.unit;
-  const uint32_t row_up = lane_copy(sg.grow);  // row step, held in VGPRs across the loop
-  const uint32_t row_down = lane_copy(0u - sg.grow);
+  const uint32_t far_y = lane_copy(sg.far_y), near_y = lane_copy(sg.near_y);  // held in VGPRs
   const int32_t nchunks = chunks_of(nsteps);
   // Short path: whole groups of a chunk by fast_group; when a moving lane is
   // reported, the chunk is done again by the full rule.  Off for the rest of
@@ -202,7 +223,8 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
         status_known = true;
       }
       const uint64_t m_moves = __builtin_amdgcn_ballot_w64(moves_now);
-      const uint32_t step_x = moves_now ? unit : 0u, step_y = moves_now ? sg.grow : 0u;
+      const StepGeom sl = {moves_now ? sg.step_x : 0u, moves_now ? near_y : 0u,
+                           moves_now ? far_y : 0u, sg.all_far};
       // fractions outside what fast_group takes (the full rule can leave
       // some after a tie): this chunk by the full rule
       const bool usable = __builtin_amdgcn_ballot_w64(moves_now && !(fraction_usable(fx) &&
@@ -220,9 +242,9 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
         for (int q = 0; q < 8; ++q)
           kw[q] = kernel[FORWARD ? kmid + 1 + s0 + q : kmid - 1 - s0 - q];
         uint32_t word = 0;
-        reported = fast_group<T, FMA, POL, FORWARD, REC, BUF, LANE_DIR>(
-                       acc, fx, fy, pu, pv, last_u, last_v, row, word, kw, cell, step_x, step_y,
-                       lane_sign, s0, sink) &
+        reported = fast_group<T, FMA, POL, FORWARD, REC, BUF, PAIRS, LANE_DIR>(
+                       acc, fx, fy, pu, pv, last_u, last_v, row, word, kw, cell, sl, lane_sign,
+                       s0, sink) &
                    m_moves;
         if (reported != 0) break;  // uniform
         words[g0] = word;
@@ -320,12 +342,16 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
         // its position update.
         fx = fx_new;
         fy = fy_new;
-        const uint32_t step = xs ? (pos_x ? unit : 0u - unit) : (pos_y ? row_up : row_down);
+        // a y step leaves the row pair up from an odd row, down from an even one
+        const bool odd = (row & 1u) != 0u;
+        const uint32_t dist_y = !PAIRS || odd == pos_y || sg.all_far != 0u ? far_y : near_y;
+        const uint32_t step = xs ? (pos_x ? sg.step_x : 0u - sg.step_x)
+                                 : (pos_y ? dist_y : 0u - dist_y);
         const uint32_t at = moves ? row + step : row;
         const CellVal<T> cv = cell(at);
         const uint32_t jump = pad_bits(cv.pad);
         const bool edge = jump != 0u;  // the step left the image
-        row = at + jump * unit;
+        row = at + jump;
         const T next_acc = macc<FMA>(kw[q], cv.x, acc);  // src/lib.rs:353-360
         acc = live ? next_acc : acc;
         sink(s0 + q, cv.x);
