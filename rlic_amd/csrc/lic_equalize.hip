@@ -14,12 +14,15 @@
 //     when vmax == vmin every finite pixel is in bin 0;
 //   * out = cdf[bin] / N in double, rounded once to the image type.
 //
-// Four stream-ordered launches, no host round trip: the finite range (one
-// read of the image; block min/max/count, then one atomic per block on
-// order-preserving integer keys), the histogram (a second read; per-block
-// LDS histograms merged with global atomics), an inclusive scan of the
-// counts (one block), and the map (a third read and the write).  All of
-// it is integer and HBM traffic: 3 reads and 1 write of the image.
+// Five stream-ordered launches, no host round trip: the finite range (one
+// read of the image; a partial result per block on order-preserving integer
+// keys), their reduction (which also clears the counters), the histogram (a
+// second read; per-block LDS histograms merged with global atomics), an
+// inclusive scan of the counts (one block), and the map (a third read and
+// the write).  All of it is integer and HBM traffic: 3 reads and 1 write of
+// the image.  4096^2 floats, 256 bins: range 16, histogram 20, map 28 us, 70 us
+// a call (87, 74, 44 and 213 with an atomic per block on the range, 8 blocks
+// per CU on the counters and a division per pixel).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -64,11 +67,43 @@ struct KeyOf<double> {
 
 constexpr int kThreads = 256;
 
+// Bins whose values lic_eq_map keeps in LDS (16 KB in double: eight blocks
+// per CU), and whose counts every wave of lic_eq_hist keeps for itself.
+constexpr int32_t kTableBins = 2048;
+
+constexpr int kHistThreads = 1024;
+// Blocks of lic_eq_range, each with its own partial result.
+constexpr int32_t kRangeBlocks = 2048;
+
 template <typename T>
 __device__ __forceinline__ T load_px(const T* __restrict__ img, int64_t p, int32_t nx, int64_t sy,
                                      int64_t sx) {
   const int64_t i = p / nx, j = p - i * nx;
   return img[i * sy + j * sx];
+}
+
+// f(x, p) for this thread's share of the image's pixels (p: C-order index).
+// A contiguous image is read without index arithmetic, eight loads in flight
+// per lane, 256 consecutive bytes a wave (float): HBM-bound.  With a 64-bit
+// division per pixel (the strided form) reading 4096^2 floats once took 87 us;
+// this takes 16.
+template <typename T, typename F>
+__device__ __forceinline__ void each_pixel(const T* __restrict__ img, int64_t n, int32_t nx,
+                                           int64_t sy, int64_t sx, F f) {
+  const int64_t step = static_cast<int64_t>(gridDim.x) * blockDim.x;
+  int64_t p = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (sx == 1 && sy == nx) {  // uniform
+    for (; p + 7 * step < n; p += 8 * step) {
+      T x[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) x[k] = img[p + k * step];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) f(x[k], p + k * step);
+    }
+    for (; p < n; p += step) f(img[p], p);
+  } else {
+    for (; p < n; p += step) f(load_px(img, p, nx, sy, sx), p);
+  }
 }
 
 // The bin of a finite pixel (see the file comment); vmin < vmax.
@@ -105,36 +140,12 @@ __device__ __forceinline__ EqRange read_range(const EqState<T>* st, int32_t nbin
   return r;
 }
 
+// The block's smallest and largest key and count, in thread 0's arguments.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void lic_eq_init(EqState<T>* st, uint32_t* hist,
-                                                       int32_t nbins) {
-  const int32_t t = blockIdx.x * kThreads + threadIdx.x;
-  if (t == 0) {
-    st->min_key = KeyOf<T>::kMax;
-    st->max_key = 0;
-    st->count = 0;
-  }
-  for (int32_t b = t; b < nbins; b += gridDim.x * kThreads) hist[b] = 0u;
-}
-
-// Smallest and largest finite value and the count of finite pixels.
-template <typename T>
-__global__ __launch_bounds__(kThreads) void lic_eq_range(const T* __restrict__ img, int64_t n,
-                                                        int32_t nx, int64_t sy, int64_t sx,
-                                                        EqState<T>* st) {
+__device__ __forceinline__ void reduce_range(typename KeyOf<T>::type& lo,
+                                             typename KeyOf<T>::type& hi,
+                                             unsigned long long& cnt) {
   typedef typename KeyOf<T>::type Key;
-  Key lo = KeyOf<T>::kMax, hi = 0;
-  unsigned long long cnt = 0;
-  for (int64_t p = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; p < n;
-       p += static_cast<int64_t>(gridDim.x) * kThreads) {
-    const T x = load_px(img, p, nx, sy, sx);
-    if (__builtin_isfinite(x)) {
-      const Key k = order_key(x);
-      lo = k < lo ? k : lo;
-      hi = k > hi ? k : hi;
-      ++cnt;
-    }
-  }
   for (int off = 32; off > 0; off >>= 1) {
     const Key olo = __shfl_xor(lo, off), ohi = __shfl_xor(hi, off);
     lo = olo < lo ? olo : lo;
@@ -156,42 +167,80 @@ __global__ __launch_bounds__(kThreads) void lic_eq_range(const T* __restrict__ i
       hi = s_hi[k] > hi ? s_hi[k] : hi;
       cnt += s_cnt[k];
     }
-    if (cnt != 0) {
-      atomicMin(&st->min_key, lo);
-      atomicMax(&st->max_key, hi);
-      atomicAdd(&st->count, cnt);
-    }
   }
 }
 
-// Histogram of the finite pixels' bins: per-block LDS histograms (nbins up
-// to kLdsBins) merged into the global one, else global atomics.
+// The blocks' ranges to the image's (block 0), and the counters to zero.
+// (One atomic per block on the range's three words cost 60 us of a 4096^2
+// image's 80: 2048 blocks on one cache line.)
+template <typename T>
+__global__ __launch_bounds__(kThreads) void lic_eq_init(const EqState<T>* part, int32_t parts,
+                                                       EqState<T>* st, uint32_t* hist,
+                                                       int32_t nbins) {
+  typedef typename KeyOf<T>::type Key;
+  for (int32_t b = blockIdx.x * kThreads + threadIdx.x; b < nbins; b += gridDim.x * kThreads)
+    hist[b] = 0u;
+  if (blockIdx.x != 0) return;
+  Key lo = KeyOf<T>::kMax, hi = 0;
+  unsigned long long cnt = 0;
+  for (int32_t k = threadIdx.x; k < parts; k += kThreads) {
+    lo = part[k].min_key < lo ? part[k].min_key : lo;
+    hi = part[k].max_key > hi ? part[k].max_key : hi;
+    cnt += part[k].count;
+  }
+  reduce_range<T>(lo, hi, cnt);
+  if (threadIdx.x == 0) *st = EqState<T>{lo, hi, cnt};
+}
+
+// Smallest and largest finite value and the count of finite pixels, per block.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void lic_eq_range(const T* __restrict__ img, int64_t n,
+                                                        int32_t nx, int64_t sy, int64_t sx,
+                                                        EqState<T>* part) {
+  typedef typename KeyOf<T>::type Key;
+  Key lo = KeyOf<T>::kMax, hi = 0;
+  unsigned long long cnt = 0;
+  each_pixel(img, n, nx, sy, sx, [&](T x, int64_t) {
+    if (__builtin_isfinite(x)) {
+      const Key k = order_key(x);
+      lo = k < lo ? k : lo;
+      hi = k > hi ? k : hi;
+      ++cnt;
+    }
+  });
+  reduce_range<T>(lo, hi, cnt);
+  if (threadIdx.x == 0) part[blockIdx.x] = EqState<T>{lo, hi, cnt};
+}
+
+// Histogram of the finite pixels' bins: LDS histograms of a block (nbins up to
+// kLdsBins), `copies` of them (a power of two, waves dealt over them so that
+// fewer add to the same counters at once), merged into the global one;
+// without LDS, global atomics.  Few, large blocks: the merge is nbins global
+// atomics per block, and 2048 blocks on 256 counters cost 30 us.
 template <typename T, bool LDS>
-__global__ __launch_bounds__(kThreads) void lic_eq_hist(const T* __restrict__ img, int64_t n,
+__global__ __launch_bounds__(kHistThreads) void lic_eq_hist(const T* __restrict__ img, int64_t n,
                                                        int32_t nx, int64_t sy, int64_t sx,
                                                        int32_t nbins, const EqState<T>* st,
-                                                       uint32_t* __restrict__ hist) {
-  __shared__ uint32_t local[LDS ? kLdsBins : 1];
+                                                       uint32_t* __restrict__ hist,
+                                                       int32_t copies) {
+  extern __shared__ uint32_t local[];  // copies * nbins counters
   const EqRange r = read_range(st, nbins);
+  uint32_t* mine = LDS ? local + ((threadIdx.x >> 6) & (copies - 1)) * nbins : hist;
   if (LDS) {
-    for (int32_t b = threadIdx.x; b < nbins; b += kThreads) local[b] = 0u;
+    for (int32_t b = threadIdx.x; b < copies * nbins; b += kHistThreads) local[b] = 0u;
     __syncthreads();
   }
-  for (int64_t p = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; p < n;
-       p += static_cast<int64_t>(gridDim.x) * kThreads) {
-    const T x = load_px(img, p, nx, sy, sx);
-    if (!__builtin_isfinite(x)) continue;
-    const int32_t b = r.constant ? 0 : eq_bin(static_cast<double>(x), r, nbins);
-    if (LDS) {
-      atomicAdd(&local[b], 1u);
-    } else {
-      atomicAdd(&hist[b], 1u);
+  each_pixel(img, n, nx, sy, sx, [&](T x, int64_t) {
+    if (__builtin_isfinite(x))
+      atomicAdd(&mine[r.constant ? 0 : eq_bin(static_cast<double>(x), r, nbins)], 1u);
+  });
+  if (LDS) {
+    __syncthreads();
+    for (int32_t b = threadIdx.x; b < nbins; b += kHistThreads) {
+      uint32_t sum = local[b];
+      for (int32_t k = 1; k < copies; ++k) sum += local[k * nbins + b];
+      if (sum != 0u) atomicAdd(&hist[b], sum);
     }
-  }
-  if (LDS) {
-    __syncthreads();
-    for (int32_t b = threadIdx.x; b < nbins; b += kThreads)
-      if (local[b] != 0u) atomicAdd(&hist[b], local[b]);
   }
 }
 
@@ -223,23 +272,32 @@ __global__ __launch_bounds__(kScanThreads) void lic_eq_scan(uint32_t* hist_all, 
   }
 }
 
-template <typename T>
+// The map.  TABLE (nbins up to kTableBins): the value of every bin is divided
+// out once per block into LDS, so a pixel costs a lookup instead of a
+// gather of its count and a double division.
+template <typename T, bool TABLE>
 __global__ __launch_bounds__(kThreads) void lic_eq_map(const T* __restrict__ img, int64_t n,
                                                       int32_t nx, int64_t sy, int64_t sx,
                                                       int32_t nbins, const EqState<T>* st,
                                                       const uint32_t* __restrict__ cdf,
                                                       T* __restrict__ out) {
+  __shared__ T table[TABLE ? kTableBins : 1];
   const EqRange r = read_range(st, nbins);
-  for (int64_t p = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; p < n;
-       p += static_cast<int64_t>(gridDim.x) * kThreads) {
-    const T x = load_px(img, p, nx, sy, sx);
+  auto value = [&](int32_t b) {
+    return static_cast<T>(static_cast<double>(cdf[b]) / static_cast<double>(r.count));
+  };
+  if (TABLE) {
+    for (int32_t b = threadIdx.x; b < nbins; b += kThreads) table[b] = value(b);
+    __syncthreads();
+  }
+  each_pixel(img, n, nx, sy, sx, [&](T x, int64_t p) {
     T y = x;
     if (__builtin_isfinite(x)) {
       const int32_t b = r.constant ? 0 : eq_bin(static_cast<double>(x), r, nbins);
-      y = static_cast<T>(static_cast<double>(cdf[b]) / static_cast<double>(r.count));
+      y = TABLE ? table[b] : value(b);
     }
     out[p] = y;
-  }
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -255,12 +313,10 @@ __global__ __launch_bounds__(kThreads) void lic_eq_bins(const T* __restrict__ im
                                                        int32_t nbins, const EqState<T>* st,
                                                        int32_t* __restrict__ bins) {
   const EqRange r = read_range(st, nbins);
-  for (int64_t p = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; p < n;
-       p += static_cast<int64_t>(gridDim.x) * kThreads) {
-    const T x = load_px(img, p, nx, sy, sx);
+  each_pixel(img, n, nx, sy, sx, [&](T x, int64_t p) {
     bins[p] = __builtin_isfinite(x) ? (r.constant ? 0 : eq_bin(static_cast<double>(x), r, nbins))
                                     : -1;
-  }
+  });
 }
 
 // Sliding tile: out = (finite window pixels with a bin <= the pixel's) /
@@ -453,9 +509,44 @@ int grid_for(int64_t n, int32_t per_cu) {
 
 }  // namespace
 
+// Scratch: the state, the blocks' ranges, the counters.
+template <typename T>
+static size_t counters_offset() {
+  return (sizeof(EqState<T>) * (1 + kRangeBlocks) + 255) & ~size_t{255};
+}
+
 template <typename T>
 size_t equalize_scratch_bytes(int32_t nbins) {
-  return ((sizeof(EqState<T>) + 255) & ~size_t{255}) + sizeof(uint32_t) * static_cast<size_t>(nbins);
+  return counters_offset<T>() + sizeof(uint32_t) * static_cast<size_t>(nbins);
+}
+
+// The image's finite range into st[0], and its nbins counters cleared.
+template <typename T>
+static void launch_range(const T* img, int64_t n, int32_t nx, int64_t sy, int64_t sx,
+                         int32_t nbins, EqState<T>* st, uint32_t* hist, hipStream_t stream) {
+  const int g = std::min(grid_for(n, 8), kRangeBlocks);
+  hipLaunchKernelGGL(lic_eq_range<T>, dim3(g), dim3(kThreads), 0, stream, img, n, nx, sy, sx,
+                     st + 1);
+  const int blocks = std::min(1024, (nbins + kThreads - 1) / kThreads);
+  hipLaunchKernelGGL(lic_eq_init<T>, dim3(blocks < 1 ? 1 : blocks), dim3(kThreads), 0, stream,
+                     st + 1, g, st, hist, nbins);
+}
+
+// The global histogram of the image, into cleared counters.
+template <typename T>
+static void launch_hist(const T* img, int64_t n, int32_t nx, int64_t sy, int64_t sx, int32_t nbins,
+                        const EqState<T>* st, uint32_t* hist, hipStream_t stream) {
+  const int gh = (grid_for(n, 8) + 3) / 4;  // two blocks of 16 waves per CU at most
+  if (nbins <= kLdsBins) {
+    const int32_t copies = nbins <= kTableBins ? 4 : 1;
+    const size_t lds = sizeof(uint32_t) * static_cast<size_t>(copies) * nbins;  // at most 64 KB
+    hipLaunchKernelGGL((lic_eq_hist<T, true>), dim3(gh), dim3(kHistThreads),
+                       static_cast<unsigned>(lds), stream, img, n, nx, sy, sx, nbins, st, hist,
+                       copies);
+  } else {
+    hipLaunchKernelGGL((lic_eq_hist<T, false>), dim3(gh), dim3(kHistThreads), 0, stream, img, n,
+                       nx, sy, sx, nbins, st, hist, 1);
+  }
 }
 
 template <typename T>
@@ -463,28 +554,18 @@ hipError_t launch_equalize(const T* img, int64_t sy, int64_t sx, int32_t ny, int
                            int32_t nbins, T* out, void* scratch, hipStream_t stream) {
   const int64_t n = static_cast<int64_t>(ny) * nx;
   auto* st = static_cast<EqState<T>*>(scratch);
-  auto* hist = reinterpret_cast<uint32_t*>(static_cast<char*>(scratch) +
-                                           ((sizeof(EqState<T>) + 255) & ~size_t{255}));
-  const int init_blocks = static_cast<int>((nbins + kThreads - 1) / kThreads > 1024
-                                               ? 1024
-                                               : (nbins + kThreads - 1) / kThreads);
-  hipLaunchKernelGGL(lic_eq_init<T>, dim3(init_blocks < 1 ? 1 : init_blocks), dim3(kThreads), 0,
-                     stream, st, hist, nbins);
+  auto* hist = reinterpret_cast<uint32_t*>(static_cast<char*>(scratch) + counters_offset<T>());
+  launch_range<T>(img, n, nx, sy, sx, nbins, st, hist, stream);
   const int g = grid_for(n, 8);
-  hipLaunchKernelGGL(lic_eq_range<T>, dim3(g), dim3(kThreads), 0, stream, img, n, nx, sy, sx, st);
-  // LDS histograms cost nbins of initialisation and merging per block:
-  // fewer, longer blocks when nbins is large
-  const int gh = grid_for(n, nbins <= 1024 ? 8 : 2);
-  if (nbins <= kLdsBins) {
-    hipLaunchKernelGGL((lic_eq_hist<T, true>), dim3(gh), dim3(kThreads), 0, stream, img, n, nx,
-                       sy, sx, nbins, st, hist);
-  } else {
-    hipLaunchKernelGGL((lic_eq_hist<T, false>), dim3(gh), dim3(kThreads), 0, stream, img, n, nx,
-                       sy, sx, nbins, st, hist);
-  }
+  launch_hist<T>(img, n, nx, sy, sx, nbins, st, hist, stream);
   hipLaunchKernelGGL(lic_eq_scan, dim3(1), dim3(kScanThreads), 0, stream, hist, nbins);
-  hipLaunchKernelGGL(lic_eq_map<T>, dim3(g), dim3(kThreads), 0, stream, img, n, nx, sy, sx, nbins,
-                     st, hist, out);
+  if (nbins <= kTableBins) {
+    hipLaunchKernelGGL((lic_eq_map<T, true>), dim3(g), dim3(kThreads), 0, stream, img, n, nx, sy,
+                       sx, nbins, st, hist, out);
+  } else {
+    hipLaunchKernelGGL((lic_eq_map<T, false>), dim3(g), dim3(kThreads), 0, stream, img, n, nx, sy,
+                       sx, nbins, st, hist, out);
+  }
   return hipGetLastError();
 }
 
@@ -507,17 +588,11 @@ hipError_t launch_equalize_tiles(int method, const T* img, int64_t sy, int64_t s
                                  void* scratch, int32_t lds_limit, hipStream_t stream) {
   const int64_t n = static_cast<int64_t>(ny) * nx;
   auto* st = static_cast<EqState<T>*>(scratch);
-  auto* hist = reinterpret_cast<uint32_t*>(static_cast<char*>(scratch) +
-                                           ((sizeof(EqState<T>) + 255) & ~size_t{255}));
+  auto* hist = reinterpret_cast<uint32_t*>(static_cast<char*>(scratch) + counters_offset<T>());
   char* extra = static_cast<char*>(scratch) +
                 ((equalize_scratch_bytes<T>(nbins) + 255) & ~size_t{255});
-  const int init_blocks = static_cast<int>((nbins + kThreads - 1) / kThreads > 1024
-                                               ? 1024
-                                               : (nbins + kThreads - 1) / kThreads);
-  hipLaunchKernelGGL(lic_eq_init<T>, dim3(init_blocks < 1 ? 1 : init_blocks), dim3(kThreads), 0,
-                     stream, st, hist, nbins);
+  launch_range<T>(img, n, nx, sy, sx, nbins, st, hist, stream);
   const int g = grid_for(n, 8);
-  hipLaunchKernelGGL(lic_eq_range<T>, dim3(g), dim3(kThreads), 0, stream, img, n, nx, sy, sx, st);
   if (method == kEqSlidingTile) {
     // a window taller than 2 ny - 1 rows covers the image from every pixel,
     // as one of exactly 2 ny - 1 does (likewise for columns)
@@ -549,15 +624,11 @@ hipError_t launch_equalize_tiles(int method, const T* img, int64_t sy, int64_t s
                     tiles_along(nx, std::min(tw, nx))};
   const int32_t tiles = tg.tiles_y * tg.tiles_x;
   auto* tcdf = reinterpret_cast<uint32_t*>(extra);
-  const int gh = grid_for(n, nbins <= 1024 ? 8 : 2);
+  launch_hist<T>(img, n, nx, sy, sx, nbins, st, hist, stream);
   if (nbins <= kLdsBins) {
-    hipLaunchKernelGGL((lic_eq_hist<T, true>), dim3(gh), dim3(kThreads), 0, stream, img, n, nx,
-                       sy, sx, nbins, st, hist);
     hipLaunchKernelGGL((lic_eq_tile_hist<T, true>), dim3(tiles), dim3(kThreads), 0, stream, img,
                        ny, nx, sy, sx, nbins, st, tg, tcdf);
   } else {
-    hipLaunchKernelGGL((lic_eq_hist<T, false>), dim3(gh), dim3(kThreads), 0, stream, img, n, nx,
-                       sy, sx, nbins, st, hist);
     const int64_t counters = static_cast<int64_t>(tiles) * nbins;
     hipLaunchKernelGGL(lic_eq_zero, dim3(grid_for(counters, 8)), dim3(kThreads), 0, stream, tcdf,
                        counters);
