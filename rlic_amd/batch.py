@@ -4,8 +4,8 @@
 its own size, kernel, boundaries, uv_mode and iteration count — through
 ``rlic_convolve_batch_*`` of ``librlic_hip.so``: fields of at least 2^18
 pixels run as single-field launches, all others together in one persistent
-launch fed by a device-side work queue, instead of one launch sequence per
-field.  Each result is bit-identical to the corresponding
+launch per pass fed by a device-side work queue, instead of one launch
+sequence per field.  Each result is bit-identical to the corresponding
 ``rlic_amd.convolve`` call.
 
 Fields may hold NumPy arrays (uploaded to ``device`` and returned as NumPy)

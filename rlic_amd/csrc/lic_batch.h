@@ -17,6 +17,7 @@ namespace rlic {
 struct BatchScratch {
   void* ptr = nullptr;
   hipStream_t stream = nullptr;
+  std::vector<char> host;  // launch_queue's descriptors in upload
   BatchScratch() = default;
   BatchScratch(const BatchScratch&) = delete;
   BatchScratch& operator=(const BatchScratch&) = delete;
@@ -56,7 +57,6 @@ struct Segment {
   int64_t item0;    // set by launch_queue
   int32_t field;
   int32_t pass;     // 0 traces from the cells, > 0 replays the move record
-  int32_t prev;     // segment whose items must all be done first (-1: none)
   int32_t record;   // pass 0: write the move record
   const void* src;  // replay input: the previous pass's output
   void* dst;        // this pass's output
@@ -64,14 +64,15 @@ struct Segment {
 
 // Pads every field's kernel weights (kernel_src[k], device memory) into a
 // weight pool, packs every field's (texture, u, v) into its cells when
-// `pack`, then runs the items of every segment in one persistent launch.
-// With `deps`, the items of a segment wait for segment `prev`, which must
-// come earlier in `segs`; without, no segment may have a `prev`.  Fills the
-// fields' and segments' launch_queue members and synchronizes `stream`.
+// `pack`, then runs the segments in one launch, or with `by_pass` each run of
+// consecutive segments of one pass in a launch of its own, in order.  Fills
+// the fields' and segments' launch_queue members; everything is enqueued on
+// `stream`, nothing waited for: the caller keeps `host` (the descriptors
+// being uploaded) until the stream's work is done.
 template <typename T>
 int launch_queue(std::vector<BatchField<T>>& fields, const std::vector<const T*>& kernel_src,
-                 std::vector<Segment>& segs, bool deps, bool pack, int profile,
-                 hipStream_t stream, std::string& err);
+                 std::vector<Segment>& segs, bool pack, bool by_pass, int profile,
+                 hipStream_t stream, std::vector<char>& host, std::string& err);
 
 // The element checks of rlic.convolve (src/rlic/_lib.py:174, :194) for
 // one field or every field of a batch at once, on the device.
@@ -98,8 +99,8 @@ hipError_t launch_check_values(const CheckField<T>* table, const CheckPack<T>* p
                                int32_t nfields, int64_t max_pixels, uint32_t* flags,
                                hipStream_t stream);
 
-// Runs every field of the batch (already validated) in one persistent
-// launch; synchronizes `stream` before returning.
+// Enqueues every field of the batch (already validated) on `stream`, one
+// persistent launch per pass; `scratch` is in use until that work is done.
 template <typename T, typename FieldSpec>
 int batch_run(const FieldSpec* specs, int64_t nfields, int profile, hipStream_t stream,
               BatchScratch& scratch, std::string& err);

@@ -1,20 +1,21 @@
-// Many fields in one persistent launch from a device work queue.
+// Many fields per launch from a device work queue.
 //
 // Each field is one `rlic.convolve` call (src/lib.rs:408-443) with its own
 // size, kernel, boundaries, uv_mode and iteration count.  Work items are
 // square pixel regions of one pass of one field; a segment is the run of
-// items of one (field, pass).  The waves of a persistent grid pop items from
-// one atomic counter.  Pass 0 traces the streamlines from the packed cells
-// (and records the moves when more passes follow); later passes replay the
-// moves with gathers through L2.
+// items of one (field, pass).  A launch runs the segments of one pass of
+// every field that has one: the waves of a persistent grid take an item each
+// and then pop items from one atomic counter.  Pass 0 traces the streamlines
+// from the packed cells (and records the moves when more passes follow);
+// later passes replay the moves with gathers through L2.
 //
-// The batched call queues every pass of every field in one launch,
-// pass-major (every field's pass 0, then every field's pass 1, ...), and a
-// pass-p item waits until the field's pass p-1 is complete.  The items it
-// waits for were queued earlier, so they were popped by waves that are
-// already running and whose own waits point further back: every wait ends
-// (a wait longer than a time limit still ends, and makes the call fail).
-// A serving step queues one pass of each active field, with no waits.
+// The batched call launches pass 0 of every field, then pass 1 of every field
+// that has one, and so on; a serving step is one such launch.  The launch
+// boundary orders a field's passes.  (All passes in one launch, items waiting
+// on done-counters for their field's previous pass, was slower: its waits
+// held the wave slots, its counters and the queue head were one contended
+// cache line each, and every published completion wrote back L2.  64 fields
+// of sides 32..256, up to 10 passes: 3.59 ms so, 1.42 ms now.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -30,9 +31,6 @@
 #include "lic_steps.h"
 
 namespace rlic {
-
-constexpr int32_t kPendSlots = 8;       // segments a wave holds unpublished counts for
-constexpr uint32_t kPublishItems = 32;  // completed items per release of a wave
 
 // Kernel weights of every field into its zero-padded slot (one block per field).
 template <typename T>
@@ -81,10 +79,6 @@ __global__ __launch_bounds__(256) void lic_pack_batch(const BatchField<T>* field
       f.cells, gi, gj, f.g,
       guarded_cell(f.tex, f.tsy, f.tsx, f.u, f.usy, f.usx, f.v, f.vsy, f.vsx, f.g, gi, gj),
       f.epoch);
-}
-
-__global__ void lic_zero_u32(uint32_t* p, int64_t n) {
-  for (int64_t t = blockIdx.x * 256 + threadIdx.x; t < n; t += gridDim.x * 256) p[t] = 0u;
 }
 
 template <typename T, bool FMA, bool BRANCHLESS, int POL, int REC, bool BUF>
@@ -167,81 +161,35 @@ __device__ __forceinline__ int64_t lane0_value(uint64_t x) {
   return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
-// Persistent kernel: every wave is an independent worker.  A wave pops one
-// work item (a square region of one pass of one field), waits if needed
-// (DEPS) for the segment it depends on, computes the region's pixels as
-// squares of 8 x 8 lanes, then (DEPS) counts the item done.  Regions are
-// 8 << sq_log2 pixels on a side (16, 32 or 64).  There is no block barrier
+// Persistent kernel: every wave is an independent worker.  A wave starts with
+// the item of its own number and then pops items from `queue` (the launch
+// sets it to 0; items up to the number of waves are taken without it), and
+// computes the item's region as squares of 8 x 8 lanes.  Regions are
+// 8 << sq_log2 pixels on a side (8, 16, 32 or 64).  There is no block barrier
 // in the loop, so waves of one block never wait for each other, and every
 // branch that steers the loop is wave-uniform.
-template <typename T, bool FMA, bool BRANCHLESS, bool BUF, bool DEPS>
+template <typename T, bool FMA, bool BRANCHLESS, bool BUF>
 __global__ __launch_bounds__(256) void lic_batch_persistent(const BatchField<T>* __restrict__ fields,
                                                             const Segment* __restrict__ segs,
                                                             const T* __restrict__ kpool,
-                                                            int32_t nsegs,
-                                                            int64_t total_items,
+                                                            int32_t nsegs, int64_t total_items,
                                                             unsigned long long* queue,
-                                                            uint32_t* done, uint32_t* failed,
-                                                            int64_t wait_ticks, int32_t sq_log2) {
+                                                            int32_t sq_log2) {
   __shared__ uint32_t delta_s[4][16];
   const int32_t lane = threadIdx.x & 63;
   uint32_t* delta = delta_s[threadIdx.x >> 6];
   const int32_t py = lane >> 3, px = lane & 7;  // replays: rows of the 8 x 8 square
   // traces: quads of lanes on 2 x 2 pixels of it (pixel_of_quads)
   const int32_t ty = ((lane >> 4) << 1) | ((lane >> 1) & 1), tx = ((lane >> 1) & 6) | (lane & 1);
-  // Completed items are published in batches: per-segment counts of up to
-  // kPendSlots segments are held by the wave and published together behind
-  // one release fence (the fence writes back L2, too costly per item) once
-  // kPublishItems items are pending, when a new segment finds no free slot,
-  // before the wave waits (so no wave waits while it holds unpublished
-  // work) and when the queue is drained.
-  int32_t pseg[kPendSlots] = {};
-  uint32_t pcnt[kPendSlots] = {};
-  int32_t npend = 0;
-  uint32_t pitems = 0;
-  int32_t fenced_prev = -1;  // segment whose completion the last acquire covered
-  auto publish = [&]() {
-    if (npend != 0) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-      __builtin_amdgcn_wave_barrier();
-      if (lane == 0) {
-#pragma unroll
-        for (int32_t k = 0; k < kPendSlots; ++k)
-          if (k < npend)
-            __hip_atomic_fetch_add(&done[pseg[k]], pcnt[k], __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-      }
-      npend = 0;
-      pitems = 0;
-    }
-  };
-  auto note_done = [&](int32_t sgi) {
-    bool found = false;
-#pragma unroll
-    for (int32_t k = 0; k < kPendSlots; ++k) {
-      if (k < npend && pseg[k] == sgi) {
-        pcnt[k] += 1u;
-        found = true;
-      }
-    }
-    if (!found) {
-      if (npend == kPendSlots) publish();
-#pragma unroll
-      for (int32_t k = 0; k < kPendSlots; ++k) {
-        if (k == npend) {
-          pseg[k] = sgi;
-          pcnt[k] = 1u;
-        }
-      }
-      ++npend;
-    }
-    if (++pitems >= kPublishItems) publish();
-  };
-  for (;;) {
-    uint64_t got = 0;
-    if (lane == 0) got = atomicAdd(queue, 1ull);
-    const int64_t item = lane0_value(got);
-    if (item >= total_items) break;  // the queue is drained
+  // blocks are dealt round-robin to the XCDs: the first items of an XCD's
+  // blocks are consecutive, so that a field's cells, record and texture are
+  // mostly in one XCD's L2
+  const int32_t blocks = gridDim.x, xcd = blockIdx.x & (kXcds - 1);
+  const int32_t first = xcd * (blocks / kXcds) + min(xcd, blocks % kXcds) +
+                        static_cast<int32_t>(blockIdx.x >> 3);
+  int64_t item = __builtin_amdgcn_readfirstlane(first * 4 + static_cast<int32_t>(threadIdx.x >> 6));
+  const int64_t waves = static_cast<int64_t>(blocks) * 4;
+  while (item < total_items) {
     int32_t lo = 0, hi = nsegs - 1;
     while (lo < hi) {
       const int32_t mid = (lo + hi + 1) >> 1;
@@ -249,37 +197,6 @@ __global__ __launch_bounds__(256) void lic_batch_persistent(const BatchField<T>*
     }
     const Segment seg = segs[lo];
     const BatchField<T>& f = fields[seg.field];
-    if (DEPS && seg.prev >= 0) {
-      // every item of this field's previous pass must be complete; those
-      // items were queued earlier, hence popped by running waves whose own
-      // waits point further back
-      auto complete = [&]() {
-        return __builtin_amdgcn_readfirstlane(__hip_atomic_load(
-                   &done[seg.prev], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >=
-               static_cast<uint32_t>(f.regions);
-      };
-      if (!complete()) {
-        publish();
-        const int64_t t0 = wall_clock64();
-        bool stuck = false;
-        while (!complete()) {
-          if (wall_clock64() - t0 > wait_ticks) {
-            stuck = true;
-            break;
-          }
-          __builtin_amdgcn_s_sleep(4);
-        }
-        if (stuck) {
-          if (lane == 0) atomicOr(failed, 1u);
-          break;
-        }
-        fenced_prev = -1;  // a completion newer than the last acquire
-      }
-      if (seg.prev != fenced_prev) {
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // see the previous pass's stores
-        fenced_prev = seg.prev;
-      }
-    }
     if (seg.pass > 0) {
       __builtin_amdgcn_wave_barrier();
       if (lane < 16) delta[lane] = move_delta(lane, f.g, BUF ? sizeof(T) : 1u);
@@ -308,23 +225,24 @@ __global__ __launch_bounds__(256) void lic_batch_persistent(const BatchField<T>*
       batch_replay_region<T, FMA, BUF>(f, kern, static_cast<const T*>(seg.src), dst, delta,
                                        i_base, j_base, sq_log2);
     }
-    if (DEPS) note_done(lo);
+    uint64_t got = 0;
+    if (lane == 0) got = atomicAdd(queue, 1ull);
+    item = waves + lane0_value(got);
   }
-  if (DEPS) publish();
 }
 
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
 
-template <typename T, bool DEPS>
+template <typename T>
 static const void* persistent_fn(int profile, bool buf) {
   const bool fma = profile & 1, bl = profile & 2;
 #define RLIC_PICK(BUF)                                                                           \
-  (fma && bl ? reinterpret_cast<const void*>(&lic_batch_persistent<T, true, true, BUF, DEPS>)    \
-   : fma     ? reinterpret_cast<const void*>(&lic_batch_persistent<T, true, false, BUF, DEPS>)   \
-   : bl      ? reinterpret_cast<const void*>(&lic_batch_persistent<T, false, true, BUF, DEPS>)   \
-             : reinterpret_cast<const void*>(&lic_batch_persistent<T, false, false, BUF, DEPS>))
+  (fma && bl ? reinterpret_cast<const void*>(&lic_batch_persistent<T, true, true, BUF>)          \
+   : fma     ? reinterpret_cast<const void*>(&lic_batch_persistent<T, true, false, BUF>)         \
+   : bl      ? reinterpret_cast<const void*>(&lic_batch_persistent<T, false, true, BUF>)         \
+             : reinterpret_cast<const void*>(&lic_batch_persistent<T, false, false, BUF>))
   return buf ? RLIC_PICK(true) : RLIC_PICK(false);
 #undef RLIC_PICK
 }
@@ -345,28 +263,50 @@ static int persistent_grid(const void* fn) {
 
 static size_t align_up(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
-// Work-item region side: RLIC_BATCH_REGION (16, 32 or 64), default 32.
-// Measured on the 512-field batches: 16 and 32 tie on small fields (sides
-// 32..256), 32 is 4% faster than 16 on large ones (sides 128..2048), 64 is
-// slower on both.
+// Work-item region side, as log2 of its 8-pixel squares: RLIC_BATCH_REGION
+// (8, 16, 32 or 64), else the largest of 32, 16 and 8 that gives the first
+// pass at least kWaveRounds items per resident wave: few fields need small
+// regions to reach every wave (64 fields of sides 32..256: 1.42 ms with 8,
+// 1.63 with 16, 3.43 with 32), many need few pops of the one queue head (512
+// such fields: 10.2, 8.6, 11.3 ms; 512 of sides 128..2048: 144, 131.5, 133).
+constexpr int64_t kWaveRounds = 4;
+
 template <typename T>
-static int32_t region_sq_log2(const std::vector<BatchField<T>>&) {
+static int64_t regions_of(const std::vector<BatchField<T>>& fields, int32_t sq_log2) {
+  const int64_t side = int64_t{8} << sq_log2;
+  int64_t n = 0;
+  for (const BatchField<T>& f : fields)
+    n += ((f.g.ny + side - 1) / side) * ((f.g.nx + side - 1) / side);
+  return n;
+}
+
+template <typename T>
+static int32_t region_sq_log2(const std::vector<BatchField<T>>& fields, int64_t waves) {
   const char* env = std::getenv("RLIC_BATCH_REGION");
-  const int side = (env && *env) ? std::atoi(env) : 32;
-  return side == 16 ? 1 : side == 64 ? 3 : 2;
+  if (env && *env) {
+    const int side = std::atoi(env);
+    return side == 8 ? 0 : side == 16 ? 1 : side == 64 ? 3 : 2;
+  }
+  for (int32_t sq = 2; sq > 0; --sq)
+    if (regions_of(fields, sq) >= kWaveRounds * waves) return sq;
+  return 0;
 }
 
 template <typename T>
 int launch_queue(std::vector<BatchField<T>>& fields, const std::vector<const T*>& kernel_src,
-                 std::vector<Segment>& segs, bool deps, bool pack, int profile,
-                 hipStream_t stream, std::string& err) {
+                 std::vector<Segment>& segs, bool pack, bool by_pass, int profile,
+                 hipStream_t stream, std::vector<char>& host, std::string& err) {
   const size_t nfields = fields.size();
   if (nfields == 0) return RLIC_OK;
-  const int32_t sq_log2 = region_sq_log2(fields);
+  bool buf = true;
+  for (const BatchField<T>& f : fields)
+    if (cell_slots(f.g) * static_cast<int64_t>(sizeof(Cell<T>)) > 0xFFFFFFFFll) buf = false;
+  const void* fn = persistent_fn<T>(profile, buf);
+  const int full_grid = persistent_grid(fn);
+  const int32_t sq_log2 = region_sq_log2(fields, int64_t{4} * full_grid);
   const int32_t region = 8 << sq_log2;
   // per-field regions, pack blocks and weight-pool slots
   int64_t pack_blocks = 0, pool_len = 0;
-  bool buf = true;
   for (BatchField<T>& f : fields) {
     f.regions_x = (f.g.nx + region - 1) / region;
     f.regions = f.regions_x * ((f.g.ny + region - 1) / region);
@@ -377,21 +317,29 @@ int launch_queue(std::vector<BatchField<T>>& fields, const std::vector<const T*>
       pack_blocks += static_cast<int64_t>((f.g.nx + 2 + 63) / 64) * ((f.g.ny + 2 + 3) / 4);
     f.kernel_off = pool_len + kKernelPad;
     pool_len += f.klen + 2 * kKernelPad;
-    if (cell_slots(f.g) * static_cast<int64_t>(sizeof(Cell<T>)) > 0xFFFFFFFFll)
-      buf = false;
   }
-  int64_t items = 0;
-  for (Segment& sg : segs) {
-    sg.item0 = items;
-    items += fields[sg.field].regions;
+  // the launches and their items, counted from 0
+  struct Launch {
+    size_t seg0, seg1;
+    int64_t items;
+  };
+  std::vector<Launch> launches;
+  for (size_t k = 0; k < segs.size(); ++k) {
+    if (launches.empty() || (by_pass && segs[k].pass != segs[k - 1].pass))
+      launches.push_back({k, k, 0});
+    Launch& l = launches.back();
+    segs[k].item0 = l.items;
+    l.items += fields[segs[k].field].regions;
+    l.seg1 = k + 1;
   }
-  // one scratch block: fields | kernel pointers | segments | counters | weight pool
+  // one scratch block: fields | kernel pointers | segments | queue heads
+  // (zeros) | weight pool; all but the pool uploaded in one copy
   const size_t off_fields = 0;
   const size_t off_kptrs = align_up(sizeof(BatchField<T>) * nfields);
   const size_t off_segs = align_up(off_kptrs + sizeof(const T*) * nfields);
-  const size_t off_done = align_up(off_segs + sizeof(Segment) * std::max<size_t>(segs.size(), 1));
-  const size_t n_counters = segs.size() + 4;  // done per segment, queue head (8 B), failure flag
-  const size_t off_pool = align_up(off_done + sizeof(uint32_t) * n_counters);
+  const size_t off_heads = align_up(off_segs + sizeof(Segment) * std::max<size_t>(segs.size(), 1));
+  const size_t off_pool =
+      align_up(off_heads + sizeof(unsigned long long) * std::max<size_t>(launches.size(), 1));
   const size_t bytes = off_pool + sizeof(T) * static_cast<size_t>(pool_len);
   CallScratch scratch;  // descriptors: reused from the per-stream cache
   if (hipError_t e = scratch.get(bytes, stream); e != hipSuccess) {
@@ -401,12 +349,12 @@ int launch_queue(std::vector<BatchField<T>>& fields, const std::vector<const T*>
   char* base = static_cast<char*>(scratch.ptr());
   T* d_pool = reinterpret_cast<T*>(base + off_pool);
   for (BatchField<T>& f : fields) f.kernel = d_pool + f.kernel_off;
-  std::vector<char> host(off_done);
+  host.assign(off_pool, 0);
   std::memcpy(host.data() + off_fields, fields.data(), sizeof(BatchField<T>) * nfields);
   std::memcpy(host.data() + off_kptrs, kernel_src.data(), sizeof(const T*) * nfields);
   if (!segs.empty())
     std::memcpy(host.data() + off_segs, segs.data(), sizeof(Segment) * segs.size());
-  hipError_t e = hipMemcpyAsync(base, host.data(), off_done, hipMemcpyHostToDevice, stream);
+  hipError_t e = hipMemcpyAsync(base, host.data(), off_pool, hipMemcpyHostToDevice, stream);
   if (e != hipSuccess) {
     err = std::string("uploading queue descriptors: ") + hipGetErrorString(e);
     return RLIC_ERR_HIP;
@@ -414,13 +362,8 @@ int launch_queue(std::vector<BatchField<T>>& fields, const std::vector<const T*>
   auto* d_fields = reinterpret_cast<const BatchField<T>*>(base + off_fields);
   auto* d_kptrs = reinterpret_cast<const T* const*>(base + off_kptrs);
   auto* d_segs = reinterpret_cast<const Segment*>(base + off_segs);
-  auto* d_done = reinterpret_cast<uint32_t*>(base + off_done);
-  auto* d_queue = reinterpret_cast<unsigned long long*>(d_done + segs.size() + (segs.size() & 1));
-  auto* d_failed = reinterpret_cast<uint32_t*>(d_queue + 1);
+  auto* d_heads = reinterpret_cast<unsigned long long*>(base + off_heads);
 
-  hipLaunchKernelGGL(lic_zero_u32, dim3(static_cast<unsigned>(std::min<size_t>(
-                                       (n_counters + 255) / 256, 1024))),
-                     dim3(256), 0, stream, d_done, static_cast<int64_t>(n_counters));
   hipLaunchKernelGGL(lic_pad_batch<T>, dim3(static_cast<unsigned>(nfields)), dim3(256), 0, stream,
                      d_fields, d_kptrs);
   if (pack && pack_blocks > 0) {
@@ -431,42 +374,21 @@ int launch_queue(std::vector<BatchField<T>>& fields, const std::vector<const T*>
     err = std::string("queue set-up kernels: ") + hipGetErrorString(e);
     return RLIC_ERR_HIP;
   }
-  if (items > 0) {
-    // four waves (workers) per block; with deps, a wait is declared stuck
-    // after RLIC_BATCH_WAIT_MS milliseconds (default 2000) of the device's
-    // wall clock
-    const void* fn = deps ? persistent_fn<T, true>(profile, buf) : persistent_fn<T, false>(profile, buf);
-    const int grid =
-        static_cast<int>(std::min<int64_t>((items + 3) / 4, persistent_grid(fn)));
-    int dev = 0, khz = 100000;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess ||
-        khz <= 0) {
-      (void)hipGetLastError();
-      khz = 100000;
-    }
-    const char* env = std::getenv("RLIC_BATCH_WAIT_MS");
-    const int64_t wait_ticks = (env ? std::max<int64_t>(0, std::atoll(env)) : 2000) * khz;
-    const int32_t nsegs = static_cast<int32_t>(segs.size());
-    int32_t sq = sq_log2;
-    void* args[] = {&d_fields, &d_segs, &d_pool, const_cast<int32_t*>(&nsegs), &items,
-                    &d_queue, &d_done, &d_failed, const_cast<int64_t*>(&wait_ticks), &sq};
+  for (size_t k = 0; k < launches.size(); ++k) {
+    const Launch& l = launches[k];
+    if (l.items == 0) continue;
+    // four waves (workers) per block
+    const int grid = static_cast<int>(std::min<int64_t>((l.items + 3) / 4, full_grid));
+    const Segment* first = d_segs + l.seg0;
+    int32_t nsegs = static_cast<int32_t>(l.seg1 - l.seg0), sq = sq_log2;
+    int64_t items = l.items;
+    unsigned long long* head = d_heads + k;
+    void* args[] = {&d_fields, &first, &d_pool, &nsegs, &items, &head, &sq};
     e = hipLaunchKernel(fn, dim3(grid), dim3(256), args, 0, stream);
     if (e != hipSuccess) {
       err = std::string("queue kernel: ") + hipGetErrorString(e);
       return RLIC_ERR_HIP;
     }
-  }
-  uint32_t failed = 0;
-  e = hipMemcpyAsync(&failed, d_failed, sizeof(failed), hipMemcpyDeviceToHost, stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(stream);
-  if (e != hipSuccess) {
-    err = std::string("queue completion: ") + hipGetErrorString(e);
-    return RLIC_ERR_HIP;
-  }
-  if (failed) {
-    err = "a work item waited too long for the previous pass of its field";
-    return RLIC_ERR_HIP;
   }
   return RLIC_OK;
 }
@@ -588,7 +510,6 @@ int batch_run(const FieldSpec* specs, int64_t nfields, int profile, hipStream_t 
   // n-1-p is even and the ping-pong partner otherwise, so the last pass
   // lands in `out`
   std::vector<Segment> segs;
-  std::vector<int32_t> last_seg(nfields, -1);
   for (int64_t pass = 0; pass < max_it; ++pass) {
     for (int64_t k = 0; k < nfields; ++k) {
       const FieldSpec& s = specs[k];
@@ -597,23 +518,22 @@ int batch_run(const FieldSpec* specs, int64_t nfields, int profile, hipStream_t 
       Segment sg{};
       sg.field = static_cast<int32_t>(k);
       sg.pass = static_cast<int32_t>(pass);
-      sg.prev = last_seg[k];
       sg.record = (pass == 0 && s.iterations > 1) ? 1 : 0;
       sg.src = pass > 0 ? buffer(pass - 1) : nullptr;
       sg.dst = buffer(pass);
-      last_seg[k] = static_cast<int32_t>(segs.size());
       segs.push_back(sg);
     }
   }
-  return launch_queue<T>(fields, ksrc, segs, /*deps=*/true, /*pack=*/true, profile, stream, err);
+  return launch_queue<T>(fields, ksrc, segs, /*pack=*/true, /*by_pass=*/true, profile, stream,
+                         scratch.host, err);
 }
 
 template int launch_queue<float>(std::vector<BatchField<float>>&, const std::vector<const float*>&,
                                  std::vector<Segment>&, bool, bool, int, hipStream_t,
-                                 std::string&);
+                                 std::vector<char>&, std::string&);
 template int launch_queue<double>(std::vector<BatchField<double>>&,
                                   const std::vector<const double*>&, std::vector<Segment>&, bool,
-                                  bool, int, hipStream_t, std::string&);
+                                  bool, int, hipStream_t, std::vector<char>&, std::string&);
 template hipError_t launch_check_values<float>(const CheckField<float>*, const CheckPack<float>*,
                                                int32_t, int64_t, uint32_t*, hipStream_t);
 template hipError_t launch_check_values<double>(const CheckField<double>*,

@@ -173,6 +173,7 @@ struct StepWork {
   std::vector<Segment> segs;
   std::vector<Resident<T>*> stepped, singles;
   std::vector<int64_t> handles, single_handles;
+  std::vector<char> host;  // descriptors in upload
 };
 
 template <typename T>
@@ -202,7 +203,6 @@ void Server::plan_dtype(StepWork<T>& w, std::vector<int64_t>& finished) {
     f.iterations = static_cast<int32_t>(std::min<int64_t>(r.target - r.done, INT32_MAX));
     Segment sg{};
     sg.field = static_cast<int32_t>(w.fields.size());
-    sg.prev = -1;
     const int out_buf = r.cur < 0 ? 0 : 1 - r.cur;
     sg.dst = r.buf[out_buf];
     if (r.done == 0) {
@@ -288,13 +288,16 @@ int Server::step(std::vector<int64_t>& finished, std::string& err) {
   int rc = launch_singles(w32, side, lane.data(), err);
   if (rc == RLIC_OK) rc = launch_singles(w64, side, lane.data() + w32.singles.size(), err);
   if (rc == RLIC_OK && !w32.fields.empty())
-    rc = launch_queue<float>(w32.fields, w32.ksrc, w32.segs, /*deps=*/false, /*pack=*/false,
-                             profile_, stream_, err);
+    rc = launch_queue<float>(w32.fields, w32.ksrc, w32.segs, /*pack=*/false,
+                             /*by_pass=*/false, profile_, stream_, w32.host, err);
   if (rc == RLIC_OK && !w64.fields.empty())
-    rc = launch_queue<double>(w64.fields, w64.ksrc, w64.segs, /*deps=*/false, /*pack=*/false,
-                              profile_, stream_, err);
-  if (rc != RLIC_OK) return rc;  // side work still running is waited for by ~SideWork
-  if (n_single > 0) {  // the step is synchronous
+    rc = launch_queue<double>(w64.fields, w64.ksrc, w64.segs, /*pack=*/false,
+                              /*by_pass=*/false, profile_, stream_, w64.host, err);
+  if (rc != RLIC_OK) {  // side work still running is waited for by ~SideWork
+    (void)hipStreamSynchronize(stream_);
+    return rc;
+  }
+  if (n_single > 0 || !w32.fields.empty() || !w64.fields.empty()) {  // the step is synchronous
     hipError_t e = side.join();
     if (hipError_t se = hipStreamSynchronize(stream_); e == hipSuccess) e = se;
     if (e != hipSuccess) {
