@@ -159,16 +159,35 @@ int env_int(const char* name, int dflt) {
 
 // How a call's passes 2..n replay: lds = 1, LDS-staged with a th x tw tile;
 // lds = 2, the hybrid (64 x 64 tiles, the first `band` steps of each
-// direction from an LDS box of that halo, the rest from the image); lds =
+// direction from an LDS box of that halo, the rest from the image), or with
+// 32 x 32 tiles boxes cut to the lines (launch_replay_box); lds =
 // 0, L2 gathers over a tile map (strip height `band`, wave shape).
 struct ReplayPlan {
   int32_t lds, th, tw, band, wave_w_log2;
 };
 
+constexpr ReplayPlan kBoxPlan{2, 32, 32, 0, 0};
+bool is_box_plan(const ReplayPlan& p) { return p.lds == 2 && p.th == 32; }
+
+// A field's move record: the codes, and the lines' bounds that the box plan
+// keeps (nullptr: no box plan) with whether they are filled.
+struct Record {
+  const uint4* codes;
+  rlic::ReplayBounds* bounds;
+  bool bounded;
+};
+
 template <typename T>
 hipError_t launch_plan(const ReplayPlan& p, const T* src, T* dst, const T* kernel, int32_t klen,
-                       const rlic::FieldGeom& g, int profile, const uint4* codes,
+                       const rlic::FieldGeom& g, int profile, Record& record,
                        hipStream_t stream) {
+  const uint4* codes = record.codes;
+  if (is_box_plan(p)) {
+    const hipError_t e = rlic::launch_replay_box<T>(src, kernel, klen, g, profile, dst, codes,
+                                                    record.bounds, !record.bounded, stream);
+    if (e == hipSuccess) record.bounded = true;
+    return e;
+  }
   if (p.lds == 2)
     return rlic::launch_replay_lds_hybrid<T>(src, kernel, klen, g, p.band, profile, dst, codes,
                                              stream);
@@ -214,15 +233,52 @@ int32_t hybrid_halo(int32_t klen, int64_t n) {
   return hybrid_allowed<T>(klen, n, halo) ? halo : 0;
 }
 
-// Default plan: the hybrid when it applies (kmid above its halo, an image
-// of at least 2^18 pixels), else the largest LDS tile whose whole box fits
-// (from 2^18 pixels), else L2 gathers over the tracing pass's tile map.  Measured per pass (4096^2 float,
+// Boxes cut to the lines (launch_replay_box), for a call that replays
+// `replays` passes.  A pass takes less the longer the kernel, but the first
+// also finds the boxes.  First and later passes, us, against the plans below:
+//   f32  4096^2      L=97  717, 303 vs 590, 382    L=129  758, 353 vs 692, 486
+//                    L=151 1082, 487 vs 1132, 830  L=201 1658, 969 vs 2173, 1643
+//        1600x1800   L=129 154, 91 vs 119, 97      L=151  240, 139 vs 222, 159
+//                    L=201 385, 255 vs 388, 309    L=257  487, 379 vs 542, 463
+//        512x513     L=151 46, 34 vs 61, 56        L=201  68, 55 vs 104, 96
+//   f64  2048^2      L=75  250, 104 vs 218, 120    L=101  310, 169 vs 309, 235
+//        1021x1537   L=101 121, 90 vs 136, 119     L=151  217, 158 vs 228, 206
+//        1600x1800   L=97  179, 103 vs 178, 122    L=257  706, 555 vs 781, 589
+// So from a half length of 72 (float) or 48 (double) with two passes to
+// replay, of 100 with one, and of 64 in float with four on a large image
+// (the whole box beside it is at its best there).  Not where the plans below
+// take one full round of the 256 CUs with their 64 x 64 tiles, their best
+// case (1024^2: L=151 87, 60 vs 67, 53; f64 L=201 216, 183 vs 191, 157; but
+// 1100^2, 324 tiles, 88, 66 vs 115, 101 and 243, 208 vs 300, 281).
+// RLIC_REPLAY_BOX = 0: never, 2: wherever they fit (tests).
+template <typename T>
+bool box_allowed(int32_t klen, const rlic::FieldGeom& g, int64_t replays) {
+  const int box = env_int("RLIC_REPLAY_BOX", 1);
+  if (box == 0 || replays < 1 || !rlic::box_replay_fits<T>(klen, g)) return false;
+  if (box == 2) return true;
+  const int64_t n = static_cast<int64_t>(g.ny) * g.nx;
+  if (!lds_allowed(n) || env_int("RLIC_REPLAY_LDS", 1) != 1 ||
+      env_int("RLIC_REPLAY_HYBRID", 1) != 1)
+    return false;
+  const int64_t tiles = ((int64_t{g.ny} + 63) / 64) * ((int64_t{g.nx} + 63) / 64);
+  if (tiles >= 192 && tiles <= 256) return false;
+  const int32_t kmid = klen / 2;
+  if (sizeof(T) == 4 && kmid >= 64 && replays >= 4 && n >= (int64_t{1} << 23)) return true;
+  return kmid >= (replays == 1 ? 100 : sizeof(T) == 4 ? 72 : 48);
+}
+
+// Default plan: boxes cut to the lines where box_allowed, else the hybrid
+// when it applies (kmid above its halo, an image of at least 2^18 pixels),
+// else the largest LDS tile whose whole box fits (from 2^18 pixels), else L2
+// gathers over the tracing pass's tile map.  Measured per pass (4096^2 float,
 // 2048^2 double): the hybrid beat every whole box, e.g. float L=135 0.59
 // vs 0.64 ms (64x64 box), L=151 0.76 vs 1.27 ms (32x32), double L=75 0.12
 // vs 0.15 ms (64x64): its box is smaller and only the last few steps of a
 // line leave it.
 template <typename T>
-ReplayPlan default_plan(int32_t klen, int64_t n) {
+ReplayPlan default_plan(int32_t klen, const rlic::FieldGeom& g, const Record& record) {
+  const int64_t n = static_cast<int64_t>(g.ny) * g.nx;
+  if (record.bounds) return kBoxPlan;  // only given where box_allowed
   if (const int32_t halo = hybrid_halo<T>(klen, n)) return {2, 64, 64, halo, 0};
   const rlic::LdsTile t = rlic::lds_replay_tile<T>(klen);
   if (lds_allowed(n) && t.h > 0) return {1, t.h, t.w, 0, 0};
@@ -279,7 +335,11 @@ void tuner_load_locked() {
 
 // A plan from the table is used only if it can run here.
 template <typename T>
-bool plan_usable(const ReplayPlan& p, int32_t klen, int64_t n) {
+bool plan_usable(const ReplayPlan& p, int32_t klen, const rlic::FieldGeom& g,
+                 const Record& record) {
+  const int64_t n = static_cast<int64_t>(g.ny) * g.nx;
+  if (is_box_plan(p))
+    return p.tw == 32 && record.bounds != nullptr && rlic::box_replay_fits<T>(klen, g);
   if (p.lds == 2) return p.th == 64 && p.tw == 64 && rlic::lds_hybrid_fits<T>(klen, n, p.band);
   if (p.lds) {
     const rlic::LdsTile big = rlic::lds_replay_tile<T>(klen);
@@ -303,8 +363,11 @@ void tuner_store_locked(const TuneKey& k, const TuneEntry& e) {
 }
 
 template <typename T>
-std::vector<ReplayPlan> replay_candidates(int32_t klen, int64_t n) {
+std::vector<ReplayPlan> replay_candidates(int32_t klen, const rlic::FieldGeom& g,
+                                          const Record& record) {
+  const int64_t n = static_cast<int64_t>(g.ny) * g.nx;
   std::vector<ReplayPlan> c;
+  if (record.bounds) c.push_back(kBoxPlan);
   const rlic::LdsTile big = rlic::lds_replay_tile<T>(klen);
   if (env_int("RLIC_REPLAY_LDS", 1) != 0 && big.h > 0) {
     if (big.h == 64) c.push_back({1, 64, 64, 0, 0});
@@ -321,16 +384,19 @@ std::vector<ReplayPlan> replay_candidates(int32_t klen, int64_t n) {
 template <typename T>
 hipError_t tune_replay(const std::vector<ReplayPlan>& cands, const T* src, T* dst,
                        const T* kernel, int32_t klen, const rlic::FieldGeom& g, int profile,
-                       const uint4* codes, hipStream_t stream, TuneEntry& best) {
+                       Record& record, hipStream_t stream, TuneEntry& best) {
   std::vector<hipEvent_t> ev(cands.size() + 1, nullptr);
   hipError_t e = hipSuccess;
   for (auto& x : ev)
     if (e == hipSuccess) e = hipEventCreate(&x);
+  // a record's first launch of the box plan also finds the bounds: not timed
+  if (!cands.empty() && is_box_plan(cands[0]) && !record.bounded && e == hipSuccess)
+    e = launch_plan<T>(cands[0], src, dst, kernel, klen, g, profile, record, stream);
   if (e == hipSuccess) e = hipEventRecord(ev[0], stream);
   for (size_t k = 0; k < cands.size() && e == hipSuccess; ++k) {
     {
       LaunchTimer timer(plan_kernel_name(cands[k]), stream);
-      e = launch_plan<T>(cands[k], src, dst, kernel, klen, g, profile, codes, stream);
+      e = launch_plan<T>(cands[k], src, dst, kernel, klen, g, profile, record, stream);
     }
     if (e == hipSuccess) e = hipEventRecord(ev[k + 1], stream);
   }
@@ -357,10 +423,11 @@ struct ReplayKey {
   const void* b;
   const void* kernel;
   const void* codes;
+  const void* bounds;
   int32_t klen;
   rlic::FieldGeom g;
   ReplayPlan plan;
-  int32_t profile, pad;  // pad: no implicit padding bytes (compared with memcmp)
+  int32_t profile;  // no implicit padding bytes: compared with memcmp
   int64_t iterations;
   bool operator<(const ReplayKey& o) const { return std::memcmp(this, &o, sizeof(*this)) < 0; }
 };
@@ -376,13 +443,13 @@ GraphCache g_graphs;
 
 template <typename T>
 hipError_t launch_replays(const ReplayPlan& plan, const T* kernel, int32_t klen,
-                          const rlic::FieldGeom& g, int profile, T* a, T* b, const uint4* codes,
+                          const rlic::FieldGeom& g, int profile, T* a, T* b, Record record,
                           int64_t first, int64_t iterations, hipStream_t stream) {
   // pass `it` (1-based) reads A when even, B when odd, and writes the other
   for (int64_t it = first; it <= iterations; ++it) {
     const T* src = (it % 2 == 0) ? a : b;
     T* dst = (it % 2 == 0) ? b : a;
-    const hipError_t e = launch_plan<T>(plan, src, dst, kernel, klen, g, profile, codes, stream);
+    const hipError_t e = launch_plan<T>(plan, src, dst, kernel, klen, g, profile, record, stream);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -392,7 +459,7 @@ hipError_t launch_replays(const ReplayPlan& plan, const T* kernel, int32_t klen,
 // available here (the caller then launches the passes directly).
 template <typename T>
 bool replay_graph(int device, const ReplayPlan& plan, const T* kernel, int32_t klen,
-                  const rlic::FieldGeom& g, int profile, T* a, T* b, const uint4* codes,
+                  const rlic::FieldGeom& g, int profile, T* a, T* b, const Record& record,
                   int64_t iterations, hipStream_t stream) {
   if (device < 0 || device >= 256) return false;
   ReplayKey key;
@@ -402,7 +469,8 @@ bool replay_graph(int device, const ReplayPlan& plan, const T* kernel, int32_t k
   key.a = a;
   key.b = b;
   key.kernel = kernel;
-  key.codes = codes;
+  key.codes = record.codes;
+  key.bounds = record.bounds;
   key.klen = klen;
   key.g = g;
   key.plan = plan;
@@ -426,7 +494,7 @@ bool replay_graph(int device, const ReplayPlan& plan, const T* kernel, int32_t k
       (void)hipGetLastError();
       return false;
     }
-    const hipError_t le = launch_replays<T>(plan, kernel, klen, g, profile, a, b, codes, 2,
+    const hipError_t le = launch_replays<T>(plan, kernel, klen, g, profile, a, b, record, 2,
                                             iterations, cap);
     const hipError_t ce = hipStreamEndCapture(cap, &graph);
     if (le != hipSuccess || ce != hipSuccess || !graph ||
@@ -462,7 +530,7 @@ bool replay_graph(int device, const ReplayPlan& plan, const T* kernel, int32_t k
 // image).  `codes` is where the move record starts; `codes + code_bytes`
 // is the whole block with the record, `codes` without it.
 struct ScratchLayout {
-  size_t cells, tmp, codes, code_bytes;
+  size_t cells, tmp, codes, code_bytes, bounds_bytes;  // bounds after the record
 };
 
 template <typename T>
@@ -476,6 +544,7 @@ ScratchLayout scratch_layout(const rlic::FieldGeom& g, int32_t klen, bool need_t
   l.codes = l.tmp + (need_tmp ? up(sizeof(T) * n) : 0);
   // code_chunks(klen) 16-byte chunks per pixel
   l.code_bytes = sizeof(uint4) * static_cast<size_t>(rlic::code_chunks(klen)) * n;
+  l.bounds_bytes = rlic::replay_bounds_bytes(g);
   return l;
 }
 
@@ -556,7 +625,7 @@ int run_on_device(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
     if (replay && off_codes + code_bytes > fixed->bytes) replay = false;  // trace every pass
     base = static_cast<char*>(fixed->ptr);
   } else {
-    hipError_t ae = scratch.get(off_codes + (replay ? code_bytes : 0), stream);
+    hipError_t ae = scratch.get(off_codes + (replay ? code_bytes + lay.bounds_bytes : 0), stream);
     if (ae != hipSuccess && replay) {  // no room for the record: trace every pass
       (void)hipGetLastError();
       replay = false;
@@ -569,6 +638,12 @@ int run_on_device(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
   auto* c = reinterpret_cast<rlic::Cell<T>*>(base + off_cells);
   T* tmp = need_tmp ? reinterpret_cast<T*>(base + off_tmp) : nullptr;
   uint4* code_ptr = replay ? reinterpret_cast<uint4*>(base + off_codes) : nullptr;
+  const bool bounds = replay && box_allowed<T>(klen, g, iterations - 1) &&
+                      (!fixed || off_codes + code_bytes + lay.bounds_bytes <= fixed->bytes);
+  Record record{
+      code_ptr,
+      bounds ? reinterpret_cast<rlic::ReplayBounds*>(base + off_codes + code_bytes) : nullptr,
+      false};
   const uint32_t epoch = rlic::next_epoch();
   {
     // the cells and the padded weight copy in one launch
@@ -619,7 +694,7 @@ int run_on_device(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
     }
     if (iterations == 1) return RLIC_OK;  // recorded only for the statistics
     // the replay plan: tuned (see Tuner), or the default
-    ReplayPlan plan = default_plan<T>(klen, n);
+    ReplayPlan plan = default_plan<T>(klen, g, record);
     int64_t first = 2;
     if (env_int("RLIC_AUTOTUNE", 1) != 0 && iterations >= 3 && n >= (int64_t{1} << 18)) {
       // an allocation-free call uses a tuned plan when the table has one,
@@ -629,11 +704,11 @@ int run_on_device(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
       tuner_load_locked();
       auto hit = g_tuner.table.find(key);
       if (hit != g_tuner.table.end()) {
-        if (plan_usable<T>(hit->second.plan, klen, n)) plan = hit->second.plan;
+        if (plan_usable<T>(hit->second.plan, klen, g, record)) plan = hit->second.plan;
       } else if (!fixed) {
-        const std::vector<ReplayPlan> cands = replay_candidates<T>(klen, n);
+        const std::vector<ReplayPlan> cands = replay_candidates<T>(klen, g, record);
         TuneEntry best{plan, -1.f};
-        RLIC_HIP_TRY(tune_replay<T>(cands, a, b, kernel, klen, g, profile, codes, stream, best),
+        RLIC_HIP_TRY(tune_replay<T>(cands, a, b, kernel, klen, g, profile, record, stream, best),
                      "tuning the replay");
         tuner_store_locked(key, best);
         plan = best.plan;
@@ -643,13 +718,13 @@ int run_on_device(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
     // passes first..n: direct launches, or one captured graph with
     // RLIC_GRAPH=1 (measured no faster on MI355X: kept as an option)
     if (first == 2 && !fixed && env_int("RLIC_GRAPH", 0) != 0 &&
-        replay_graph<T>(dev, plan, kernel, klen, g, profile, a, b, codes, iterations, stream))
+        replay_graph<T>(dev, plan, kernel, klen, g, profile, a, b, record, iterations, stream))
       return RLIC_OK;
     for (int64_t it = first; it <= iterations; ++it) {
       const T* src = (it % 2 == 0) ? a : b;
       T* dst = (it % 2 == 0) ? b : a;
       LaunchTimer timer(plan_kernel_name(plan), stream);
-      RLIC_HIP_TRY(launch_plan<T>(plan, src, dst, kernel, klen, g, profile, codes, stream),
+      RLIC_HIP_TRY(launch_plan<T>(plan, src, dst, kernel, klen, g, profile, record, stream),
                    "replay");
     }
     return RLIC_OK;
@@ -1240,9 +1315,10 @@ namespace rlic {
 template <typename T>
 hipError_t replay_pass(const T* src, T* dst, const T* kernel, int32_t klen, const FieldGeom& g,
                        int profile, const uint4* codes, hipStream_t stream) {
-  const ReplayPlan plan = default_plan<T>(klen, static_cast<int64_t>(g.ny) * g.nx);
+  Record record{codes, nullptr, false};
+  const ReplayPlan plan = default_plan<T>(klen, g, record);
   LaunchTimer timer(plan_kernel_name(plan), stream);
-  return launch_plan<T>(plan, src, dst, kernel, klen, g, profile, codes, stream);
+  return launch_plan<T>(plan, src, dst, kernel, klen, g, profile, record, stream);
 }
 
 template hipError_t replay_pass<float>(const float*, float*, const float*, int32_t,

@@ -378,15 +378,6 @@ __device__ __forceinline__ double copy_sign_of(double x, double s) {
   const Words a = __builtin_bit_cast(Words, x), b = __builtin_bit_cast(Words, s);
   return __builtin_bit_cast(double, Words{a.lo, bitop3<0x78>(a.hi, b.hi, 0x80000000u)});
 }
-// word * 16 + the code bits of a step in its two low bits (y axis where `mx`
-// is clear, toward lower indices where `neg` is set, with FLIP clear); the
-// two bits above are left over from the masks.
-template <bool FLIP>
-__device__ __forceinline__ uint32_t push_code(uint32_t word, uint32_t neg, uint32_t mx) {
-  const uint32_t bits = bitop3<FLIP ? 0x1B : 0xB1>(neg, mx, 1u << 28);
-  return __builtin_amdgcn_alignbit(word, bits, 28);
-}
-
 // n / d correctly rounded, for n, d >= 0 within the ranges above and d > 0:
 // the refinement steps of the IEEE division (reciprocal, Newton, quotient,
 // exact remainder, correction: Markstein 1990) without its scaling and
@@ -515,24 +506,36 @@ __device__ __forceinline__ void store_guarded_cell(Cell<T>* __restrict__ cells, 
   if (velocity_wide(c.u) || velocity_wide(c.v)) *reinterpret_cast<uint32_t*>(cells) = epoch;
 }
 
-// Move codes recorded by the tracing pass (4 bits per step, 8 per word), a
-// bit field: kMoveMoved for a step to a neighbouring cell, plus kMoveAxisY
-// for a step along y (rows), kMoveNeg toward lower indices and kMoveEdge
-// when the step left the image (the boundary rule of that side then
-// applies); kMoveStay for no move and kMoveStop where the streamline ended
-// on a NaN vector (src/lib.rs:336-338).  Codes 1-6 do not occur.
+// Move codes recorded by the tracing pass (4 bits per step, 8 per word): a
+// step to a neighbouring cell along x, or with kMoveAxisY along y (rows),
+// toward higher indices or with kMoveNeg lower ones, with kMoveEdge when it
+// left the image over a periodic side; kMoveStay for no move (a zero vector,
+// or a step held at a closed side) and kMoveStop where the streamline ended
+// on a NaN vector (src/lib.rs:336-338).  A code without its lowest bit is a
+// byte selector of v_perm_b32: 0, 2, 4, 6 pick one of four 16-bit deltas, 8 the
+// sign byte of the first, which is zero (replay_box).
 enum : uint32_t {
-  kMoveStay = 0,
-  kMoveNeg = 1,
+  kMoveEdge = 1,
   kMoveAxisY = 2,
-  kMoveEdge = 4,
-  kMoveStop = 7,
-  kMoveMoved = 8,
-  kMoveXPlus = kMoveMoved,
-  kMoveXMinus = kMoveMoved | kMoveNeg,
-  kMoveYPlus = kMoveMoved | kMoveAxisY,
-  kMoveYMinus = kMoveMoved | kMoveAxisY | kMoveNeg
+  kMoveNeg = 4,
+  kMoveStay = 8,
+  kMoveStop = 9,
+  kMoveXPlus = 0,
+  kMoveXMinus = kMoveNeg,
+  kMoveYPlus = kMoveAxisY,
+  kMoveYMinus = kMoveAxisY | kMoveNeg
 };
+constexpr uint32_t kWordStay = 0x11111111u * kMoveStay;
+
+// word * 16 + a step's code: kMoveAxisY where `mx` is clear, kMoveNeg where
+// `neg` is set (with FLIP clear); the lowest and the highest bit of the code
+// are left over from the masks.
+template <bool FLIP>
+__device__ __forceinline__ uint32_t push_code(uint32_t word, uint32_t neg, uint32_t mx) {
+  static_assert(kMoveNeg == 4 && kMoveAxisY == 2, "bits 30 and 29 of the masks");
+  const uint32_t bits = bitop3<FLIP ? 0x1B : 0xB1>(neg, mx, 1u << 30);
+  return __builtin_amdgcn_alignbit(word, bits, 28);
+}
 
 // A word holds the codes of 8 consecutive steps, the first step in the top
 // nibble: step q in bits 28 - 4q .. 31 - 4q.  (The tracing pass shifts
@@ -544,7 +547,7 @@ __host__ __device__ inline uint32_t move_code(uint32_t word, int q) {
 
 // Bit 4k set where nibble k of `word` is the stop code.
 __host__ __device__ inline uint32_t stop_nibbles(uint32_t word) {
-  return ~(word >> 3) & (word >> 2) & (word >> 1) & word & 0x11111111u;
+  return (word >> 3) & word & 0x11111111u;
 }
 
 // Steps of a word before its first stop code (8 when it has none): with
@@ -567,19 +570,18 @@ __host__ __device__ inline bool group_has_stop(uint32_t word) {
 // Position change of each move code in `unit`s, added modulo 2^32
 // (positions are uint32_t).  `row` is the row length and `span_x`, `span_y`
 // the distance between opposite edge cells, all in units; a periodic edge
-// step jumps across the image, a closed one stays.
-__host__ __device__ inline uint32_t move_delta_units(uint32_t code, const FieldGeom& g,
-                                                     uint32_t unit, uint32_t row,
+// step jumps across the image.
+__host__ __device__ inline uint32_t move_delta_units(uint32_t code, uint32_t unit, uint32_t row,
                                                      uint32_t span_x, uint32_t span_y) {
   switch (code) {
     case kMoveXPlus: return unit;
     case kMoveXMinus: return 0u - unit;
     case kMoveYPlus: return row;
     case kMoveYMinus: return 0u - row;
-    case kMoveXPlus | kMoveEdge: return g.x_right ? 0u - span_x : 0u;
-    case kMoveXMinus | kMoveEdge: return g.x_left ? span_x : 0u;
-    case kMoveYPlus | kMoveEdge: return g.y_right ? 0u - span_y : 0u;
-    case kMoveYMinus | kMoveEdge: return g.y_left ? span_y : 0u;
+    case kMoveXPlus | kMoveEdge: return 0u - span_x;
+    case kMoveXMinus | kMoveEdge: return span_x;
+    case kMoveYPlus | kMoveEdge: return 0u - span_y;
+    case kMoveYMinus | kMoveEdge: return span_y;
     default: return 0u;
   }
 }
@@ -587,7 +589,7 @@ __host__ __device__ inline uint32_t move_delta_units(uint32_t code, const FieldG
 // Replay through the image itself: wraps jump across it.
 __host__ __device__ inline uint32_t move_delta(uint32_t code, const FieldGeom& g, uint32_t unit) {
   const uint32_t row = static_cast<uint32_t>(g.nx) * unit;
-  return move_delta_units(code, g, unit, row, static_cast<uint32_t>(g.nx - 1) * unit,
+  return move_delta_units(code, unit, row, static_cast<uint32_t>(g.nx - 1) * unit,
                           static_cast<uint32_t>(g.ny - 1) * row);
 }
 

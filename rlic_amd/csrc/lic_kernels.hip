@@ -16,6 +16,7 @@
 
 #include "lic_device.h"
 #include "lic_launch.h"
+#include "lic_lds.h"
 #include "lic_steps.h"
 
 namespace rlic {
@@ -309,65 +310,13 @@ inline size_t lds_replay_bytes(int32_t th, int32_t tw, int32_t halo, size_t elem
 // fits (hybrid_max_halo): 64 in float (192 x 200 x 4 B), 32 in double
 // (128 x 136 x 8 B).
 
-__device__ __forceinline__ int32_t wrap_index(int32_t c, int32_t n) {
-  c %= n;
-  return c < 0 ? c + n : c;
-}
-
 // Byte-offset change in the LDS box for one move code: in the box's
 // unwrapped coordinates a periodic edge step is an ordinary step.
-__device__ __forceinline__ int32_t lds_move(uint32_t c, const FieldGeom& g, int32_t row_bytes,
-                                            int32_t elem) {
-  if ((c & kMoveMoved) == 0) return 0;  // stay, stop (and the unused codes)
-  const bool y = (c & kMoveAxisY) != 0, neg = (c & kMoveNeg) != 0;
-  const bool per = y ? (neg ? g.y_left : g.y_right) : (neg ? g.x_left : g.x_right);
-  if ((c & kMoveEdge) != 0 && !per) return 0;  // a closed edge keeps the cell
-  const int32_t d = y ? row_bytes : elem;
-  return neg ? -d : d;
+__device__ __forceinline__ int32_t lds_move(uint32_t c, int32_t row_bytes, int32_t elem) {
+  if ((c & kMoveStay) != 0) return 0;  // stay, stop (and the unused codes)
+  const int32_t d = (c & kMoveAxisY) != 0 ? row_bytes : elem;
+  return (c & kMoveNeg) != 0 ? -d : d;
 }
-
-// A line's position while replaying: an LDS byte pointer into the staged
-// box (LdsWalk) or a byte offset into the image, read with buffer loads
-// (ImageWalk, the hybrid replay's steps past the box).  Either way each
-// step is one add of a pair-table delta.
-typedef const unsigned char __attribute__((address_space(3))) lds_byte;
-
-template <typename T>
-__device__ __forceinline__ T lds_value(lds_byte* at) {
-  typedef const T __attribute__((address_space(3))) lds_t;
-  return *reinterpret_cast<lds_t*>(at);
-}
-
-// kTableFirst: the replay loop reads the pair-table entries of all of a
-// lane's lines before their gathers (LDS gathers are short; the early table
-// reads hide their latency), or each line's just before its own gathers
-// (image gathers are long; fewer registers live).
-template <typename T>
-struct LdsWalk {
-  typedef lds_byte* Pos;
-  static constexpr bool kTableFirst = true;
-  __device__ __forceinline__ T operator()(Pos at) const { return lds_value<T>(at); }
-};
-
-template <typename T>
-struct ImageWalk {
-  typedef uint32_t Pos;
-  static constexpr bool kTableFirst = false;
-  __amdgpu_buffer_rsrc_t rsrc;  // the image, n elements with n * sizeof(T) < 2^32
-  // base and size pass through readfirstlane: the descriptor must be
-  // wave-uniform (scalar registers), which the compiler does not prove here
-  __device__ __forceinline__ ImageWalk(const T* base, int64_t n) {
-    const uint64_t b = reinterpret_cast<uint64_t>(base);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(b));
-    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(b >> 32));
-    const uint32_t bytes =
-        __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(n * static_cast<int64_t>(sizeof(T))));
-    rsrc = make_rsrc(reinterpret_cast<const void*>((uint64_t{hi} << 32) | lo), bytes);
-  }
-  __device__ __forceinline__ T operator()(Pos at) const {
-    return buf_load(rsrc, at, static_cast<T*>(nullptr));
-  }
-};
 
 // The 8 values one line reads over a group of 8 moves (`word`, one 4-bit
 // move code per step), advancing its position `at`.
@@ -398,7 +347,7 @@ __device__ __forceinline__ void replay_lines(
 #pragma unroll
   for (int e = 0; e < E; ++e)
     next[e] = (ch_begin < nchunks && alive[e]) ? codes[(c0 + ch_begin) * np + p[e]]
-                                               : make_uint4(0u, 0u, 0u, 0u);
+                                               : make_uint4(kWordStay, kWordStay, kWordStay, kWordStay);
   bool any_line = false;
 #pragma unroll
   for (int e = 0; e < E; ++e) any_line = any_line || alive[e];
@@ -426,7 +375,7 @@ __device__ __forceinline__ void replay_lines(
       bool full = lim >= 8;
 #pragma unroll
       for (int e = 0; e < E; ++e) {
-        word[e] = alive[e] ? words[e][g] : 0u;  // 0 = stay
+        word[e] = alive[e] ? words[e][g] : kWordStay;
         full = full && alive[e] && !group_has_stop(word[e]);
       }
       if (__builtin_amdgcn_ballot_w64(!full) == 0) {
@@ -514,8 +463,8 @@ __global__ __launch_bounds__(kLdsThreads) void lic_replay_lds(const T* __restric
   const int32_t row_bytes = stride * elem;
   if (tid < 256) {
     // a code byte holds two steps, the earlier in its high nibble
-    const int32_t lo = lds_move(tid >> 4, g, row_bytes, elem);
-    const int32_t hi = lds_move(tid & 15, g, row_bytes, elem);
+    const int32_t lo = lds_move(tid >> 4, row_bytes, elem);
+    const int32_t hi = lds_move(tid & 15, row_bytes, elem);
     pair_delta[tid] = make_int2(lo, hi);
     if constexpr (HYBRID) {
       pair_image[tid] = make_int2(static_cast<int32_t>(move_delta(tid >> 4, g, elem)),
@@ -670,9 +619,6 @@ __global__ __launch_bounds__(kLdsThreads) void lic_replay_lds(const T* __restric
 // ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
-
-// Buffer addressing covers arrays of fewer than 2^32 bytes.
-inline bool fits_buffer(int64_t bytes) { return bytes > 0 && bytes <= 0xFFFFFFFFll; }
 
 TileMap make_tile_map(int32_t ny, int32_t nx, int32_t band, int32_t wave_w_log2) {
   TileMap m;
@@ -866,14 +812,6 @@ hipError_t launch_record_stats(const uint4* codes, int32_t klen, const FieldGeom
   hipLaunchKernelGGL(lic_record_stats, dim3(m.n_tiles), dim3(kBlock), 0, stream, codes, klen, g,
                      m, stats);
   return hipGetLastError();
-}
-
-int32_t lds_replay_limit_bytes() {
-  int dev = 0, limit = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 0;
-  if (hipDeviceGetAttribute(&limit, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
-    return 0;
-  return limit;
 }
 
 template <typename T>

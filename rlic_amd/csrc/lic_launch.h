@@ -135,4 +135,21 @@ hipError_t launch_replay_lds_hybrid(const T* x, const T* kernel, int32_t klen, c
                                     int32_t halo, int profile, T* out, const uint4* codes,
                                     hipStream_t stream);
 
+// Replay from LDS boxes cut to the lines (lic_replay_box.hip): `bounds` holds
+// replay_bounds_bytes(g) bytes, which the launch with `first` (the first
+// replay of a record) fills and later ones read.  box_replay_fits: half
+// lengths up to 8000, an image below 4 GiB, LDS for two blocks.
+// Bounds: of a tile's lines in one direction, in unwrapped coordinates
+// relative to the tile, two 16-bit integers each (row, column).
+struct ReplayBounds {
+  int32_t lo, hi;
+};
+size_t replay_bounds_bytes(const FieldGeom& g);
+template <typename T>
+bool box_replay_fits(int32_t klen, const FieldGeom& g);
+template <typename T>
+hipError_t launch_replay_box(const T* x, const T* kernel, int32_t klen, const FieldGeom& g,
+                             int profile, T* out, const uint4* codes, ReplayBounds* bounds,
+                             bool first, hipStream_t stream);
+
 }  // namespace rlic

@@ -170,12 +170,19 @@ __device__ __forceinline__ uint64_t fast_group(
     keep_in_step(acc);
   }
   if constexpr (REC != 0) {
-    word = (word & 0x33333333u) | 0x11111111u * kMoveMoved;
+    word &= 0x11111111u * (kMoveNeg | kMoveAxisY);
     if (__builtin_amdgcn_ballot_w64(jumped != 0u) != 0) {  // uniform: some line left the image
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         keep_in_step(jump[q]);  // compared here, not before the branch
-        word |= jump[q] != 0u ? kMoveEdge << (28 - 4 * q) : 0u;
+        // a jump back to the cell the step came from (as long as the step:
+        // a closed side, or the only column or row of a periodic one) stays
+        const uint32_t far = min(jump[q], 0u - jump[q]);
+        const bool stays = far == sg.step_x || far == sg.near_y || far == sg.far_y;
+        const uint32_t low = 28 - 4 * q;
+        word = jump[q] == 0u ? word
+                             : (stays ? (word & ~(15u << low)) | (kMoveStay << low)
+                                      : word | (kMoveEdge << low));
       }
       keep_in_step(word);  // a branch, not selects
     }
@@ -213,7 +220,7 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
   bool live_now = false, moves_now = false;  // set before a chunk of the short path
   bool status_known = false;
   for (int32_t ch = 0; ch < nchunks; ++ch) {
-    uint32_t words[4] = {0u, 0u, 0u, 0u};
+    uint32_t words[4] = {kWordStay, kWordStay, kWordStay, kWordStay};
     bool any_alive = true;
     int g0 = 0;
     if (BRANCHLESS && fast) {  // uniform
@@ -251,13 +258,12 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
       }
       if (reported == 0) {
         if (m_moves != __builtin_amdgcn_ballot_w64(true)) {  // uniform
-          // a zero vector stays (code 0) and has added its cell's value at
+          // a zero vector stays and has added its cell's value at
           // every step; an ended line adds nothing and records stops
           acc = live_now ? acc : acc_0;
-          const uint32_t still = live_now ? 0u : 0x11111111u * kMoveStop;
+          const uint32_t still = live_now ? kWordStay : 0x11111111u * kMoveStop;
 #pragma unroll
-          for (int g = 0; g < 4; ++g)
-            words[g] = moves_now ? words[g] : (g < full ? still : 0u);
+          for (int g = 0; g < 4; ++g) words[g] = moves_now || g >= full ? words[g] : still;
         }
         if (full == 0) {
           status_known = false;  // the full rule runs next
@@ -347,6 +353,7 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
         const uint32_t dist_y = !PAIRS || odd == pos_y || sg.all_far != 0u ? far_y : near_y;
         const uint32_t step = xs ? (pos_x ? sg.step_x : 0u - sg.step_x)
                                  : (pos_y ? dist_y : 0u - dist_y);
+        const uint32_t from = row;
         const uint32_t at = moves ? row + step : row;
         const CellVal<T> cv = cell(at);
         const uint32_t jump = pad_bits(cv.pad);
@@ -359,31 +366,32 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
         pu = cv.u;
         pv = cv.v;
         if constexpr (rec) {
-          // The code's four bits (moved, edge, y axis, negative direction;
-          // the three low bits alone for the stop code) are combined from
-          // the step's comparisons as wave lane masks on the scalar unit,
-          // then shifted into the word one at a time with an add-with-carry
-          // (word = 2 * word + bit), so the group's first step ends in the
-          // top nibble (move_code).  A line that has ended stays on its NaN
-          // cell, so it records the stop code again at every later step;
-          // readers stop at the first one.
+          // The code's four bits (stay, negative direction, y axis, edge or
+          // stop) are combined from the step's comparisons as wave lane
+          // masks on the scalar unit, then shifted into the word one at a
+          // time with an add-with-carry (word = 2 * word + bit), so the
+          // group's first step ends in the top nibble (move_code).  A line
+          // that has ended stays on its NaN cell, so it records the stop
+          // code again at every later step; readers stop at the first one.
           const uint64_t m_stop = ~__builtin_amdgcn_ballot_w64(ordered);
-          const uint64_t m_nz = __builtin_amdgcn_ballot_w64(mu != T(0)) |
-                                __builtin_amdgcn_ballot_w64(mv != T(0));
+          const uint64_t m_stay = __builtin_amdgcn_ballot_w64(row == from);
           const uint64_t m_x = __builtin_amdgcn_ballot_w64(xs);
           const uint64_t m_edge = __builtin_amdgcn_ballot_w64(edge);
           const uint64_t m_neg = ~((m_x & __builtin_amdgcn_ballot_w64(pos_x)) |
                                    (~m_x & __builtin_amdgcn_ballot_w64(pos_y)));
-          word = carry_in_bit(word, m_nz & ~m_stop);
-          word = carry_in_bit(word, (m_nz & m_edge) | m_stop);
-          word = carry_in_bit(word, (m_nz & ~m_x) | m_stop);
-          word = carry_in_bit(word, (m_nz & m_neg) | m_stop);
+          word = carry_in_bit(word, m_stay);
+          word = carry_in_bit(word, m_neg & ~m_stay);
+          word = carry_in_bit(word, ~m_x & ~m_stay);
+          word = carry_in_bit(word, (m_edge & ~m_stay) | m_stop);
         }
         alive = live;
       }
       // a last group of fewer than 8 steps: its first step to the top
       // nibble, "stay" codes after its last
-      if (rec && nsteps - s0 < 8) word <<= 4 * (8 - (nsteps - s0));
+      if (rec && nsteps - s0 < 8) {
+        const int32_t spare = 4 * (8 - (nsteps - s0));
+        word = (word << spare) | (kWordStay >> (32 - spare));
+      }
       words[g] = word;
       any_alive = __builtin_amdgcn_ballot_w64(alive) != 0;
     }
@@ -418,7 +426,7 @@ __device__ __forceinline__ T replay_direction(T acc, uint32_t pos,
     for (int g = 0; g < 4; ++g) {
       const int32_t s0 = ch * kChunkSteps + 8 * g;
       if (s0 >= nsteps) break;  // uniform
-      const uint32_t word = alive ? words[g] : 0u;  // 0 = stay
+      const uint32_t word = alive ? words[g] : kWordStay;
       T kw[8];
 #pragma unroll
       for (int q = 0; q < 8; ++q)
