@@ -98,6 +98,32 @@ int rlic_convolve_f64(const double* texture, int64_t tex_sy, int64_t tex_sx,
                       double* out,
                       int location, int profile, void* stream);
 
+/* rlic_convolve_* on device arrays together with rlic_check_values_*: the
+ * checks run on the values that the call reads anyway.  *what = the bits of
+ * rlic_check_values_*; unless it is 0, `out` holds nothing of use.  Returns
+ * once the inputs are checked; the convolution may still be running on
+ * `stream`. */
+int rlic_convolve_checked_f32(const float* texture, int64_t tex_sy, int64_t tex_sx,
+                              const float* u, int64_t u_sy, int64_t u_sx,
+                              const float* v, int64_t v_sy, int64_t v_sx,
+                              int64_t ny, int64_t nx,
+                              const float* kernel, int64_t kernel_len,
+                              int uv_mode,
+                              int x_left, int x_right, int y_left, int y_right,
+                              int64_t iterations,
+                              float* out,
+                              int profile, void* stream, int* what);
+int rlic_convolve_checked_f64(const double* texture, int64_t tex_sy, int64_t tex_sx,
+                              const double* u, int64_t u_sy, int64_t u_sx,
+                              const double* v, int64_t v_sy, int64_t v_sx,
+                              int64_t ny, int64_t nx,
+                              const double* kernel, int64_t kernel_len,
+                              int uv_mode,
+                              int x_left, int x_right, int y_left, int y_right,
+                              int64_t iterations,
+                              double* out,
+                              int profile, void* stream, int* what);
+
 /* Allocation-free variant of rlic_convolve_f32 / _f64 for device arrays.
  * No counterpart in the reference: it is for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops,

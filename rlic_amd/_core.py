@@ -203,6 +203,42 @@ def _convolve_host_numpy(fn, dtype, arrays, mode, bounds, it, prof):
     return out
 
 
+def convolve_checked(texture, u, v, kernel, uv_mode, boundaries, iterations):
+    """``convolve_f32`` / ``convolve_f64`` on validated, non-empty tensors of
+    one ROCm device, at least one pass, together with the element checks
+    (``rlic_convolve_checked_*``): the output and (texture has a negative
+    element, kernel has a non-finite weight)."""
+    import torch
+
+    lib = _native.load()
+    fn = lib.rlic_convolve_checked_f32 if texture.dtype == torch.float32 \
+        else lib.rlic_convolve_checked_f64
+    mode = _mode_code(uv_mode)
+    xl, xr, yl, yr = _bound_codes(boundaries)
+    it = _check_iterations(iterations)
+    kernel = kernel.contiguous()
+    ny, nx = texture.shape
+    device = texture.device
+    what = ctypes.c_int(0)
+    with torch.cuda.device(device):
+        out = torch.empty((ny, nx), dtype=texture.dtype, device=device)
+        stream = torch.cuda.current_stream(device).cuda_stream
+        status = fn(
+            texture.data_ptr(), texture.stride(0), texture.stride(1),
+            u.data_ptr(), u.stride(0), u.stride(1),
+            v.data_ptr(), v.stride(0), v.stride(1),
+            ny, nx,
+            kernel.data_ptr(), kernel.shape[0],
+            mode, xl, xr, yl, yr,
+            it,
+            out.data_ptr(),
+            DEFAULT_PROFILE, ctypes.c_void_p(stream), ctypes.byref(what),
+        )
+    if not what.value:
+        _native.raise_for_status(status)
+    return out, (bool(what.value & 1), bool(what.value & 2))
+
+
 def convolve_f32(texture, uv, kernel, boundaries, iterations=1, *, profile=None):
     """float32 line integral convolution (reference ``src/lib.rs:450-465``)."""
     return _convolve(

@@ -27,7 +27,7 @@ from typing import TYPE_CHECKING, Any
 import numpy as np
 
 from rlic_amd._boundaries import BoundarySet
-from rlic_amd._core import convolve_f32, convolve_f64
+from rlic_amd._core import convolve_checked, convolve_f32, convolve_f64
 
 if sys.version_info >= (3, 11):
     _ExceptionGroup = ExceptionGroup  # noqa: F821
@@ -219,6 +219,16 @@ def convolve(
       When more than one problem is found; all are reported.
     """
     texture, u, v, kernel = (_from_dlpack(a) for a in (texture, u, v, kernel))
+    if _checked_on_device(texture, u, v, kernel, uv_mode, boundaries, iterations):
+        bs = BoundarySet.from_spec(boundaries)
+        try:
+            out, flags = convolve_checked(texture, u, v, kernel, uv_mode, (bs.x, bs.y), iterations)
+        except (RuntimeError, MemoryError, ValueError):
+            # values are reported before what the device could not do
+            _raise_for_values(*_value_flags(texture, kernel))
+            raise
+        _raise_for_values(*flags)
+        return out
     bs, dtype = validate(
         texture, u, v, kernel=kernel, uv_mode=uv_mode, boundaries=boundaries, iterations=iterations
     )
@@ -227,6 +237,55 @@ def convolve(
 
     native = convolve_f32 if dtype == np.dtype("float32") else convolve_f64
     return native(texture, (u, v, uv_mode), kernel, (bs.x, bs.y), iterations)
+
+
+def _checked_on_device(texture, u, v, kernel, uv_mode, boundaries, iterations) -> bool:
+    """Whether nothing but the arrays' elements can be wrong, and the device
+    can check those while it convolves: non-empty float32 or float64 tensors
+    of fitting shapes on one ROCm device."""
+    if not (_is_torch(texture) and _is_torch(u) and _is_torch(v) and _is_torch(kernel)):
+        return False
+    dtype, device = texture.dtype, texture.device
+    if device.type != "cuda" or _np_dtype(texture) not in _SUPPORTED_DTYPES:
+        return False
+    for a in (u, v, kernel):
+        if a.dtype != dtype or a.device != device:
+            return False
+    shape = texture.shape
+    if len(shape) != 2 or u.shape != shape or v.shape != shape or kernel.dim() != 1:
+        return False
+    if not (shape[0] and shape[1] and kernel.shape[0]):
+        return False
+    if type(iterations) is not int or not 0 < iterations < 1 << 63:
+        return False
+    if uv_mode not in _KNOWN_UV_MODES:
+        return False
+    bs = BoundarySet.from_spec(boundaries)
+    return bs is not None and not bs.collect_exceptions()
+
+
+def _raise_for_values(neg_texture: bool, nonfinite_kernel: bool) -> None:
+    problems: list[Exception] = []
+    if neg_texture:
+        problems.append(_negative_texture())
+    if nonfinite_kernel:
+        problems.append(_non_finite_kernel())
+    _raise_problems(problems)
+
+
+def _negative_texture() -> Exception:
+    return ValueError("Found invalid texture element(s). Expected only positive values.")
+
+
+def _non_finite_kernel() -> Exception:
+    return ValueError("Found non-finite value(s) in kernel.")
+
+
+def _raise_problems(problems: list[Exception]) -> None:
+    if len(problems) == 1:
+        raise problems[0]
+    if problems:
+        raise _ExceptionGroup("Invalid inputs were received.", problems)
 
 
 def validate(texture, u, v, *, kernel, uv_mode, boundaries, iterations, check_values=True):
@@ -275,9 +334,7 @@ def validate(texture, u, v, *, kernel, uv_mode, boundaries, iterations, check_va
             ValueError(f"Expected a texture with exactly two dimensions. Got texture.ndim={texture.ndim}")
         )
     if neg_texture:
-        problems.append(
-            ValueError("Found invalid texture element(s). Expected only positive values.")
-        )
+        problems.append(_negative_texture())
     t_shape, u_shape, v_shape = _shape(texture), _shape(u), _shape(v)
     if u_shape != t_shape or v_shape != t_shape:
         problems.append(
@@ -291,7 +348,7 @@ def validate(texture, u, v, *, kernel, uv_mode, boundaries, iterations, check_va
             ValueError(f"Expected a kernel with exactly one dimension. Got kernel.ndim={kernel.ndim}")
         )
     if nonfinite_kernel:
-        problems.append(ValueError("Found non-finite value(s) in kernel."))
+        problems.append(_non_finite_kernel())
 
     bs = BoundarySet.from_spec(boundaries)
     if bs is None:
@@ -299,9 +356,6 @@ def validate(texture, u, v, *, kernel, uv_mode, boundaries, iterations, check_va
     else:
         problems.extend(bs.collect_exceptions())
 
-    if len(problems) == 1:
-        raise problems[0]
-    if problems:
-        raise _ExceptionGroup("Invalid inputs were received.", problems)
+    _raise_problems(problems)
     assert bs is not None
     return bs, dtypes[0]

@@ -95,6 +95,9 @@ SIGNATURES: dict[str, tuple[list, object]] = {
     "rlic_check_values_f64": ([_vp, _i64, _i64, _i64, _i64, _vp, _i64, _intp, _vp], _int),
     "rlic_convolve_f32": (_CONVOLVE_ARGTYPES, _int),
     "rlic_convolve_f64": (_CONVOLVE_ARGTYPES, _int),
+    # these take no `location` (device arrays only) and a result pointer
+    "rlic_convolve_checked_f32": (_CONVOLVE_ARGTYPES[:20] + _CONVOLVE_ARGTYPES[21:] + [_intp], _int),
+    "rlic_convolve_checked_f64": (_CONVOLVE_ARGTYPES[:20] + _CONVOLVE_ARGTYPES[21:] + [_intp], _int),
     # the allocation-free variants take no `location` (device arrays only)
     "rlic_convolve_noalloc_f32": (_CONVOLVE_ARGTYPES[:20] + _CONVOLVE_ARGTYPES[21:], _int),
     "rlic_convolve_noalloc_f64": (_CONVOLVE_ARGTYPES[:20] + _CONVOLVE_ARGTYPES[21:], _int),

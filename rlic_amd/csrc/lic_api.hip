@@ -555,6 +555,14 @@ struct FixedScratch {
   size_t bytes;
 };
 
+// The element checks of a call that computes at once (rlic_convolve_checked_*):
+// lic_pack sets the two host-mapped flags, and `packed` is recorded after it.
+struct ValueCheck {
+  uint32_t* dev_flags;
+  hipEvent_t packed;
+  bool recorded;
+};
+
 // The paired trace (two lanes per pixel, one per direction) where a field
 // has too few pixels to fill the GPU with lic_trace's one lane per pixel:
 // up to RLIC_TRACE_PAIR_MAX pixels (0: never), when it applies.
@@ -575,7 +583,7 @@ int run_on_device(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
                   const T* v, int64_t vsy, int64_t vsx, int32_t ny, int32_t nx,
                   const T* kernel, int32_t klen, int uv_mode, const rlic::FieldGeom& field,
                   int64_t iterations, T* out, int profile, hipStream_t stream,
-                  const FixedScratch* fixed = nullptr) {
+                  const FixedScratch* fixed = nullptr, ValueCheck* check = nullptr) {
   if (iterations == 0) {
     LaunchTimer timer("lic_copy2d", stream);
     RLIC_HIP_TRY(rlic::launch_copy2d<T>(tex, tsy, tsx, ny, nx, out, stream), "copy");
@@ -649,8 +657,13 @@ int run_on_device(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
     // the cells and the padded weight copy in one launch
     LaunchTimer timer("lic_pack", stream);
     RLIC_HIP_TRY(rlic::launch_pack<T>(tex, tsy, tsx, u, usy, usx, v, vsy, vsx, g, c, epoch,
-                                      stream, kernel, klen, kpad),
+                                      stream, kernel, klen, kpad,
+                                      check ? check->dev_flags : nullptr),
                  "pack");
+  }
+  if (check) {
+    check->recorded = true;  // also if the record fails: the caller then waits for the stream
+    RLIC_HIP_TRY(hipEventRecord(check->packed, stream), "recording the value checks");
   }
   kernel = kpad + pad;
   // trace tiles of 32 x 8 pixels (16 x 4 per wave) in XCD bands of 64
@@ -1044,7 +1057,8 @@ template <typename T>
 int convolve_entry(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t usy, int64_t usx,
                    const T* v, int64_t vsy, int64_t vsx, int64_t ny, int64_t nx, const T* kernel,
                    int64_t klen, int uv_mode, int xl, int xr, int yl, int yr, int64_t iterations,
-                   T* out, int location, int profile, void* stream_ptr) {
+                   T* out, int location, int profile, void* stream_ptr,
+                   ValueCheck* check = nullptr) {
   t_last_error.clear();
   if (ny < 0 || nx < 0) return set_error(RLIC_ERR_INVALID_ARGUMENT, "negative image size");
   if (klen < 0) return set_error(RLIC_ERR_INVALID_ARGUMENT, "negative kernel length");
@@ -1080,7 +1094,7 @@ int convolve_entry(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t u
   if (location == RLIC_DEVICE) {
     return run_on_device<T>(tex, tsy, tsx, u, usy, usx, v, vsy, vsx, static_cast<int32_t>(ny),
                             static_cast<int32_t>(nx), kernel, static_cast<int32_t>(klen),
-                            uv_mode, g, iterations, out, profile, stream);
+                            uv_mode, g, iterations, out, profile, stream, nullptr, check);
   }
 
   // Host arrays: upload the memory extent of each strided view, run, download.
@@ -1156,6 +1170,53 @@ int64_t server_field_bytes(int64_t ny, int64_t nx, int64_t klen, int keep, int64
 // convolve_entry with device arrays, its scratch in the fixed device array
 // (see rlic_convolve_noalloc_* below).
 int noalloc_scratch_ptr(void** ptr);
+
+// rlic_convolve_checked_*: the element checks and the convolution enqueued
+// together.  A check call of its own leaves the GPU idle while the host waits
+// for it and then launches (97 x 61 float: 41 us a call against 28; 256^2
+// double 48 against 28), and reads the texture once more.
+template <typename T>
+int convolve_checked_entry(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t usy,
+                           int64_t usx, const T* v, int64_t vsy, int64_t vsx, int64_t ny,
+                           int64_t nx, const T* kernel, int64_t klen, int uv_mode, int xl, int xr,
+                           int yl, int yr, int64_t iterations, T* out, int profile,
+                           void* stream_ptr, int* what) {
+  t_last_error.clear();
+  if (!what) return set_error(RLIC_ERR_INVALID_ARGUMENT, "null result pointer");
+  *what = 0;
+  hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
+  if (iterations <= 0 || ny <= 0 || nx <= 0 || klen <= 0 ||
+      capture != hipStreamCaptureStatusNone) {  // no pack to check in, or no waiting for it
+    if (const int rc = check_entry<T>(tex, ny, nx, tsy, tsx, kernel, klen, what, stream_ptr);
+        rc != RLIC_OK || *what != 0)
+      return rc;
+    return convolve_entry<T>(tex, tsy, tsx, u, usy, usx, v, vsy, vsx, ny, nx, kernel, klen,
+                             uv_mode, xl, xr, yl, yr, iterations, out, RLIC_DEVICE, profile,
+                             stream_ptr);
+  }
+  char* host = nullptr;
+  char* dev = nullptr;
+  RLIC_HIP_TRY(pinned_words(2 * sizeof(uint32_t), &host, &dev), "allocating the check flags");
+  std::memset(host, 0, 2 * sizeof(uint32_t));
+  ValueCheck check{reinterpret_cast<uint32_t*>(dev), nullptr, false};
+  RLIC_HIP_TRY(hipEventCreateWithFlags(&check.packed, hipEventDisableTiming),
+               "creating the check's event");
+  const int rc = convolve_entry<T>(tex, tsy, tsx, u, usy, usx, v, vsy, vsx, ny, nx, kernel, klen,
+                                   uv_mode, xl, xr, yl, yr, iterations, out, RLIC_DEVICE, profile,
+                                   stream_ptr, &check);
+  hipError_t e = hipSuccess;
+  if (check.recorded) {  // the flags are written until then
+    e = rc == RLIC_OK ? hipEventSynchronize(check.packed) : hipStreamSynchronize(stream);
+    const volatile uint32_t* flags = reinterpret_cast<uint32_t*>(host);
+    *what = (flags[0] ? 1 : 0) | (flags[1] ? 2 : 0);
+  }
+  (void)hipEventDestroy(check.packed);
+  if (rc == RLIC_OK) RLIC_HIP_TRY(e, "checking values");
+  return rc;
+}
+
 
 template <typename T>
 int convolve_noalloc_entry(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t usy,
@@ -1423,6 +1484,28 @@ int rlic_convolve_f64(const double* texture, int64_t tex_sy, int64_t tex_sx, con
   return convolve_entry<double>(texture, tex_sy, tex_sx, u, u_sy, u_sx, v, v_sy, v_sx, ny, nx,
                                 kernel, kernel_len, uv_mode, x_left, x_right, y_left, y_right,
                                 iterations, out, location, profile, stream);
+}
+
+int rlic_convolve_checked_f32(const float* texture, int64_t tex_sy, int64_t tex_sx, const float* u,
+                              int64_t u_sy, int64_t u_sx, const float* v, int64_t v_sy,
+                              int64_t v_sx, int64_t ny, int64_t nx, const float* kernel,
+                              int64_t kernel_len, int uv_mode, int x_left, int x_right, int y_left,
+                              int y_right, int64_t iterations, float* out, int profile,
+                              void* stream, int* what) {
+  return convolve_checked_entry<float>(texture, tex_sy, tex_sx, u, u_sy, u_sx, v, v_sy, v_sx, ny, nx,
+                                     kernel, kernel_len, uv_mode, x_left, x_right, y_left, y_right,
+                                     iterations, out, profile, stream, what);
+}
+
+int rlic_convolve_checked_f64(const double* texture, int64_t tex_sy, int64_t tex_sx, const double* u,
+                              int64_t u_sy, int64_t u_sx, const double* v, int64_t v_sy,
+                              int64_t v_sx, int64_t ny, int64_t nx, const double* kernel,
+                              int64_t kernel_len, int uv_mode, int x_left, int x_right, int y_left,
+                              int y_right, int64_t iterations, double* out, int profile,
+                              void* stream, int* what) {
+  return convolve_checked_entry<double>(texture, tex_sy, tex_sx, u, u_sy, u_sx, v, v_sy, v_sx, ny, nx,
+                                     kernel, kernel_len, uv_mode, x_left, x_right, y_left, y_right,
+                                     iterations, out, profile, stream, what);
 }
 
 int rlic_convolve_noalloc_f32(const float* texture, int64_t tex_sy, int64_t tex_sx,

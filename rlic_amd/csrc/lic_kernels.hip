@@ -29,7 +29,9 @@ namespace rlic {
 // Corner cells are never reached and stay zero.  With `kpad`, the same
 // launch also writes the padded weight copy [pad zeros][kernel][pad zeros]
 // (every thread of the grid takes a share), which saves a small field's
-// call one launch.
+// call one launch.  With `flags`, it also checks the values it reads anyway
+// (launch_check_values): flags[0] = 1 for a texture element below 0, flags[1]
+// = 1 for a non-finite weight.
 template <typename T>
 __global__ __launch_bounds__(256) void lic_pack(const T* __restrict__ tex, int64_t tsy,
                                                 int64_t tsx, const T* __restrict__ u,
@@ -38,7 +40,8 @@ __global__ __launch_bounds__(256) void lic_pack(const T* __restrict__ tex, int64
                                                 int64_t vsx, FieldGeom g,
                                                 Cell<T>* __restrict__ cells,
                                                 const T* __restrict__ kernel, int32_t klen,
-                                                T* __restrict__ kpad, uint32_t epoch) {
+                                                T* __restrict__ kpad, uint32_t epoch,
+                                                uint32_t* flags) {
   if (kpad) {
     const int64_t threads = static_cast<int64_t>(gridDim.x) * gridDim.y * 256;
     const int64_t total = int64_t{klen} + 2 * kKernelPad;
@@ -46,7 +49,9 @@ __global__ __launch_bounds__(256) void lic_pack(const T* __restrict__ tex, int64
                      threadIdx.x;
          t < total; t += threads) {
       const int64_t k = t - kKernelPad;
-      kpad[t] = (k >= 0 && k < klen) ? kernel[k] : T(0);
+      const T weight = (k >= 0 && k < klen) ? kernel[k] : T(0);
+      kpad[t] = weight;
+      if (flags && !__builtin_isfinite(weight)) flags[1] = 1u;
     }
   }
   int32_t gi, gj;
@@ -54,8 +59,9 @@ __global__ __launch_bounds__(256) void lic_pack(const T* __restrict__ tex, int64
   gi += blockIdx.y * 4;
   gj += blockIdx.x * 64;
   if (gi >= g.ny + 2 || gj >= g.nx + 2) return;
-  store_guarded_cell(cells, gi, gj, g,
-                     guarded_cell(tex, tsy, tsx, u, usy, usx, v, vsy, vsx, g, gi, gj), epoch);
+  const Cell<T> c = guarded_cell(tex, tsy, tsx, u, usy, usx, v, vsy, vsx, g, gi, gj);
+  store_guarded_cell(cells, gi, gj, g, c, epoch);
+  if (flags && c.x < T(0)) flags[0] = 1u;  // a guard cell holds an image cell's value
 }
 
 // The texture slot of every cell of the guarded array from the C-order
@@ -643,7 +649,7 @@ template <typename T>
 hipError_t launch_pack(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t usy,
                        int64_t usx, const T* v, int64_t vsy, int64_t vsx, const FieldGeom& g,
                        Cell<T>* cells, uint32_t epoch, hipStream_t stream, const T* kernel,
-                       int32_t klen, T* kpad) {
+                       int32_t klen, T* kpad, uint32_t* flags) {
   dim3 grid((g.nx + 2 + 63) / 64, (g.ny + 2 + 3) / 4);
   if (kpad) {  // enough threads for the weights of a long kernel on a small image
     const int64_t need = (int64_t{klen} + 2 * kKernelPad + 255) / 256;
@@ -652,7 +658,7 @@ hipError_t launch_pack(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64
                          (need + grid.y - 1) / grid.y, std::max<int64_t>(grid.x, 1024)));
   }
   hipLaunchKernelGGL(lic_pack<T>, grid, dim3(256), 0, stream, tex, tsy, tsx, u, usy, usx, v, vsy,
-                     vsx, g, cells, kernel, klen, kpad, epoch);
+                     vsx, g, cells, kernel, klen, kpad, epoch, flags);
   return hipGetLastError();
 }
 
@@ -957,7 +963,7 @@ hipError_t launch_replay_lds_hybrid(const T* x, const T* kernel, int32_t klen, c
 #define RLIC_INSTANTIATE(T)                                                                     \
   template hipError_t launch_pack<T>(const T*, int64_t, int64_t, const T*, int64_t, int64_t,   \
                                      const T*, int64_t, int64_t, const FieldGeom&, Cell<T>*,   \
-                                     uint32_t, hipStream_t, const T*, int32_t, T*);                      \
+                                     uint32_t, hipStream_t, const T*, int32_t, T*, uint32_t*);  \
   template hipError_t launch_repack_texture<T>(const T*, const FieldGeom&, Cell<T>*,           \
                                                hipStream_t);                                    \
   template hipError_t launch_copy2d<T>(const T*, int64_t, int64_t, int32_t, int32_t, T*,       \
