@@ -1375,17 +1375,24 @@ namespace rlic {
 
 template <typename T>
 hipError_t replay_pass(const T* src, T* dst, const T* kernel, int32_t klen, const FieldGeom& g,
-                       int profile, const uint4* codes, hipStream_t stream) {
-  Record record{codes, nullptr, false};
+                       int profile, const uint4* codes, ReplayBounds* bounds, bool& bounded,
+                       int64_t replays, hipStream_t stream) {
+  // with the bounds found, a pass alone decides: as one of many
+  const bool boxes = box_allowed<T>(klen, g, bounded ? INT32_MAX : replays);
+  Record record{codes, boxes ? bounds : nullptr, bounded};
   const ReplayPlan plan = default_plan<T>(klen, g, record);
   LaunchTimer timer(plan_kernel_name(plan), stream);
-  return launch_plan<T>(plan, src, dst, kernel, klen, g, profile, record, stream);
+  const hipError_t e = launch_plan<T>(plan, src, dst, kernel, klen, g, profile, record, stream);
+  bounded = record.bounded;
+  return e;
 }
 
 template hipError_t replay_pass<float>(const float*, float*, const float*, int32_t,
-                                       const FieldGeom&, int, const uint4*, hipStream_t);
+                                       const FieldGeom&, int, const uint4*, ReplayBounds*, bool&,
+                                       int64_t, hipStream_t);
 template hipError_t replay_pass<double>(const double*, double*, const double*, int32_t,
-                                        const FieldGeom&, int, const uint4*, hipStream_t);
+                                        const FieldGeom&, int, const uint4*, ReplayBounds*, bool&,
+                                        int64_t, hipStream_t);
 
 }  // namespace rlic
 

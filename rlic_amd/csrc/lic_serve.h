@@ -17,13 +17,17 @@ namespace rlic {
 // One replay pass (src -> dst along the move record `codes`) of a field as
 // a single-field launch with the default replay plan (LDS box, hybrid or L2
 // gathers; no tuning).  `kernel`: the first weight of a copy padded with
-// kernel_pad() zeros on each side.  Defined in lic_api.hip.
+// kernel_pad() zeros on each side.  `bounds` holds the lines' bounds of the
+// record once `bounded` (launch_replay_box), which the call sets where it fills
+// them; `replays`: how many passes, this one included, are known to replay.
+// Defined in lic_api.hip.
 template <typename T>
 hipError_t replay_pass(const T* src, T* dst, const T* kernel, int32_t klen, const FieldGeom& g,
-                       int profile, const uint4* codes, hipStream_t stream);
+                       int profile, const uint4* codes, ReplayBounds* bounds, bool& bounded,
+                       int64_t replays, hipStream_t stream);
 
 // Device state of one admitted field, in one allocation:
-// [padded weights | cells | buffer 0 | buffer 1 | move record].  The weights
+// [padded weights | cells | buffer 0 | buffer 1 | move record | its bounds].  The weights
 // are kept with kernel_pad() zeros on each side (the single-field replay
 // kernels read them so); `weights` points at the first weight.
 template <typename T>
@@ -42,10 +46,12 @@ struct Resident {
   Cell<T>* cells = nullptr;
   T* buf[2] = {nullptr, nullptr};
   uint4* codes = nullptr;  // nullptr: the field keeps no move record
+  ReplayBounds* bounds = nullptr;  // of the record's lines, filled once `bounded`
   int64_t done = 0;        // passes computed
   int64_t target = 0;      // passes requested so far
   int cur = -1;            // buffer holding the latest output (-1: none yet)
   bool recorded = false;   // `codes` holds the move record
+  bool bounded = false;    // `bounds` holds its lines' bounds
 };
 
 class Server {

@@ -122,8 +122,10 @@ int Server::admit(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
   r.bytes = bytes;
   choose_row_order<T>(r.g);
   // the charge counts the cells themselves, the block their slots as well
-  // (half a row pair more when ny is odd)
-  r.block_bytes = size_class(block_bytes<T>(cell_slots(r.g), ny, nx, klen, record));
+  // (half a row pair more when ny is odd) and 16 bytes a tile for the record's
+  // bounds
+  const size_t record_end = block_bytes<T>(cell_slots(r.g), ny, nx, klen, record);
+  r.block_bytes = size_class(record_end + (record ? replay_bounds_bytes(r.g) : 0));
   if (hipError_t e = take_block(bytes, r.block_bytes, &r.block); e != hipSuccess) {
     (void)hipGetLastError();
     err = std::string("allocating resident field: ") + hipGetErrorString(e);
@@ -142,6 +144,8 @@ int Server::admit(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
   r.buf[1] = reinterpret_cast<T*>(p);
   p += align256(sizeof(T) * n);
   r.codes = record ? reinterpret_cast<uint4*>(p) : nullptr;
+  r.bounds = record ? reinterpret_cast<ReplayBounds*>(static_cast<char*>(r.block) + record_end)
+                    : nullptr;
   r.target = iterations;
   // zeros on both sides of the weights (no graph captures this stream)
   hipError_t e = hipMemsetAsync(padded, 0, sizeof(T) * pad, stream_);
@@ -229,7 +233,8 @@ int Server::launch_singles(StepWork<T>& w, const SideWork& side, const int* lane
     Resident<T>* r = w.singles[k];
     const hipStream_t s = side.streams.empty() ? stream_ : side.streams[lane[k]];
     if (hipError_t e = replay_pass<T>(r->buf[r->cur], r->buf[1 - r->cur], r->weights, r->klen,
-                                      r->g, profile_, r->codes, s);
+                                      r->g, profile_, r->codes, r->bounds, r->bounded,
+                                      r->target - r->done, s);
         e != hipSuccess) {
       (void)hipGetLastError();
       err = std::string("replay pass: ") + hipGetErrorString(e);
