@@ -142,10 +142,12 @@ hipError_t launch_replay_lds_hybrid(const T* x, const T* kernel, int32_t klen, c
 // replay_bounds_bytes(g) bytes, which the launch with `first` (the first
 // replay of a record) fills and later ones read.  box_replay_fits: half
 // lengths up to 8000, an image below 4 GiB, LDS for two blocks.
-// Bounds: of a tile's lines in one direction, in unwrapped coordinates
-// relative to the tile, two 16-bit integers each (row, column).
+// What a tile stages for one direction: the bounds of a box in unwrapped
+// coordinates relative to the tile, two 16-bit integers each (row, column),
+// and the waves that read it.
 struct ReplayBounds {
   int32_t lo, hi;
+  uint32_t waves, unused;
 };
 size_t replay_bounds_bytes(const FieldGeom& g);
 template <typename T>

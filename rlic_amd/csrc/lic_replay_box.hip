@@ -5,7 +5,7 @@
 // direction, the rectangle that the tile's lines visit (in unwrapped
 // coordinates: a periodic edge is just crossed), then walks them there.  The
 // rectangles are known from the moves: the first replay of a record reads it
-// twice, once to find them, and stores them (16 bytes a tile) for the later
+// twice, once to find them, and stores them (32 bytes a tile) for the later
 // passes.
 //
 // Lines of a tile follow one flow, so the rectangle is far smaller than the
@@ -14,15 +14,19 @@
 // (53,800, which fits no LDS).  So long kernels replay from LDS too, and two
 // blocks of 70 KB fit a CU: one stages while the other walks.  Both
 // directions' boxes are staged at once if they fit together (L = 129: 83% of
-// the tiles), else one after the other; a direction whose box does not fit
-// (lines that part: 10% of the tiles at L = 201) gathers from the image.
+// the tiles), else one after the other.  Where a direction's box does not fit
+// (lines that part: 10% of the tiles at L = 201, 45% in double at 2048^2, L =
+// 151), the box of as many waves as fit is staged and the others gather from
+// the image beside them: a wave's 64 lines part far less than the tile's.
+// Against a tile gathering from the image as a whole: 4096^2 L = 201 969 ->
+// 700 us, L = 401 4610 -> 3107; 2048^2 double L = 151 323 -> 234.
 //
 // What bounds it: at 4096^2, L = 129, 353 us a pass, of which reading the
 // record alone takes 228 us (64 bytes a pixel); VALU and scalar issue are
 // each about 60% busy, LDS 45%.  Tried: two lines per lane, three blocks of
 // 50 KB (528 us; more tiles fall to the one-direction path), bounds per chunk
-// of 32 steps with runs of chunks that fit (masked 2111 x 1500, L = 201: 277
-// us against 285, for spilled registers and a larger record), bounds kept by
+// of 32 steps with runs of chunks that fit (for
+// spilled registers and a larger record), bounds kept by
 // the tracing pass (its step takes 12% longer, the two-way read 5-15% of a
 // replay).
 #include <algorithm>
@@ -180,16 +184,24 @@ __device__ __forceinline__ void dwords_to_lds(__amdgpu_buffer_rsrc_t rsrc, unsig
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void*)lds, 4, at, row, 0, 0);
 }
 
-// The box of a tile's lines in one direction: its origin relative to the
+// A box of lines in one direction: its origin relative to the
 // tile, its size, and the row stride it is staged with, in elements.
 struct Box {
   int32_t r_lo, c_lo, rows, columns, stride;
   __device__ __forceinline__ explicit Box(const Bounds& b)
       : r_lo(b.lo.x), c_lo(b.lo.y), rows(b.hi.x - b.lo.x + 1), columns(b.hi.y - b.lo.y + 1),
         stride(box_stride(columns)) {}
+  __device__ __forceinline__ int32_t elems() const { return rows * stride; }
 };
 
-// A tile's bounds in memory: of its forward, then of its backward lines; with
+// What a tile stages for its lines of one direction: a box and the waves that
+// it holds all lines of.
+struct Staged {
+  Bounds b;
+  uint32_t waves;
+};
+
+// A tile's boxes in memory: of its forward, then of its backward lines; with
 // FIRST the block finds and stores them.
 template <typename T, bool FMA, bool FIRST>
 __global__ __launch_bounds__(kBoxThreads, 8) void lic_replay_box(
@@ -220,7 +232,7 @@ __global__ __launch_bounds__(kBoxThreads, 8) void lic_replay_box(
     return;
   }
   ReplayBounds* const tile = bounds + 2 * (static_cast<int64_t>(ty) * m.tiles_x + tx);
-  Bounds both_ways[2];
+  Staged tiles[2];
   if constexpr (FIRST) {
     const uint4* record = codes + p;
     for (int32_t dir = 0; dir < 2; ++dir) {
@@ -243,31 +255,50 @@ __global__ __launch_bounds__(kBoxThreads, 8) void lic_replay_box(
       for (int off = 32; off > 0; off >>= 1)
         b = unite(b, {pair_of(__shfl_xor(bits_of(b.lo), off)),
                       pair_of(__shfl_xor(bits_of(b.hi), off))});
-      if (lane == 0) of_waves[wave][dir] = ReplayBounds{bits_of(b.lo), bits_of(b.hi)};
+      if (lane == 0) of_waves[wave][dir] = ReplayBounds{bits_of(b.lo), bits_of(b.hi), 0, 0};
     }
     __syncthreads();
 #pragma unroll
     for (int dir = 0; dir < 2; ++dir) {
-      Bounds b = no_bounds();
-      for (int32_t w = 0; w < kBoxWaves; ++w)
-        b = unite(b, {pair_of(of_waves[w][dir].lo), pair_of(of_waves[w][dir].hi)});
+      auto of_wave = [&](int32_t w) {
+        return Bounds{pair_of(__builtin_amdgcn_readfirstlane(of_waves[w][dir].lo)),
+                      pair_of(__builtin_amdgcn_readfirstlane(of_waves[w][dir].hi))};
+      };
       // to pixels, grown by 4 (LineBounds), to 16-byte aligned columns (stage)
-      b.lo = (b.lo >> static_cast<int16_t>(2)) - static_cast<int16_t>(4);
-      b.hi = (b.hi >> static_cast<int16_t>(2)) + static_cast<int16_t>(4);
-      b.lo.y &= ~3;
-      both_ways[dir] = b;
-      if (tid == 0) tile[dir] = ReplayBounds{bits_of(b.lo), bits_of(b.hi)};
+      auto in_pixels = [](Bounds b) {
+        b.lo = (b.lo >> static_cast<int16_t>(2)) - static_cast<int16_t>(4);
+        b.hi = (b.hi >> static_cast<int16_t>(2)) + static_cast<int16_t>(4);
+        b.lo.y &= ~3;
+        return b;
+      };
+      Bounds all = no_bounds();
+      for (int32_t w = 0; w < kBoxWaves; ++w) all = unite(all, of_wave(w));
+      tiles[dir] = {in_pixels(all), (1u << kBoxWaves) - 1};
+      if (Box(tiles[dir].b).elems() > box_elems) {  // uniform: one wave after the other, if it fits
+        Bounds some = no_bounds();
+        tiles[dir].waves = 0;
+        for (int32_t w = 0; w < kBoxWaves; ++w) {
+          const Bounds wider = unite(some, of_wave(w));
+          if (bits_of(of_wave(w).hi) == bits_of(no_bounds().hi) ||
+              Box(in_pixels(wider)).elems() > box_elems)
+            continue;
+          some = wider;
+          tiles[dir].waves |= 1u << w;
+        }
+        // no wave fits: nothing is staged, whatever the bounds
+        tiles[dir].b = in_pixels(tiles[dir].waves ? some : of_wave(0));
+      }
+      if (tid == 0)
+        tile[dir] = ReplayBounds{bits_of(tiles[dir].b.lo), bits_of(tiles[dir].b.hi),
+                                 tiles[dir].waves, 0};
     }
   } else {
-    both_ways[0] = {pair_of(tile[0].lo), pair_of(tile[0].hi)};
-    both_ways[1] = {pair_of(tile[1].lo), pair_of(tile[1].hi)};
+#pragma unroll
+    for (int dir = 0; dir < 2; ++dir)
+      tiles[dir] = {{pair_of(__builtin_amdgcn_readfirstlane(tile[dir].lo)),
+                     pair_of(__builtin_amdgcn_readfirstlane(tile[dir].hi))},
+                    static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(tile[dir].waves))};
   }
-  // every wave has the same bounds: what follows from them is uniform
-  auto uniform = [](const Bounds& b) {
-    return Bounds{pair_of(__builtin_amdgcn_readfirstlane(bits_of(b.lo))),
-                  pair_of(__builtin_amdgcn_readfirstlane(bits_of(b.hi)))};
-  };
-  const Bounds b_fwd = uniform(both_ways[0]), b_bwd = uniform(both_ways[1]);
   // Stages a box at element `first` of the dynamic LDS with direct memory ->
   // LDS loads, wrapped modulo the image size (one add or subtract where the
   // box lies within one image size of the image).  With x 16-byte aligned
@@ -387,7 +418,7 @@ __global__ __launch_bounds__(kBoxThreads, 8) void lic_replay_box(
   };
   auto direction = [&](auto forward, int32_t nsteps, const uint4* record, uint4 next,
                        const Box& box, bool fits, uint32_t lds) {
-    if (fits) {  // uniform; a lane past the image stays at the box's first element
+    if (fits) {  // uniform in the wave; a lane past the image stays at the box's first element
       const int32_t start = (py - box.r_lo) * box.stride + (px - box.c_lo);
       walk(forward, std::true_type{}, nsteps, record, next,
            lds + static_cast<uint32_t>(inside ? start * elem : 0), box.stride * elem);
@@ -396,29 +427,30 @@ __global__ __launch_bounds__(kBoxThreads, 8) void lic_replay_box(
     }
   };
 
-  const Box fwd(b_fwd), bwd(b_bwd);
-  const int32_t need_fwd = n_fwd > 0 ? fwd.rows * fwd.stride : 0, need_bwd = bwd.rows * bwd.stride;
+  const Box fwd(tiles[0].b), bwd(tiles[1].b);
+  const bool stage_fwd = n_fwd > 0 && tiles[0].waves != 0, stage_bwd = tiles[1].waves != 0;
+  const int32_t need_fwd = stage_fwd ? fwd.elems() : 0, need_bwd = stage_bwd ? bwd.elems() : 0;
   typedef unsigned char __attribute__((address_space(3))) lds_bytes;
   const uint32_t lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_bytes*)smem));
   const uint4* const rec_fwd = codes + p;
   const uint4* const rec_bwd = rec_fwd + static_cast<int64_t>(ch_fwd) * np;
   // Both directions' boxes at once (one wait, one barrier) if they fit
   // together, else one after the other.
-  const bool fits_fwd = need_fwd <= box_elems, fits_bwd = need_bwd <= box_elems;
   const bool both = need_fwd + need_bwd <= box_elems;
   const uint4 next_fwd = *rec_fwd, next_bwd = *rec_bwd;
   if (n_fwd > 0) {
-    if (fits_fwd) stage(fwd, 0);
-    if (both) stage(bwd, need_fwd);
+    if (stage_fwd) stage(fwd, 0);
+    if (both && stage_bwd) stage(bwd, need_fwd);
     staged();
-    direction(std::true_type{}, n_fwd, rec_fwd, next_fwd, fwd, fits_fwd, lds);
+    direction(std::true_type{}, n_fwd, rec_fwd, next_fwd, fwd,
+              (tiles[0].waves >> wave & 1) != 0, lds);
     if (!both) __syncthreads();  // the LDS is staged again next
   }
   if (!(both && n_fwd > 0)) {
-    if (fits_bwd) stage(bwd, 0);
+    if (stage_bwd) stage(bwd, 0);
     staged();
   }
-  direction(std::false_type{}, n_bwd, rec_bwd, next_bwd, bwd, fits_bwd,
+  direction(std::false_type{}, n_bwd, rec_bwd, next_bwd, bwd, (tiles[1].waves >> wave & 1) != 0,
             lds + static_cast<uint32_t>((both ? need_fwd : 0) * elem));
   if (inside) out[p] = acc;
 }

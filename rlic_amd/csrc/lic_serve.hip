@@ -122,7 +122,7 @@ int Server::admit(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
   r.bytes = bytes;
   choose_row_order<T>(r.g);
   // the charge counts the cells themselves, the block their slots as well
-  // (half a row pair more when ny is odd) and 16 bytes a tile for the record's
+  // (half a row pair more when ny is odd) and 32 bytes a tile for the record's
   // bounds
   const size_t record_end = block_bytes<T>(cell_slots(r.g), ny, nx, klen, record);
   r.block_bytes = size_class(record_end + (record ? replay_bounds_bytes(r.g) : 0));
