@@ -234,37 +234,33 @@ int32_t hybrid_halo(int32_t klen, int64_t n) {
 }
 
 // Boxes cut to the lines (launch_replay_box), for a call that replays
-// `replays` passes.  A pass takes less the longer the kernel, but the first
-// also finds the boxes.  First and later passes, us, against the plans below:
-//   f32  4096^2      L=97  717, 303 vs 590, 382    L=129  758, 353 vs 692, 486
-//                    L=151 1082, 487 vs 1132, 830  L=201 1658, 969 vs 2173, 1643
-//        1600x1800   L=129 154, 91 vs 119, 97      L=151  240, 139 vs 222, 159
-//                    L=201 385, 255 vs 388, 309    L=257  487, 379 vs 542, 463
-//        512x513     L=151 46, 34 vs 61, 56        L=201  68, 55 vs 104, 96
-//   f64  2048^2      L=75  250, 104 vs 218, 120    L=101  310, 169 vs 309, 235
-//        1021x1537   L=101 121, 90 vs 136, 119     L=151  217, 158 vs 228, 206
-//        1600x1800   L=97  179, 103 vs 178, 122    L=257  706, 555 vs 781, 589
-// So from a half length of 72 (float) or 48 (double) with two passes to
-// replay, of 100 with one, and of 64 in float with four on a large image
-// (the whole box beside it is at its best there).  Not where the plans below
-// take one full round of the 256 CUs with their 64 x 64 tiles, their best
-// case (1024^2: L=151 87, 60 vs 67, 53; f64 L=201 216, 183 vs 191, 157; but
-// 1100^2, 324 tiles, 88, 66 vs 115, 101 and 243, 208 vs 300, 281).
-// RLIC_REPLAY_BOX = 0: never, 2: wherever they fit (tests).
+// `replays` passes.  A pass takes less, but the first also finds the boxes.
+// First and later passes, us, against the plans below:
+//   f32  4096^2     L=65   486, 236 vs 346, 264    L=97   676, 297 vs 572, 373
+//                   L=129  774, 342 vs 646, 470    L=151 1032, 438 vs 1187, 817
+//                   L=201 1468, 700 vs 2180, 1616  L=401 4871, 3107 vs 6083, 4840
+//        2048^2     L=65   124, 62 vs 89, 69       L=113  220, 88 vs 173, 109
+//                   L=145  297, 126 vs 254, 161    L=151  347, 129 vs 312, 211
+//        1400x1300  L=97   77, 40 vs 64, 52        L=145  109, 56 vs 99, 79
+//        1024^2     L=129  56, 31 vs 45, 36        L=201  124, 65 vs 129, 103
+//        520x600    L=65   22, 11 vs 22, 19        L=145  42, 19 vs 49, 40
+//   f64  2048^2     L=49   161, 64 vs 107, 60      L=67   253, 91 vs 209, 117
+//                   L=97   281, 111 vs 253, 169    L=151  478, 234 vs 572, 434
+//        1400x1300  L=67   95, 48 vs 79, 59        L=113  131, 69 vs 135, 116
+//        520x600    L=67   32, 18 vs 36, 31        L=129  52, 37 vs 77, 70
+// so the fewer passes there are to pay for the first, the longer the kernel
+// must be.  RLIC_REPLAY_BOX = 0: never, 2: wherever they fit (tests).
 template <typename T>
 bool box_allowed(int32_t klen, const rlic::FieldGeom& g, int64_t replays) {
   const int box = env_int("RLIC_REPLAY_BOX", 1);
   if (box == 0 || replays < 1 || !rlic::box_replay_fits<T>(klen, g)) return false;
   if (box == 2) return true;
-  const int64_t n = static_cast<int64_t>(g.ny) * g.nx;
-  if (!lds_allowed(n) || env_int("RLIC_REPLAY_LDS", 1) != 1 ||
+  if (!lds_allowed(static_cast<int64_t>(g.ny) * g.nx) || env_int("RLIC_REPLAY_LDS", 1) != 1 ||
       env_int("RLIC_REPLAY_HYBRID", 1) != 1)
     return false;
-  const int64_t tiles = ((int64_t{g.ny} + 63) / 64) * ((int64_t{g.nx} + 63) / 64);
-  if (tiles >= 192 && tiles <= 256) return false;
   const int32_t kmid = klen / 2;
-  if (sizeof(T) == 4 && kmid >= 64 && replays >= 4 && n >= (int64_t{1} << 23)) return true;
-  return kmid >= (replays == 1 ? 100 : sizeof(T) == 4 ? 72 : 48);
+  if (sizeof(T) == 4) return kmid >= (replays == 1 ? 88 : replays < 4 ? 72 : replays < 8 ? 48 : 32);
+  return kmid >= (replays == 1 ? 56 : replays < 4 ? 48 : 33);
 }
 
 // Default plan: boxes cut to the lines where box_allowed, else the hybrid
