@@ -240,7 +240,7 @@ typedef struct {
 /* Batched convolution: n_fields independent rlic_convolve_* calls (device
  * memory only).  Fields of at least 2^18 pixels (RLIC_BATCH_SINGLE_MIN)
  * run as single-field launches; the rest run together in one persistent
- * launch fed by a device-side work queue.  Results are the same, bit for
+ * launch per pass, fed by a device-side work queue.  Results are the same, bit for
  * bit, as the single calls.  Returns after the work has completed on
  * `stream`.  No counterpart in the
  * reference (which has one call per field, src/lib.rs:450-482); each field

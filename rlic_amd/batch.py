@@ -1,4 +1,4 @@
-"""Many convolutions in one persistent GPU launch.
+"""Many convolutions in one persistent GPU launch a pass.
 
 ``convolve_batch(fields)`` runs one ``convolve`` per field — each field with
 its own size, kernel, boundaries, uv_mode and iteration count — through

@@ -8,8 +8,9 @@
 //      strided arrays (any strides, including transposed views);
 //   2. lic_trace runs pass 1 and, when more passes follow, records the move
 //      of every streamline step;
-//   3. lic_replay runs passes 2..n from the recorded moves, ping-ponging
-//      two device buffers so that the last pass lands in `out`.
+//   3. a replay plan (lic_replay_box, lic_replay_lds or lic_replay) runs
+//      passes 2..n from the recorded moves, ping-ponging two device buffers
+//      so that the last pass lands in `out`.
 // When the move record would not fit the memory budget, every pass is
 // traced again instead (texture slot re-packed between passes).
 #include <hip/hip_runtime.h>
@@ -969,7 +970,7 @@ int batch_entry(const FieldSpec* fields, int64_t nfields, int profile, void* str
   hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
   // Fields of at least RLIC_BATCH_SINGLE_MIN pixels (default 2^18; 0 or
   // less: none) run as single-field launches (trace, then LDS-staged or
-  // tuned replays); the rest share one persistent launch.  Either way a
+  // tuned replays); the rest share one persistent launch a pass.  Either way a
   // field gives the bits of its single call.
   const int single_min = env_int("RLIC_BATCH_SINGLE_MIN", 1 << 18);
   std::vector<FieldSpec> rest;

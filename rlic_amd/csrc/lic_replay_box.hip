@@ -201,6 +201,8 @@ struct Staged {
   uint32_t waves;
 };
 
+}  // namespace
+
 // A tile's boxes in memory: of its forward, then of its backward lines; with
 // FIRST the block finds and stores them.
 template <typename T, bool FMA, bool FIRST>
@@ -454,8 +456,6 @@ __global__ __launch_bounds__(kBoxThreads, 8) void lic_replay_box(
             lds + static_cast<uint32_t>((both ? need_fwd : 0) * elem));
   if (inside) out[p] = acc;
 }
-
-}  // namespace
 
 size_t replay_bounds_bytes(const FieldGeom& g) {
   const int64_t tiles = ((int64_t{g.ny} + kBoxTile - 1) / kBoxTile) *

@@ -1,5 +1,5 @@
 // Serving core (lic_serve.hip): fields resident in device memory, advanced
-// one pass per step, many fields per step in one persistent launch.
+// one pass per step, many fields per step in one persistent launch per dtype.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -4,10 +4,10 @@
 // copies its kernel weights and packs (u, v, texture) into device memory
 // that stays resident until the field is released; each step then runs one
 // pass of every field that has passes left, all fields of a dtype in one
-// persistent launch over square regions (launch_queue without waits: the
-// step boundary orders the passes), except the replay passes of fields of
-// at least 2^18 pixels, which run as single-field launches (LDS box or
-// hybrid replay, as a single convolve call would).  A field's first pass traces and, when
+// persistent launch over square regions (launch_queue; the step boundary
+// orders the passes), except the replay passes of fields of
+// at least 2^18 pixels, which run as single-field launches (boxes
+// cut to the lines, LDS box or hybrid replay, as a single convolve call would).  A field's first pass traces and, when
 // it keeps a move record, records the moves; later passes (and follow-up
 // passes requested after the field finished) replay them.  The two output
 // buffers alternate, so a field's passes give the same bits as one
