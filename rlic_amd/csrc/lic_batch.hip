@@ -93,7 +93,7 @@ __device__ __forceinline__ void batch_trace_pixel(const BatchField<T>& f,
   const int64_t p = static_cast<int64_t>(i0) * f.g.nx + j0;
   const uint32_t row0 = static_cast<uint32_t>(cell_slot(f.g, i0 + 1, j0 + 1));
   const CellVal<T> c0 = cell(row0);
-  const bool short_path = !wide_mark(f.cells, f.epoch);
+  bool short_path = !wide_mark(f.cells, f.epoch);
   T acc = macc<FMA>(kernel[kmid], c0.x, T(0));  // src/lib.rs:375-383
   acc = trace_direction<T, FMA, BRANCHLESS, POL, true, REC, BUF, true>(
       acc, c0.u, c0.v, row0, cell, kernel, kmid, n_fwd, sg, f.codes, np, p, 0, short_path);

@@ -111,7 +111,7 @@ __global__ __launch_bounds__(256) void lic_trace(const Cell<T>* __restrict__ cel
   const int64_t p = static_cast<int64_t>(i0) * g.nx + j0;
   const uint32_t row0 = static_cast<uint32_t>(cell_slot(g, i0 + 1, j0 + 1));
   const CellVal<T> c0 = cell(row0);
-  const bool short_path = !wide_mark(cells, epoch);
+  bool short_path = !wide_mark(cells, epoch);
   T acc = macc<FMA>(kernel[kmid], c0.x, T(0));  // src/lib.rs:375-383
   acc = trace_direction<T, FMA, BRANCHLESS, POL, true, REC, BUF, BUF>(
       acc, c0.u, c0.v, row0, cell, kernel, kmid, n_fwd, sg, codes, np, p, 0, short_path);
@@ -164,12 +164,13 @@ __global__ __launch_bounds__(64) void lic_trace_pair(
     const uint32_t row0 = static_cast<uint32_t>(cell_slot(g, i0 + 1, j0 + 1));
     const CellVal<T> c0 = cell(row0);
     acc = macc<FMA>(kernel[kmid], c0.x, T(0));  // src/lib.rs:375-383
+    bool short_path = !wide_mark(cells, epoch);
     // every lane stores (no branch in the step): forward lanes into the
     // spare row kmid
     auto keep = [&](int32_t s, T x) { vals[32 * (fwd ? kmid : s)] = x; };
     acc = trace_direction<T, FMA, BRANCHLESS, POL, true, REC, true, true, true>(
         acc, c0.u, c0.v, row0, cell, kernel, kmid, kmid, sg, codes, np, p,
-        fwd ? 0 : chunks_of(kmid), !wide_mark(cells, epoch), fwd, keep, &live_steps);
+        fwd ? 0 : chunks_of(kmid), short_path, fwd, keep, &live_steps);
   }
   __syncthreads();
   const int32_t nb = __shfl(live_steps, k + 32);  // the backward partner's

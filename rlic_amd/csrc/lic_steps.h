@@ -199,7 +199,7 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
                                              const T* __restrict__ kernel, int32_t kmid,
                                              int32_t nsteps, const StepGeom& sg,
                                              uint4* __restrict__ codes, int64_t np, int64_t p,
-                                             int32_t c0, bool short_path,
+                                             int32_t c0, bool& short_path,
                                              bool fwd_lane = true, Sink sink = Sink{},
                                              int32_t* live_steps = nullptr) {
   constexpr bool pol = POL != 0, rec = REC != 0;
@@ -213,9 +213,12 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
   // reported, the chunk is done again by the full rule.  Off for the rest of
   // the direction after a chunk that reports many lanes (a field of ties,
   // e.g. u = v everywhere) or a second chunk that reports any, so that such
-  // a line costs little more than the full rule alone.  (One saved state per
-  // chunk: saving it for every group cost 2 VALU instructions per step.)
-  bool fast = BRANCHLESS && short_path;
+  // a line costs little more than the full rule alone; many lanes turn it off
+  // for the line's other direction too, and lines that start on a tie never
+  // try it (u = v = 1 everywhere, 2048^2, L = 129: 727 -> 681 us).  (One saved state
+  // per chunk: saving it for every group cost 2 VALU instructions per step.)
+  bool fast = BRANCHLESS && short_path &&
+              __popcll(__builtin_amdgcn_ballot_w64(abs_t(pu) == abs_t(pv) && pu != T(0))) < 8;
   int32_t misses = 0;
   bool live_now = false, moves_now = false;  // set before a chunk of the short path
   bool status_known = false;
@@ -273,7 +276,9 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
           any_alive = __builtin_amdgcn_ballot_w64(alive) != 0;
         }
       } else {
-        fast = ++misses < 2 && __popcll(reported) < 8;
+        const bool many = __popcll(reported) >= 8;
+        fast = ++misses < 2 && !many;
+        short_path = short_path && !many;
         status_known = false;
         acc = acc_0;
         fx = fx_0;
