@@ -279,18 +279,23 @@ __global__ __launch_bounds__(kBoxThreads, 8) void lic_replay_box(
       for (int32_t w = 0; w < kBoxWaves; ++w) all = unite(all, of_wave(w));
       tiles[dir] = {in_pixels(all), (1u << kBoxWaves) - 1};
       if (Box(tiles[dir].b).elems() > box_elems) {  // uniform: one wave after the other, if it fits
-        Bounds some = no_bounds();
-        tiles[dir].waves = 0;
-        for (int32_t w = 0; w < kBoxWaves; ++w) {
-          const Bounds wider = unite(some, of_wave(w));
-          if (bits_of(of_wave(w).hi) == bits_of(no_bounds().hi) ||
-              Box(in_pixels(wider)).elems() > box_elems)
-            continue;
-          some = wider;
-          tiles[dir].waves |= 1u << w;
+        // from both ends of the tile: the set of more waves
+        tiles[dir] = {in_pixels(of_wave(0)), 0};  // no wave fits: nothing is staged
+        for (int32_t flip = 0; flip < kBoxWaves; flip += kBoxWaves - 1) {
+          Bounds some = no_bounds();
+          uint32_t waves = 0;
+          for (int32_t k = 0; k < kBoxWaves; ++k) {
+            const int32_t w = k ^ flip;
+            const Bounds wider = unite(some, of_wave(w));
+            if (bits_of(of_wave(w).hi) == bits_of(no_bounds().hi) ||
+                Box(in_pixels(wider)).elems() > box_elems)
+              continue;
+            some = wider;
+            waves |= 1u << w;
+          }
+          if (__builtin_popcount(waves) > __builtin_popcount(tiles[dir].waves))
+            tiles[dir] = {in_pixels(some), waves};
         }
-        // no wave fits: nothing is staged, whatever the bounds
-        tiles[dir].b = in_pixels(tiles[dir].waves ? some : of_wave(0));
       }
       if (tid == 0)
         tile[dir] = ReplayBounds{bits_of(tiles[dir].b.lo), bits_of(tiles[dir].b.hi),
