@@ -74,6 +74,19 @@ __device__ __forceinline__ Bounds unite(const Bounds& a, const Bounds& b) {
   return {__builtin_elementwise_min(a.lo, b.lo), __builtin_elementwise_max(a.hi, b.hi)};
 }
 
+// United over each row of 16 lanes, by rotations within it (all lanes active).
+template <int N>
+__device__ __forceinline__ Bounds rotated(const Bounds& b) {
+  return {pair_of(__builtin_amdgcn_mov_dpp(bits_of(b.lo), 0x120 + N, 15, 15, false)),
+          pair_of(__builtin_amdgcn_mov_dpp(bits_of(b.hi), 0x120 + N, 15, 15, false))};
+}
+__device__ __forceinline__ Bounds unite_rows(Bounds b) {
+  b = unite(b, rotated<8>(b));
+  b = unite(b, rotated<4>(b));
+  b = unite(b, rotated<2>(b));
+  return unite(b, rotated<1>(b));
+}
+
 // A line's bounds in one direction, in quarter pixels: of its positions after
 // every word of 8 steps (and of its start).  Between two of them it strays at
 // most 4 pixels further.  Stay and stop codes do not move, and an edge step
@@ -255,48 +268,67 @@ __global__ __launch_bounds__(kBoxThreads, 8) void lic_replay_box(
         }
       }
       Bounds b = inside ? line.b : no_bounds();
+      b = unite_rows(b);
 #pragma unroll
-      for (int off = 32; off > 0; off >>= 1)
+      for (int off = 32; off > 8; off >>= 1)
         b = unite(b, {pair_of(__shfl_xor(bits_of(b.lo), off)),
                       pair_of(__shfl_xor(bits_of(b.hi), off))});
       if (lane == 0) of_waves[wave][dir] = ReplayBounds{bits_of(b.lo), bits_of(b.hi), 0, 0};
     }
     __syncthreads();
+    // lanes 0..15 the waves' forward bounds, 16..31 the backward ones
+    static_assert(kBoxWaves == 16, "a row of lanes");
+    const ReplayBounds mine = of_waves[lane & 15][lane >> 4 & 1];
+    const Bounds in_rows = unite_rows({pair_of(mine.lo), pair_of(mine.hi)});
+    // to pixels, grown by 4 (LineBounds), to 16-byte aligned columns (stage)
+    auto in_pixels = [](Bounds b) {
+      b.lo = (b.lo >> static_cast<int16_t>(2)) - static_cast<int16_t>(4);
+      b.hi = (b.hi >> static_cast<int16_t>(2)) + static_cast<int16_t>(4);
+      b.lo.y &= ~3;
+      return b;
+    };
+    auto in_lane = [](const Bounds& b, int32_t l) {
+      return Bounds{pair_of(__builtin_amdgcn_readlane(bits_of(b.lo), l)),
+                    pair_of(__builtin_amdgcn_readlane(bits_of(b.hi), l))};
+    };
+    tiles[0] = {in_pixels(in_lane(in_rows, 0)), (1u << kBoxWaves) - 1};
+    tiles[1] = {in_pixels(in_lane(in_rows, 16)), (1u << kBoxWaves) - 1};
+    const bool fits[2] = {Box(tiles[0].b).elems() <= box_elems,
+                          Box(tiles[1].b).elems() <= box_elems};
+    if (!fits[0] || !fits[1]) {  // uniform
+      // A direction whose box does not fit: the waves taken one after the
+      // other if they still fit, each lane of a row in an order of its own
+      // (by the wave's number xor the lane's); the order that takes most.
+      Bounds some = no_bounds();
+      uint32_t waves = 0;
+      for (int32_t k = 0; k < kBoxWaves; ++k) {
+        const int32_t w = k ^ (lane & 15);
+        const ReplayBounds r = of_waves[w][lane >> 4 & 1];
+        const Bounds wider = unite(some, {pair_of(r.lo), pair_of(r.hi)});
+        const bool take = r.hi != bits_of(no_bounds().hi) &&
+                          Box(in_pixels(wider)).elems() <= box_elems;
+        some = take ? wider : some;
+        waves |= take ? 1u << w : 0u;
+      }
+      const int32_t key = __builtin_popcount(waves) * 16 + (lane & 15);
+      int32_t best = max(key, __builtin_amdgcn_mov_dpp(key, 0x128, 15, 15, false));
+      best = max(best, __builtin_amdgcn_mov_dpp(best, 0x124, 15, 15, false));
+      best = max(best, __builtin_amdgcn_mov_dpp(best, 0x122, 15, 15, false));
+      best = max(best, __builtin_amdgcn_mov_dpp(best, 0x121, 15, 15, false));
+#pragma unroll
+      for (int dir = 0; dir < 2; ++dir) {
+        if (fits[dir]) continue;
+        const int32_t l = 16 * dir + (__builtin_amdgcn_readlane(best, 16 * dir) & 15);
+        tiles[dir].waves =
+            static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int32_t>(waves), l));
+        // no wave fits: nothing is staged, whatever the bounds
+        tiles[dir].b = in_pixels(
+            tiles[dir].waves ? in_lane(some, l)
+                             : in_lane({pair_of(mine.lo), pair_of(mine.hi)}, 16 * dir));
+      }
+    }
 #pragma unroll
     for (int dir = 0; dir < 2; ++dir) {
-      auto of_wave = [&](int32_t w) {
-        return Bounds{pair_of(__builtin_amdgcn_readfirstlane(of_waves[w][dir].lo)),
-                      pair_of(__builtin_amdgcn_readfirstlane(of_waves[w][dir].hi))};
-      };
-      // to pixels, grown by 4 (LineBounds), to 16-byte aligned columns (stage)
-      auto in_pixels = [](Bounds b) {
-        b.lo = (b.lo >> static_cast<int16_t>(2)) - static_cast<int16_t>(4);
-        b.hi = (b.hi >> static_cast<int16_t>(2)) + static_cast<int16_t>(4);
-        b.lo.y &= ~3;
-        return b;
-      };
-      Bounds all = no_bounds();
-      for (int32_t w = 0; w < kBoxWaves; ++w) all = unite(all, of_wave(w));
-      tiles[dir] = {in_pixels(all), (1u << kBoxWaves) - 1};
-      if (Box(tiles[dir].b).elems() > box_elems) {  // uniform: one wave after the other, if it fits
-        // from both ends of the tile: the set of more waves
-        tiles[dir] = {in_pixels(of_wave(0)), 0};  // no wave fits: nothing is staged
-        for (int32_t flip = 0; flip < kBoxWaves; flip += kBoxWaves - 1) {
-          Bounds some = no_bounds();
-          uint32_t waves = 0;
-          for (int32_t k = 0; k < kBoxWaves; ++k) {
-            const int32_t w = k ^ flip;
-            const Bounds wider = unite(some, of_wave(w));
-            if (bits_of(of_wave(w).hi) == bits_of(no_bounds().hi) ||
-                Box(in_pixels(wider)).elems() > box_elems)
-              continue;
-            some = wider;
-            waves |= 1u << w;
-          }
-          if (__builtin_popcount(waves) > __builtin_popcount(tiles[dir].waves))
-            tiles[dir] = {in_pixels(some), waves};
-        }
-      }
       if (tid == 0)
         tile[dir] = ReplayBounds{bits_of(tiles[dir].b.lo), bits_of(tiles[dir].b.hi),
                                  tiles[dir].waves, 0};
