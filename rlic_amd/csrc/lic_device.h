@@ -268,7 +268,10 @@ struct VelocityRange<float> {
 };
 template <>
 struct VelocityRange<double> {
-  static constexpr double kMin = 0x1p-300, kMax = 0x1p300;
+  // With numerators of at least 2^-300 the times taken are at least 2^-450,
+  // what they add to a fraction at least 2^-750 and a multiple of 2^-802, and
+  // so are numerators: no quotient of one by up to 2^150 underflows.
+  static constexpr double kMin = 0x1p-300, kMax = 0x1p150;
 };
 
 template <typename T>
@@ -293,8 +296,7 @@ __device__ __forceinline__ double near_tie(double*) { return 0x1p-40; }
 // Key of a numerator n >= 0 that puts zero last: below numerator_key_min
 // for 0 < n < 2^-60 (float), 2^-300 (double).  A double key reads the top
 // word only: fractions, and with them numerators, that start at zero or at
-// least 2^-300 (fraction_usable) stay multiples of 2^-1004, for products of a
-// quotient of at least 2^-600 and a component of at least 2^-300 are.
+// least 2^-300 (fraction_usable) stay multiples of 2^-802 (VelocityRange).
 __device__ __forceinline__ uint32_t numerator_key(float n) {
   return __builtin_bit_cast(uint32_t, n) - 1u;
 }
@@ -305,6 +307,10 @@ __device__ __forceinline__ uint32_t numerator_key_min(float*) { return ((127u - 
 __device__ __forceinline__ uint32_t numerator_key_min(double*) {
   return ((1023u - 300u) << 20) - 1u;
 }
+
+// Float products n |w| from here on have quotients n / |w'| that do not round to
+// zero, for every |w'| up to kMax: 2 kMax^2 times the smallest number.
+constexpr float kProductMin = 0x1p-68f;
 
 // Fractions the short path starts from: in [0, 1], zero or at least 2^-300.
 // It keeps them in [0, 1]: away from ties the step ends before the other

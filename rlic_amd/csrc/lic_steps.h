@@ -73,7 +73,10 @@ struct NoSink {
 // their roundings compare as the exact ones do; otherwise (an exact or a near tie, both components zero, a NaN component:
 // every one of them fails the comparison) the lane is reported.  The
 // quotient is quotient_rn's, which needs a numerator that is zero or not tiny
-// (numerator_key_min): smaller ones are reported too.  A chunk in which a moving
+// (numerator_key_min): smaller ones are reported too.  A time of zero (n = 0)
+// compares below the other one only if that does not underflow to zero: in
+// float, lanes with |e| below kProductMin are reported (0.7% of a trace); in
+// double it cannot (VelocityRange).  A chunk in which a moving
 // lane is reported is thrown away and done again by the full rule, so the
 // results are the full rule's bit for bit.  A reported lane may pick a wrong
 // axis until the chunk ends, but a step always leads from an image cell to
@@ -109,6 +112,7 @@ __device__ __forceinline__ uint64_t fast_group(
   constexpr bool kFlip = !FORWARD && !LANE_DIR;
   uint32_t apart = 0xFFFFFFFFu;  // sign bit: no near tie so far
   uint32_t low = 0xFFFFFFFFu;    // smallest numerator seen (numerator_key)
+  T least = T(1);                // and |e| (float)
   uint32_t jump[8], jumped = 0;
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
@@ -131,6 +135,7 @@ __device__ __forceinline__ uint64_t fast_group(
     const T cy = ny * abs_t(mu);
     const T e = fma_t(nx, abs_t(mv), -cy);
     const uint32_t mx = sign_mask(e);  // step along x
+    if constexpr (sizeof(T) == 4) least = min(least, abs_t(e));
     apart &= top_word(fma_t(near_tie(static_cast<T*>(nullptr)), cy, -abs_t(e)));
     // where the picked component is nonzero (or the lane is reported),
     // pos_x and pos_y of the full rule are the sign tests already made
@@ -149,6 +154,7 @@ __device__ __forceinline__ uint64_t fast_group(
     if (q & 1) {
       keep_in_step(apart);
       keep_in_step(low);
+      if constexpr (sizeof(T) == 4) keep_in_step(least);
     }
     const T fy_after_x = macc<FMA>(t, mv, fy);
     const T fx_after_y = macc<FMA>(t, mu, fx);
@@ -189,6 +195,7 @@ __device__ __forceinline__ uint64_t fast_group(
   }
   return __builtin_amdgcn_ballot_w64(static_cast<int32_t>(apart) >= 0) |
          __builtin_amdgcn_ballot_w64(low < numerator_key_min(static_cast<T*>(nullptr))) |
+         __builtin_amdgcn_ballot_w64(least < T(kProductMin)) |
          __builtin_amdgcn_ballot_w64(__builtin_isunordered(fx, fy));
 }
 
