@@ -93,13 +93,20 @@ __device__ __forceinline__ void batch_trace_pixel(const BatchField<T>& f,
   const int64_t p = static_cast<int64_t>(i0) * f.g.nx + j0;
   const uint32_t row0 = static_cast<uint32_t>(cell_slot(f.g, i0 + 1, j0 + 1));
   const CellVal<T> c0 = cell(row0);
-  bool short_path = !wide_mark(f.cells, f.epoch);
   T acc = macc<FMA>(kernel[kmid], c0.x, T(0));  // src/lib.rs:375-383
-  acc = trace_direction<T, FMA, BRANCHLESS, POL, true, REC, BUF, true>(
-      acc, c0.u, c0.v, row0, cell, kernel, kmid, n_fwd, sg, f.codes, np, p, 0, short_path);
-  acc = trace_direction<T, FMA, BRANCHLESS, POL, false, REC, BUF, true>(
-      acc, c0.u, c0.v, row0, cell, kernel, kmid, n_bwd, sg, f.codes, np, p, chunks_of(n_fwd),
-      short_path);
+  auto line = [&](auto narrow) {
+    constexpr bool kNarrow = decltype(narrow)::value;
+    bool short_path = true;
+    SavedRegisters<T> saved;
+    acc = trace_direction<T, FMA, BRANCHLESS, POL, true, REC, BUF, true, kNarrow>(
+        acc, c0.u, c0.v, row0, cell, kernel, kmid, n_fwd, sg, f.codes, np, p, 0, short_path, saved);
+    acc = trace_direction<T, FMA, BRANCHLESS, POL, false, REC, BUF, true, kNarrow>(
+        acc, c0.u, c0.v, row0, cell, kernel, kmid, n_bwd, sg, f.codes, np, p, chunks_of(n_fwd),
+        short_path, saved);
+  };
+  const bool wide = !BRANCHLESS || wide_mark(f.cells, f.epoch);  // uniform
+  if (wide) line(std::false_type{});
+  else line(std::bool_constant<BRANCHLESS>{});
   dst[p] = acc;
 }
 

@@ -179,23 +179,6 @@ __device__ __forceinline__ double xor_sign(double x, uint32_t sign) {
   return __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, x) ^ (uint64_t{sign} << 32));
 }
 
-// 2 * x + (this lane's bit of the wave64 lane mask `mask`) in one VALU
-// instruction: the mask is the add's carry-in.
-__device__ __forceinline__ uint32_t carry_in_bit(uint32_t x, uint64_t mask) {
-  uint32_t r;
-  uint64_t carry_out;
-  asm("v_addc_co_u32_e64 %0, %1, %2, %2, %3" : "=v"(r), "=s"(carry_out) : "v"(x), "s"(mask));
-  return r;
-}
-
-// This lane's bit of the wave64 lane mask `mask`, as 0 or 1.
-__device__ __forceinline__ uint32_t lane_bit(uint64_t mask) {
-  uint32_t r;
-  uint64_t carry_out;
-  asm("v_addc_co_u32_e64 %0, %1, 0, 0, %2" : "=v"(r), "=s"(carry_out) : "s"(mask));
-  return r;
-}
-
 __device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
 __device__ __forceinline__ float abs_t(float a) { return __builtin_fabsf(a); }
@@ -219,6 +202,68 @@ __device__ __forceinline__ T macc(T a, T b, T c) {
   }
 }
 
+// Lane masks (0 or all ones) in VGPRs, and selections by them: v_bitop3
+// issues in half the cycles of v_cndmask and v_bfi, and written as builtins
+// they are not turned back into compares and selects.
+__device__ __forceinline__ uint32_t sign_mask(float x) {
+  return static_cast<uint32_t>(__builtin_bit_cast(int32_t, x) >> 31);
+}
+__device__ __forceinline__ uint32_t sign_mask(double x) {
+  return static_cast<uint32_t>(static_cast<int32_t>(__builtin_bit_cast(uint64_t, x) >> 32) >> 31);
+}
+template <uint32_t TABLE>
+__device__ __forceinline__ uint32_t bitop3(uint32_t a, uint32_t b, uint32_t c) {
+  return static_cast<uint32_t>(__builtin_amdgcn_bitop3_b32(a, b, c, TABLE));
+}
+// where the mask is set a, else b
+__device__ __forceinline__ uint32_t pick(uint32_t m, uint32_t a, uint32_t b) {
+  return bitop3<0xCA>(m, a, b);
+}
+struct Words {
+  uint32_t lo, hi;
+};
+__device__ __forceinline__ float pick(uint32_t m, float a, float b) {
+  return __builtin_bit_cast(float, pick(m, __builtin_bit_cast(uint32_t, a),
+                                        __builtin_bit_cast(uint32_t, b)));
+}
+__device__ __forceinline__ double pick(uint32_t m, double a, double b) {
+  const Words x = __builtin_bit_cast(Words, a), y = __builtin_bit_cast(Words, b);
+  return __builtin_bit_cast(double, Words{pick(m, x.lo, y.lo), pick(m, x.hi, y.hi)});
+}
+// 2 where the mask is clear (FLIP: set), else +0
+template <bool FLIP>
+__device__ __forceinline__ float two_where(uint32_t m, float*) {
+  return __builtin_bit_cast(float, bitop3<FLIP ? 0xC0 : 0x30>(0x40000000u, m, m));
+}
+template <bool FLIP>
+__device__ __forceinline__ double two_where(uint32_t m, double*) {
+  return __builtin_bit_cast(double, Words{0u, bitop3<FLIP ? 0xC0 : 0x30>(0x40000000u, m, m)});
+}
+// x where the mask is clear (FLIP: set), else +0
+template <bool FLIP>
+__device__ __forceinline__ uint32_t keep_bits(uint32_t x, uint32_t m) {
+  return bitop3<FLIP ? 0xC0 : 0x30>(x, m, m);
+}
+template <bool FLIP>
+__device__ __forceinline__ float keep_where(float x, uint32_t m) {
+  return __builtin_bit_cast(float, keep_bits<FLIP>(__builtin_bit_cast(uint32_t, x), m));
+}
+template <bool FLIP>
+__device__ __forceinline__ double keep_where(double x, uint32_t m) {
+  const Words w = __builtin_bit_cast(Words, x);
+  return __builtin_bit_cast(double, Words{keep_bits<FLIP>(w.lo, m), keep_bits<FLIP>(w.hi, m)});
+}
+// 1 where the mask `neg` is set (FLIP: clear), else 0
+template <bool FLIP>
+__device__ __forceinline__ float edge_fraction(uint32_t neg, float*) {
+  const uint32_t one = 0x3F800000u;
+  return __builtin_bit_cast(float, bitop3<FLIP ? 0x0C : 0xC0>(neg, one, one));
+}
+template <bool FLIP>
+__device__ __forceinline__ double edge_fraction(uint32_t neg, double*) {
+  const uint32_t one = 0x3FF00000u;
+  return __builtin_bit_cast(double, Words{0u, bitop3<FLIP ? 0x0C : 0xC0>(neg, one, one)});
+}
 // Time to reach the next cell edge along one axis (src/lib.rs:157-180).
 // Correctly rounded division (IEEE round-to-nearest-even, denormals kept):
 // hipcc's float and double division (v_div_scale / v_rcp / v_div_fmas /
@@ -231,40 +276,36 @@ __device__ __forceinline__ double div_rn(double a, double b) { return a / b; }
 
 // `velocity` is never NaN here: NaN vectors end the streamline first
 // (src/lib.rs:336-338).
-// `negative` is the sign bit of `velocity` (the branchless rule's
-// 1 + signum(velocity)), given by the caller, which tests it once for
-// both uses.
-template <typename T, bool FMA, bool BRANCHLESS>
-__device__ __forceinline__ T time_to_next_pixel(T velocity, T frac, bool negative) {
-  if constexpr (!BRANCHLESS) {
-    if (velocity > T(0)) return div_rn(T(1) - frac, velocity);
-    if (velocity < T(0)) return -div_rn(frac, velocity);
-    return inf_t<T>();
-  } else {
-    // 1 + signum(velocity): 0 when the sign bit is set (also -0.0), else 2.
-    const T factor = negative ? T(0) : T(2);
-    const T remaining = macc<FMA>(factor, T(0.5) - frac, frac);
-    return abs_t(div_rn(remaining, velocity));
-  }
-}
-
-template <typename T, bool FMA, bool BRANCHLESS>
+template <typename T>
 __device__ __forceinline__ T time_to_next_pixel(T velocity, T frac) {
-  return time_to_next_pixel<T, FMA, BRANCHLESS>(velocity, frac, __builtin_signbit(velocity));
+  if (velocity > T(0)) return div_rn(T(1) - frac, velocity);
+  if (velocity < T(0)) return -div_rn(frac, velocity);
+  return inf_t<T>();
 }
 
-// Ranges of the step's short path (fast_group).  A field is "wide" when a
-// velocity component is infinite or nonzero below kMin / above kMax in
-// magnitude; the packing kernels look at every component and mark such a
-// field (wide_mark), whose lines then take the full rule throughout.
-// Within these ranges and with numerators of at least numerator_min (or
-// zero) the products n |w|, the quotient and its remainder are normal
-// numbers or exact, so no scaling is needed.
+// The branchless rule divides this by the velocity: 1 + signum(velocity) is 0
+// when the sign bit is set (also -0.0), else 2.  `sign` is the mask of that
+// bit (FLIP: the opposite), which the caller uses otherwise too.
+template <typename T, bool FMA, bool FLIP>
+__device__ __forceinline__ T step_numerator(T frac, uint32_t sign) {
+  return macc<FMA>(two_where<FLIP>(sign, static_cast<T*>(nullptr)), T(0.5) - frac, frac);
+}
+
+// Ranges of the step's short path (fast_group) and quick quotient
+// (full_group).  A field is "wide" when a velocity component is infinite or
+// nonzero below kMin / above kMax in magnitude (float: 2^-60 = 8.7e-19 to 2^40 =
+// 1.1e12); the packing kernels look at every component and mark such a field
+// (wide_mark), whose lines then take the divisions throughout: a limit on speed,
+// not on results.
+// Within these ranges and with numerators of at least numerator_key_min (or
+// zero) the quotient and its remainder are normal numbers or exact, so no
+// scaling is needed, and so are the products n |w| compared in fast_group
+// wherever they are not below kProductMin.
 template <typename T>
 struct VelocityRange;
 template <>
 struct VelocityRange<float> {
-  static constexpr float kMin = 0x1p-40f, kMax = 0x1p40f;
+  static constexpr float kMin = 0x1p-60f, kMax = 0x1p40f;
 };
 template <>
 struct VelocityRange<double> {
@@ -303,6 +344,15 @@ __device__ __forceinline__ uint32_t numerator_key(float n) {
 __device__ __forceinline__ uint32_t numerator_key(double n) {
   return static_cast<uint32_t>(__builtin_bit_cast(uint64_t, n) >> 32) - 1u;
 }
+// |w|, or for a zero w far less than any other divisor: numerators that are not
+// tiny over it exceed every quotient by a |w| within VelocityRange.
+__device__ __forceinline__ float positive_divisor(float w) {
+  return __builtin_amdgcn_fmed3f(abs_t(w), 0x1p-125f, inf_t<float>());
+}
+// The lanes with a nonzero numerator below what quotient_rn takes.
+__device__ __forceinline__ uint64_t tiny_numerators(float n) {
+  return __builtin_amdgcn_ballot_w64(n != 0.0f) & __builtin_amdgcn_ballot_w64(abs_t(n) < 0x1p-60f);
+}
 __device__ __forceinline__ uint32_t numerator_key_min(float*) { return ((127u - 60u) << 23) - 1u; }
 __device__ __forceinline__ uint32_t numerator_key_min(double*) {
   return ((1023u - 300u) << 20) - 1u;
@@ -320,59 +370,6 @@ __device__ __forceinline__ bool fraction_usable(double f) {
   return f == 0.0 || (f >= 0x1p-300 && f <= 1.0);
 }
 
-// Lane masks (0 or all ones) in VGPRs, and selections by them: v_bitop3
-// issues in half the cycles of v_cndmask and v_bfi, and written as builtins
-// they are not turned back into compares and selects.
-__device__ __forceinline__ uint32_t sign_mask(float x) {
-  return static_cast<uint32_t>(__builtin_bit_cast(int32_t, x) >> 31);
-}
-__device__ __forceinline__ uint32_t sign_mask(double x) {
-  return static_cast<uint32_t>(static_cast<int32_t>(__builtin_bit_cast(uint64_t, x) >> 32) >> 31);
-}
-template <uint32_t TABLE>
-__device__ __forceinline__ uint32_t bitop3(uint32_t a, uint32_t b, uint32_t c) {
-  return static_cast<uint32_t>(__builtin_amdgcn_bitop3_b32(a, b, c, TABLE));
-}
-// where the mask is set a, else b
-__device__ __forceinline__ uint32_t pick(uint32_t m, uint32_t a, uint32_t b) {
-  return bitop3<0xCA>(m, a, b);
-}
-struct Words {
-  uint32_t lo, hi;
-};
-__device__ __forceinline__ float pick(uint32_t m, float a, float b) {
-  return __builtin_bit_cast(float, pick(m, __builtin_bit_cast(uint32_t, a),
-                                        __builtin_bit_cast(uint32_t, b)));
-}
-__device__ __forceinline__ double pick(uint32_t m, double a, double b) {
-  const Words x = __builtin_bit_cast(Words, a), y = __builtin_bit_cast(Words, b);
-  return __builtin_bit_cast(double, Words{pick(m, x.lo, y.lo), pick(m, x.hi, y.hi)});
-}
-// x where the mask is clear (FLIP: set), else +0
-template <bool FLIP>
-__device__ __forceinline__ uint32_t keep_bits(uint32_t x, uint32_t m) {
-  return bitop3<FLIP ? 0xC0 : 0x30>(x, m, m);
-}
-template <bool FLIP>
-__device__ __forceinline__ float keep_where(float x, uint32_t m) {
-  return __builtin_bit_cast(float, keep_bits<FLIP>(__builtin_bit_cast(uint32_t, x), m));
-}
-template <bool FLIP>
-__device__ __forceinline__ double keep_where(double x, uint32_t m) {
-  const Words w = __builtin_bit_cast(Words, x);
-  return __builtin_bit_cast(double, Words{keep_bits<FLIP>(w.lo, m), keep_bits<FLIP>(w.hi, m)});
-}
-// 1 where the mask `neg` is set (FLIP: clear), else 0
-template <bool FLIP>
-__device__ __forceinline__ float edge_fraction(uint32_t neg, float*) {
-  const uint32_t one = 0x3F800000u;
-  return __builtin_bit_cast(float, bitop3<FLIP ? 0x0C : 0xC0>(neg, one, one));
-}
-template <bool FLIP>
-__device__ __forceinline__ double edge_fraction(uint32_t neg, double*) {
-  const uint32_t one = 0x3FF00000u;
-  return __builtin_bit_cast(double, Words{0u, bitop3<FLIP ? 0x0C : 0xC0>(neg, one, one)});
-}
 __device__ __forceinline__ uint32_t top_word(float x) { return __builtin_bit_cast(uint32_t, x); }
 __device__ __forceinline__ uint32_t top_word(double x) { return __builtin_bit_cast(Words, x).hi; }
 // x with its sign bit xor-ed with that of s
@@ -532,6 +529,7 @@ enum : uint32_t {
   kMoveYMinus = kMoveAxisY | kMoveNeg
 };
 constexpr uint32_t kWordStay = 0x11111111u * kMoveStay;
+constexpr uint32_t kWordMoves = 0x11111111u * (kMoveNeg | kMoveAxisY);
 
 // word * 16 + a step's code: kMoveAxisY where `mx` is clear, kMoveNeg where
 // `neg` is set (with FLIP clear); the lowest and the highest bit of the code

@@ -23,15 +23,13 @@ __host__ __device__ inline int32_t chunks_of(int32_t nsteps) {
 
 // One streamline direction of one pixel (src/lib.rs:304-362), starting from
 // the vector (pu, pv) of the start cell, already loaded.  The position `row`
-// is the cell's slot (cell_slot).  Returns the updated accumulator.  With REC, writes the move code of every step.
+// is the cell's slot (cell_slot).  Returns the updated accumulator.  With REC,
+// writes the move code of every step.
 //
-// The step is written without divergent branches: a lane whose line has
-// ended (NaN vector) keeps executing with its position frozen and its
-// accumulator untouched, and a lane with a zero vector keeps its position
-// (src/lib.rs:242-244); steps run in groups of 8 (one code word, one batch
-// of 8 weights) and a wave leaves the loop once all its lines have ended.
-// With `short_path` (the field's velocities are not wide, velocity_wide),
-// whole groups of the branchless rule run as fast_group.
+// Steps run in groups of 8 (one code word) without divergent branches, and a
+// wave leaves the loop once all its lines have ended: whole groups by
+// fast_group while `short_path` holds, others by full_group.
+// NARROW: the branchless rule, and a field that is not wide (velocity_wide).
 //
 // The cells form a guarded array (guarded_cells: (ny + 2) x (nx + 2)
 // with a ring of guard cells around the image).
@@ -54,6 +52,14 @@ struct NoSink {
   template <typename T>
   __device__ __forceinline__ void operator()(int32_t, T) const {}
 };
+
+// Whether a step of `jump` slots on from a guard cell leads back to the cell it
+// came from: a jump as long as a step (a closed side, or the only column or
+// row of a periodic one).
+__device__ __forceinline__ bool jump_stays(uint32_t jump, const StepGeom& sg) {
+  const uint32_t far = min(jump, 0u - jump);
+  return far == sg.step_x || far == sg.near_y || far == sg.far_y;
+}
 
 // Eight steps of the default step rule on the short path: what trace_direction
 // does in its full group, with the two divisions of a step replaced by one.
@@ -176,19 +182,15 @@ __device__ __forceinline__ uint64_t fast_group(
     keep_in_step(acc);
   }
   if constexpr (REC != 0) {
-    word &= 0x11111111u * (kMoveNeg | kMoveAxisY);
+    word &= kWordMoves;
     if (__builtin_amdgcn_ballot_w64(jumped != 0u) != 0) {  // uniform: some line left the image
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         keep_in_step(jump[q]);  // compared here, not before the branch
-        // a jump back to the cell the step came from (as long as the step:
-        // a closed side, or the only column or row of a periodic one) stays
-        const uint32_t far = min(jump[q], 0u - jump[q]);
-        const bool stays = far == sg.step_x || far == sg.near_y || far == sg.far_y;
         const uint32_t low = 28 - 4 * q;
-        word = jump[q] == 0u ? word
-                             : (stays ? (word & ~(15u << low)) | (kMoveStay << low)
-                                      : word | (kMoveEdge << low));
+        const uint32_t left = jump_stays(jump[q], sg) ? (word & ~(15u << low)) | (kMoveStay << low)
+                                                      : word | (kMoveEdge << low);
+        word = jump[q] == 0u ? word : left;
       }
       keep_in_step(word);  // a branch, not selects
     }
@@ -199,33 +201,248 @@ __device__ __forceinline__ uint64_t fast_group(
          __builtin_amdgcn_ballot_w64(__builtin_isunordered(fx, fy));
 }
 
+// A lane's state at the start of a chunk, for doing the chunk again: kept in
+// registers, or (SavedLds) in its kWords values of LDS.  The vector is not
+// kept: it is gathered again.
+template <typename T>
+struct SavedRegisters {
+  T a, x, y, u, v;
+  __device__ __forceinline__ void put(T acc, T fx, T fy, T lu, T lv) {
+    a = acc;
+    x = fx;
+    y = fy;
+    u = lu;
+    v = lv;
+  }
+  __device__ __forceinline__ T acc() const { return a; }
+  __device__ __forceinline__ void get(T& acc, T& fx, T& fy, T& lu, T& lv) const {
+    acc = a;
+    fx = x;
+    fy = y;
+    lu = u;
+    lv = v;
+  }
+};
+template <typename T, bool POL>
+struct SavedLds {
+  static constexpr int32_t kWords = POL ? 5 : 3;
+  // volatile: stored, not carried along in registers
+  typedef volatile T __attribute__((address_space(3))) lds_t;
+  lds_t* at;
+  __device__ __forceinline__ void put(T acc, T fx, T fy, T lu, T lv) {
+    at[0] = acc;
+    at[1] = fx;
+    at[2] = fy;
+    if constexpr (POL) {
+      at[3] = lu;
+      at[4] = lv;
+    }
+  }
+  __device__ __forceinline__ T acc() const { return at[0]; }
+  __device__ __forceinline__ void get(T& acc, T& fx, T& fy, T& lu, T& lv) const {
+    acc = at[0];
+    fx = at[1];
+    fy = at[2];
+    if constexpr (POL) {
+      lu = at[3];
+      lv = at[4];
+    }
+  }
+};
+
+// A group of up to 8 steps by the full rule (src/lib.rs:304-362), for lanes in
+// any state: a lane whose line has ended (NaN vector) keeps executing with its
+// position frozen and its accumulator untouched, a lane with a zero vector
+// keeps its position (src/lib.rs:242-244).  `m_live` receives the lanes whose
+// line had not ended before the last step.
+//
+// QUICK (float, branchless rule, velocities within VelocityRange): the step
+// times by quotient_rn, which is what the division gives but for tiny
+// numerators; a step in which a moving lane has one is done again with the
+// division (in double the tests cost what the shorter quotient saves).
+//
+// What bounds it: VALU issue, and the chain from a cell's vector to the next
+// address.  So selections are bit operations on lane masks, as in fast_group,
+// rare cases are tested behind the gather's issue (before it, the test's
+// branch cost 8%), and eight steps are one block of straight code (a branch out
+// of it for a short last group made the compiler copy the state at each step).
+// A step is 51 VALU instructions, with the record 57, QUICK 47 and 53; 49 and 54
+// before row pairs and the short path existed, 57 and 69 with them at first.
+// 2048^2, L = 129, a field with one component out of range, us a call then, at
+// first, now: float 601, 638, 606, double 1015, 1043, 990; with the record (L =
+// 65, two passes) 426, 478, 420 and 662, 702, 649.
 template <typename T, bool FMA, bool BRANCHLESS, int POL, bool FORWARD, int REC, bool BUF,
-          bool PAIRS, bool LANE_DIR = false, typename Sink = NoSink>
+          bool PAIRS, bool LANE_DIR, bool QUICK, typename Sink>
+__device__ __forceinline__ void full_group(T& acc, T& fx, T& fy, T& pu, T& pv, T& last_u,
+                                           T& last_v, uint32_t& row, uint64_t& m_live,
+                                           uint32_t& word, const T* __restrict__ taps,
+                                           const CellGather<T, BUF>& cell, const StepGeom& sg,
+                                           uint32_t lane_sign, int32_t s0, int32_t steps,
+                                           Sink& sink, int32_t* live_steps) {
+  constexpr bool kFlip = !FORWARD && !LANE_DIR;
+  uint32_t marks = 0, moved = 0;  // codes of steps that left the image; steps that moved
+  auto one = [&](int32_t q) {
+    const T weight = taps[FORWARD ? q : -q];
+    // a NaN component ends the line (src/lib.rs:336-338), which stays on its cell
+    const bool live = !__builtin_isunordered(pu, pv);
+    m_live = __builtin_amdgcn_ballot_w64(live);
+    if constexpr (POL != 0) {  // src/lib.rs:339-347, unfused dot product
+      const T d1 = pu * last_u;
+      const T d2 = pv * last_v;
+      const bool flip = d1 + d2 < T(0);
+      pu = flip ? -pu : pu;
+      pv = flip ? -pv : pv;
+      last_u = pu;
+      last_v = pv;
+    }
+    // src/lib.rs:348-351
+    const T mu = LANE_DIR ? xor_sign(pu, lane_sign) : (FORWARD ? pu : -pu);
+    const T mv = LANE_DIR ? xor_sign(pv, lane_sign) : (FORWARD ? pv : -pv);
+    // masks of the sign bits of mu, mv, read off pu, pv (kFlip: the opposite),
+    // so that a backward step does not materialize -pu, -pv for them: the
+    // divisions and products take the negation as a modifier
+    const uint32_t sx = sign_mask(LANE_DIR ? mu : pu), sy = sign_mask(LANE_DIR ? mv : pv);
+    // no move when both components are +-0 (src/lib.rs:242-244)
+    const bool moves = live & ((mu != T(0)) | (mv != T(0)));
+    T tx, ty;
+    uint32_t mx, sp, at;
+    auto step_to = [&](uint32_t neg_y) {
+      // x edge first when tx < ty; ties and NaN go to y (src/lib.rs:249-269)
+      mx = tx < ty ? ~0u : 0u;
+      sp = pick(mx, sx, neg_y);  // toward lower indices (kFlip: higher)
+      uint32_t dist_y = sg.far_y;
+      if constexpr (PAIRS)  // up from an odd row, down from an even one: another pair
+        dist_y = pick(bitop3<kFlip ? 0xEB : 0xBE>(0u - (row & 1u), sp, sg.all_far), sg.far_y,
+                      sg.near_y);
+      const uint32_t step = moves ? pick(mx, sg.step_x, dist_y) : 0u;
+      at = kFlip ? row + sp - (step ^ sp) : row - sp + (step ^ sp);
+    };
+    auto divide = [&]() {
+      if constexpr (BRANCHLESS) {
+        tx = abs_t(div_rn(step_numerator<T, FMA, kFlip>(fx, sx), mu));
+        ty = abs_t(div_rn(step_numerator<T, FMA, kFlip>(fy, sy), mv));
+      } else {
+        tx = time_to_next_pixel(mu, fx);
+        ty = time_to_next_pixel(mv, fy);
+      }
+    };
+    uint64_t tiny = 0;
+    if constexpr (QUICK) {
+      const T nx = step_numerator<T, FMA, kFlip>(fx, sx);
+      const T ny = step_numerator<T, FMA, kFlip>(fy, sy);
+      tx = abs_t(quotient_rn(nx, abs_t(mu)));
+      // beside any other time, one over a component of 0 is as good as infinite
+      ty = abs_t(quotient_rn(ny, positive_divisor(mv)));
+      tiny = tiny_numerators(nx) | tiny_numerators(ny);
+    } else {
+      divide();
+    }
+    step_to(sy);
+    CellVal<T> cv = cell(at);
+    // Tested while the cell is on its way.  Toward lower indices is mu < 0, mv
+    // < 0 (src/lib.rs:217): the sign bit, but for y steps with mv = -0 (ty
+    // infinite or NaN).
+    const uint64_t m_mv = __builtin_amdgcn_ballot_w64(mv != T(0));
+    const uint64_t level = ~m_mv & ~__builtin_amdgcn_ballot_w64(tx < ty);
+    if ((m_live & (m_mv | __builtin_amdgcn_ballot_w64(mu != T(0))) & (level | tiny)) != 0) {
+      if constexpr (QUICK) divide();  // uniform
+      step_to(mv == T(0) ? (kFlip ? ~0u : 0u) : sy);
+      cv = cell(at);
+    }
+    // update_state (src/lib.rs:208-233) for either axis, keeping one.  The
+    // fractions need no "moves" gate: a lane that does not move never moves
+    // again (an ended line stays on its NaN cell, a zero vector stays on its
+    // cell, whose vector stays zero, polarization flips included), so its
+    // fractions are never read again: they only feed step times, whose
+    // results are masked out of its codes and its position update.
+    const T fy_after_x = macc<FMA>(tx, mv, fy);
+    const T fx_after_y = macc<FMA>(ty, mu, fx);
+    const T edge = edge_fraction<kFlip>(sp, static_cast<T*>(nullptr));
+    fx = pick(mx, edge, fx_after_y);
+    fy = pick(mx, fy_after_x, edge);
+    const uint32_t jump = pad_bits(cv.pad);  // not 0: the step left the image
+    row = at + jump;
+    const T next_acc = macc<FMA>(weight, cv.x, acc);  // src/lib.rs:353-360
+    acc = live ? next_acc : acc;
+    keep_in_step(acc);
+    sink(s0 + q, cv.x);
+    if (live_steps) *live_steps = live ? s0 + q + 1 : *live_steps;
+    pu = cv.u;
+    pv = cv.v;
+    if constexpr (REC != 0) {
+      word = push_code<kFlip>(word, sp, mx);
+      keep_in_step(word);
+      moved += moves ? 1u : 0u;
+      if (__builtin_amdgcn_ballot_w64(jump != 0u) != 0) {  // uniform
+        uint32_t code = jump_stays(jump, sg) ? kMoveStay : kMoveEdge;
+        keep_in_step(code);  // shifted after: the select's constants stay inline
+        marks |= jump != 0u ? code << (28 - 4 * q) : 0u;
+        keep_in_step(marks);  // a branch, not selects
+      }
+    }
+  };
+  if (!LANE_DIR && steps == 8) {  // uniform
+#pragma unroll
+    for (int32_t q = 0; q < 8; ++q) one(q);
+  } else {
+#pragma unroll 1
+    for (int32_t q = 0; q < steps; ++q) one(q);
+  }
+  if constexpr (REC != 0) {
+    // a last group of fewer than 8 steps: its first step to the top nibble
+    if (steps < 8) word <<= 4 * (8 - steps);
+    const uint32_t stays = marks & kWordStay;
+    word = (word & kWordMoves & ~(stays >> 1 | stays >> 2)) | marks;
+    if (steps < 8 || __builtin_amdgcn_ballot_w64(moved < 8) != 0) {  // uniform
+      // A lane that stops moving stays so: "stay" from there on, or "stop" on
+      // a NaN cell (readers stop at the first one).
+      const bool ended = moved < static_cast<uint32_t>(steps) && __builtin_isunordered(pu, pv);
+      const uint32_t still = ended ? 0x11111111u * kMoveStop : kWordStay;
+      word = moved < 8 ? (word & ~(~0u >> (4 * moved))) | (still >> (4 * moved)) : word;
+    }
+  }
+}
+
+template <typename T, bool FMA, bool BRANCHLESS, int POL, bool FORWARD, int REC, bool BUF,
+          bool PAIRS, bool NARROW, bool LANE_DIR = false, typename Saved, typename Sink = NoSink>
 __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
                                              const CellGather<T, BUF>& cell,
                                              const T* __restrict__ kernel, int32_t kmid,
                                              int32_t nsteps, const StepGeom& sg,
                                              uint4* __restrict__ codes, int64_t np, int64_t p,
-                                             int32_t c0, bool& short_path,
+                                             int32_t c0, bool& short_path, Saved& saved,
                                              bool fwd_lane = true, Sink sink = Sink{},
                                              int32_t* live_steps = nullptr) {
-  constexpr bool pol = POL != 0, rec = REC != 0;
+  constexpr bool rec = REC != 0;
   const uint32_t lane_sign = fwd_lane ? 0u : 0x80000000u;  // LANE_DIR: negate on backward lanes
   T fx = T(0.5), fy = T(0.5);      // src/lib.rs:315-318
   T last_u = T(0), last_v = T(0);  // src/lib.rs:320-323
-  bool alive = true;
-  const uint32_t far_y = lane_copy(sg.far_y), near_y = lane_copy(sg.near_y);  // held in VGPRs
+  // held in VGPRs
+  const StepGeom sl = {sg.step_x, lane_copy(sg.near_y), lane_copy(sg.far_y), sg.all_far};
   const int32_t nchunks = chunks_of(nsteps);
   // Short path: whole groups of a chunk by fast_group; when a moving lane is
-  // reported, the chunk is done again by the full rule.  Off for the rest of
-  // the direction after a chunk that reports many lanes (a field of ties,
-  // e.g. u = v everywhere) or a second chunk that reports any, so that such
-  // a line costs little more than the full rule alone; many lanes turn it off
-  // for the line's other direction too, and lines that start on a tie never
-  // try it (u = v = 1 everywhere, 2048^2, L = 129: 727 -> 681 us).  (One saved state
-  // per chunk: saving it for every group cost 2 VALU instructions per step.)
-  bool fast = BRANCHLESS && short_path &&
-              __popcll(__builtin_amdgcn_ballot_w64(abs_t(pu) == abs_t(pv) && pu != T(0))) < 8;
+  // reported, the chunk is done again by the full rule (one saved state per
+  // chunk: saving it for every group cost 2 VALU instructions per step).  What
+  // is thrown away costs a group at least, so the path is left for the rest of
+  // the line and for its other direction where more reports are likely: after
+  // one of many lanes, one in a chunk's first two groups, or a second one; in
+  // double, where a step saves 1/6 (float: 1/4), after any, and it is not tried
+  // where lanes of the wave start on a tie or only some of them move.
+  // 2048^2, L = 129, us a call before this path existed, with two tries in each
+  // direction, now: float 1% of cells NaN 596, 720, 582, 10% zero 577, 644, 535,
+  // whole numbers (ties and zeros) 583, 654, 587, u = v 579, 635, 524; double
+  // 991, 1202, 1027, then 970, 998, 890, then 922, 1020, 955, then 939, 989, 941.
+  const uint64_t m_tie = __builtin_amdgcn_ballot_w64(abs_t(pu) == abs_t(pv)) &
+                         __builtin_amdgcn_ballot_w64(pu != T(0));
+  bool fast = NARROW && short_path;
+  if constexpr (sizeof(T) == 4) {
+    fast = fast && __popcll(m_tie) < 8;
+  } else {
+    const uint64_t m_rest = __builtin_amdgcn_ballot_w64(__builtin_isunordered(pu, pv)) |
+                            (__builtin_amdgcn_ballot_w64(pu == T(0)) &
+                             __builtin_amdgcn_ballot_w64(pv == T(0)));
+    fast = fast && m_tie == 0 && (m_rest == 0 || m_rest == __builtin_amdgcn_ballot_w64(true));
+  }
   int32_t misses = 0;
   bool live_now = false, moves_now = false;  // set before a chunk of the short path
   bool status_known = false;
@@ -233,23 +450,22 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
     uint32_t words[4] = {kWordStay, kWordStay, kWordStay, kWordStay};
     bool any_alive = true;
     int g0 = 0;
-    if (BRANCHLESS && fast) {  // uniform
+    if (NARROW && fast) {  // uniform
       if (!status_known) {  // lanes that do not move never move again
-        live_now = alive && !__builtin_isunordered(pu, pv);
+        live_now = !__builtin_isunordered(pu, pv);
         moves_now = live_now && (pu != T(0) || pv != T(0));
         status_known = true;
       }
       const uint64_t m_moves = __builtin_amdgcn_ballot_w64(moves_now);
-      const StepGeom sl = {moves_now ? sg.step_x : 0u, moves_now ? near_y : 0u,
-                           moves_now ? far_y : 0u, sg.all_far};
+      const StepGeom sm = {moves_now ? sl.step_x : 0u, moves_now ? sl.near_y : 0u,
+                           moves_now ? sl.far_y : 0u, sl.all_far};
       // fractions outside what fast_group takes (the full rule can leave
       // some after a tie): this chunk by the full rule
       const bool usable = __builtin_amdgcn_ballot_w64(moves_now && !(fraction_usable(fx) &&
                                                                       fraction_usable(fy))) == 0;
       const int full = usable ? min(4, (nsteps - ch * kChunkSteps) >> 3) : 0;
-      const T acc_0 = acc, fx_0 = fx, fy_0 = fy, pu_0 = pu, pv_0 = pv, lu_0 = last_u,
-              lv_0 = last_v;
       const uint32_t row_0 = row;
+      saved.put(acc, fx, fy, last_u, last_v);
       uint64_t reported = 0;
 #pragma unroll 1
       for (; g0 < full; ++g0) {
@@ -260,7 +476,7 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
           kw[q] = kernel[FORWARD ? kmid + 1 + s0 + q : kmid - 1 - s0 - q];
         uint32_t word = 0;
         reported = fast_group<T, FMA, POL, FORWARD, REC, BUF, PAIRS, LANE_DIR>(
-                       acc, fx, fy, pu, pv, last_u, last_v, row, word, kw, cell, sl, lane_sign,
+                       acc, fx, fy, pu, pv, last_u, last_v, row, word, kw, cell, sm, lane_sign,
                        s0, sink) &
                    m_moves;
         if (reported != 0) break;  // uniform
@@ -270,7 +486,7 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
         if (m_moves != __builtin_amdgcn_ballot_w64(true)) {  // uniform
           // a zero vector stays and has added its cell's value at
           // every step; an ended line adds nothing and records stops
-          acc = live_now ? acc : acc_0;
+          if (!live_now) acc = saved.acc();
           const uint32_t still = live_now ? kWordStay : 0x11111111u * kMoveStop;
 #pragma unroll
           for (int g = 0; g < 4; ++g) words[g] = moves_now || g >= full ? words[g] : still;
@@ -278,23 +494,18 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
         if (full == 0) {
           status_known = false;  // the full rule runs next
         } else {
-          alive = live_now;
           if (live_steps) *live_steps = live_now ? ch * kChunkSteps + 8 * full : *live_steps;
-          any_alive = __builtin_amdgcn_ballot_w64(alive) != 0;
+          any_alive = __builtin_amdgcn_ballot_w64(live_now) != 0;
         }
       } else {
-        const bool many = __popcll(reported) >= 8;
-        fast = ++misses < 2 && !many;
-        short_path = short_path && !many;
+        fast = sizeof(T) == 4 && g0 >= 2 && ++misses < 2 && __popcll(reported) < 8;
+        short_path = short_path && fast;
         status_known = false;
-        acc = acc_0;
-        fx = fx_0;
-        fy = fy_0;
-        pu = pu_0;
-        pv = pv_0;
-        last_u = lu_0;
-        last_v = lv_0;
+        saved.get(acc, fx, fy, last_u, last_v);
         row = row_0;
+        const CellVal<T> cv = cell(row);  // the vector there, not kept for this
+        pu = cv.u;
+        pv = cv.v;
         g0 = 0;
       }
     }
@@ -302,110 +513,15 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
     for (int g = g0; g < 4; ++g) {
       const int32_t s0 = ch * kChunkSteps + 8 * g;
       if (s0 >= nsteps || !any_alive) break;  // uniform
-      T kw[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q)
-        kw[q] = kernel[FORWARD ? kmid + 1 + s0 + q : kmid - 1 - s0 - q];
       uint32_t word = 0;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        if (s0 + q >= nsteps) break;  // uniform: last group only
-        // a NaN component ends the line (src/lib.rs:336-338)
-        const bool ordered = !__builtin_isunordered(pu, pv);
-        const bool live = alive && ordered;
-        if constexpr (pol) {  // src/lib.rs:339-347, unfused dot product
-          const T d1 = pu * last_u;
-          const T d2 = pv * last_v;
-          const bool flip = d1 + d2 < T(0);
-          pu = flip ? -pu : pu;
-          pv = flip ? -pv : pv;
-          last_u = pu;
-          last_v = pv;
-        }
-        // src/lib.rs:348-351
-        const T mu = LANE_DIR ? xor_sign(pu, lane_sign) : (FORWARD ? pu : -pu);
-        const T mv = LANE_DIR ? xor_sign(pv, lane_sign) : (FORWARD ? pv : -pv);
-        // sign tests of mu, mv read pu, pv (negation flips the sign bit), so
-        // that a backward step does not materialize -pu, -pv for them: the
-        // divisions and products take the negation as a source modifier
-        const bool neg_x = LANE_DIR  ? __builtin_signbit(mu)
-                           : FORWARD ? __builtin_signbit(pu)
-                                     : !__builtin_signbit(pu);
-        const bool neg_y = LANE_DIR  ? __builtin_signbit(mv)
-                           : FORWARD ? __builtin_signbit(pv)
-                                     : !__builtin_signbit(pv);
-        const T tx = time_to_next_pixel<T, FMA, BRANCHLESS>(mu, fx, neg_x);
-        const T ty = time_to_next_pixel<T, FMA, BRANCHLESS>(mv, fy, neg_y);
-        // x edge first when tx < ty; ties and NaN go to y (src/lib.rs:249-269)
-        const bool xs = tx < ty;
-        // no move when both components are +-0 (src/lib.rs:242-244)
-        const bool moves = live && (mu != T(0) || mv != T(0));
-        // update_state (src/lib.rs:208-233) for either axis, then keep one
-        // pos_x only matters when the x edge comes first (tx < ty), which
-        // needs a finite tx and so a nonzero, non-NaN mu: there it equals
-        // mu >= 0 (src/lib.rs:217), and the sign test is the one the step
-        // time already made.  pos_y is used for y steps, which also happen
-        // with mv = -0 (tx and ty both infinite), so it stays mv >= 0.
-        const bool pos_x = !neg_x;
-        const bool pos_y = LANE_DIR ? mv >= T(0) : FORWARD ? pv >= T(0) : pv <= T(0);  // mv >= 0
-        const T fy_after_x = macc<FMA>(tx, mv, fy);
-        const T fx_after_y = macc<FMA>(ty, mu, fx);
-        const T fx_new = xs ? (pos_x ? T(0) : T(1)) : fx_after_y;
-        const T fy_new = xs ? fy_after_x : (pos_y ? T(0) : T(1));
-        // The fractions need no "moves" gate: a lane that does not move
-        // never moves again (an ended line stays on its NaN cell, a zero
-        // vector stays on its cell, whose vector stays zero, polarization
-        // flips included), so its fractions are never read again: they only
-        // feed step times, whose results are masked out of its code bits and
-        // its position update.
-        fx = fx_new;
-        fy = fy_new;
-        // a y step leaves the row pair up from an odd row, down from an even one
-        const bool odd = (row & 1u) != 0u;
-        const uint32_t dist_y = !PAIRS || odd == pos_y || sg.all_far != 0u ? far_y : near_y;
-        const uint32_t step = xs ? (pos_x ? sg.step_x : 0u - sg.step_x)
-                                 : (pos_y ? dist_y : 0u - dist_y);
-        const uint32_t from = row;
-        const uint32_t at = moves ? row + step : row;
-        const CellVal<T> cv = cell(at);
-        const uint32_t jump = pad_bits(cv.pad);
-        const bool edge = jump != 0u;  // the step left the image
-        row = at + jump;
-        const T next_acc = macc<FMA>(kw[q], cv.x, acc);  // src/lib.rs:353-360
-        acc = live ? next_acc : acc;
-        sink(s0 + q, cv.x);
-        if (live_steps) *live_steps = live ? s0 + q + 1 : *live_steps;
-        pu = cv.u;
-        pv = cv.v;
-        if constexpr (rec) {
-          // The code's four bits (stay, negative direction, y axis, edge or
-          // stop) are combined from the step's comparisons as wave lane
-          // masks on the scalar unit, then shifted into the word one at a
-          // time with an add-with-carry (word = 2 * word + bit), so the
-          // group's first step ends in the top nibble (move_code).  A line
-          // that has ended stays on its NaN cell, so it records the stop
-          // code again at every later step; readers stop at the first one.
-          const uint64_t m_stop = ~__builtin_amdgcn_ballot_w64(ordered);
-          const uint64_t m_stay = __builtin_amdgcn_ballot_w64(row == from);
-          const uint64_t m_x = __builtin_amdgcn_ballot_w64(xs);
-          const uint64_t m_edge = __builtin_amdgcn_ballot_w64(edge);
-          const uint64_t m_neg = ~((m_x & __builtin_amdgcn_ballot_w64(pos_x)) |
-                                   (~m_x & __builtin_amdgcn_ballot_w64(pos_y)));
-          word = carry_in_bit(word, m_stay);
-          word = carry_in_bit(word, m_neg & ~m_stay);
-          word = carry_in_bit(word, ~m_x & ~m_stay);
-          word = carry_in_bit(word, (m_edge & ~m_stay) | m_stop);
-        }
-        alive = live;
-      }
-      // a last group of fewer than 8 steps: its first step to the top
-      // nibble, "stay" codes after its last
-      if (rec && nsteps - s0 < 8) {
-        const int32_t spare = 4 * (8 - (nsteps - s0));
-        word = (word << spare) | (kWordStay >> (32 - spare));
-      }
+      uint64_t m_live = 0;
+      full_group<T, FMA, BRANCHLESS, POL, FORWARD, REC, BUF, PAIRS, LANE_DIR,
+                 NARROW && sizeof(T) == 4>(
+          acc, fx, fy, pu, pv, last_u, last_v, row, m_live, word,
+          kernel + (FORWARD ? kmid + 1 + s0 : kmid - 1 - s0), cell, sl, lane_sign, s0,
+          min(8, nsteps - s0), sink, live_steps);
       words[g] = word;
-      any_alive = __builtin_amdgcn_ballot_w64(alive) != 0;
+      any_alive = m_live != 0;
     }
     if (rec) codes[(c0 + ch) * np + p] = make_uint4(words[0], words[1], words[2], words[3]);
     if (!any_alive) break;  // every line of the wave ended
