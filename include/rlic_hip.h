@@ -102,7 +102,10 @@ int rlic_convolve_f64(const double* texture, int64_t tex_sy, int64_t tex_sx,
  * checks run on the values that the call reads anyway.  *what = the bits of
  * rlic_check_values_*; unless it is 0, `out` holds nothing of use.  Returns
  * once the inputs are checked; the convolution may still be running on
- * `stream`. */
+ * `stream`, also that of refused inputs if it is small (fewer than 2^31 steps:
+ * pixels times kernel_len - 1 times passes, twice that in double).  Larger
+ * calls, and calls that measure replay plans, compute nothing on refused
+ * inputs. */
 int rlic_convolve_checked_f32(const float* texture, int64_t tex_sy, int64_t tex_sx,
                               const float* u, int64_t u_sy, int64_t u_sx,
                               const float* v, int64_t v_sy, int64_t v_sx,

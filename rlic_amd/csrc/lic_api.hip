@@ -556,9 +556,24 @@ struct FixedScratch {
 // lic_pack sets the two host-mapped flags, and `packed` is recorded after it.
 struct ValueCheck {
   uint32_t* dev_flags;
+  const volatile uint32_t* flags;  // the same on the host
   hipEvent_t packed;
   bool recorded;
+  // Waits for the flags: whether the values are refused.
+  hipError_t wait(bool& refused) {
+    const hipError_t e = hipEventSynchronize(packed);
+    refused = e == hipSuccess && (flags[0] != 0 || flags[1] != 0);
+    return e;
+  }
 };
+
+// A call of at least this many steps (a double one counts twice) is checked
+// before it is traced, so that refused values cost nothing more: it takes a
+// millisecond at least, and the GPU's wait for the host is lost in it (4096^2, L =
+// 129, 5 passes: 3546 us with and without).  Smaller calls are enqueued whole and
+// then checked, which is why they are fast (convolve_checked_entry); what a
+// refused one of them still runs takes less than 2 ms.
+constexpr int64_t kCheckFirstSteps = int64_t{1} << 31;
 
 // The paired trace (two lanes per pixel, one per direction) where a field
 // has too few pixels to fill the GPU with lic_trace's one lane per pixel:
@@ -650,6 +665,7 @@ int run_on_device(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
       bounds ? reinterpret_cast<rlic::ReplayBounds*>(base + off_codes + code_bytes) : nullptr,
       false};
   const uint32_t epoch = rlic::next_epoch();
+  if (check) check->recorded = true;  // also if a launch fails: the caller waits for the stream
   {
     // the cells and the padded weight copy in one launch
     LaunchTimer timer("lic_pack", stream);
@@ -658,9 +674,14 @@ int run_on_device(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
                                       check ? check->dev_flags : nullptr),
                  "pack");
   }
+  bool refused = false;
   if (check) {
-    check->recorded = true;  // also if the record fails: the caller then waits for the stream
     RLIC_HIP_TRY(hipEventRecord(check->packed, stream), "recording the value checks");
+    const int64_t per_pass = n * (klen - 1) * static_cast<int64_t>(sizeof(T) / 4);
+    if (per_pass > 0 && iterations >= (kCheckFirstSteps + per_pass - 1) / per_pass) {
+      RLIC_HIP_TRY(check->wait(refused), "checking values");
+      if (refused) return RLIC_OK;
+    }
   }
   kernel = kpad + pad;
   // trace tiles of 32 x 8 pixels (16 x 4 per wave) in XCD bands of 64
@@ -716,6 +737,9 @@ int run_on_device(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
       if (hit != g_tuner.table.end()) {
         if (plan_usable<T>(hit->second.plan, klen, g, record)) plan = hit->second.plan;
       } else if (!fixed) {
+        // nothing is measured on values that will be refused
+        if (check) RLIC_HIP_TRY(check->wait(refused), "checking values");
+        if (refused) return RLIC_OK;
         const std::vector<ReplayPlan> cands = replay_candidates<T>(klen, g, record);
         TuneEntry best{plan, -1.f};
         RLIC_HIP_TRY(tune_replay<T>(cands, a, b, kernel, klen, g, profile, record, stream, best),
@@ -1169,7 +1193,7 @@ int64_t server_field_bytes(int64_t ny, int64_t nx, int64_t klen, int keep, int64
 int noalloc_scratch_ptr(void** ptr);
 
 // rlic_convolve_checked_*: the element checks and the convolution enqueued
-// together.  A check call of its own leaves the GPU idle while the host waits
+// together (but kCheckFirstSteps).  A check call of its own leaves the GPU idle while the host waits
 // for it and then launches (97 x 61 float: 41 us a call against 28; 256^2
 // double 48 against 28), and reads the texture once more.
 template <typename T>
@@ -1197,7 +1221,8 @@ int convolve_checked_entry(const T* tex, int64_t tsy, int64_t tsx, const T* u, i
   char* dev = nullptr;
   RLIC_HIP_TRY(pinned_words(2 * sizeof(uint32_t), &host, &dev), "allocating the check flags");
   std::memset(host, 0, 2 * sizeof(uint32_t));
-  ValueCheck check{reinterpret_cast<uint32_t*>(dev), nullptr, false};
+  ValueCheck check{reinterpret_cast<uint32_t*>(dev), reinterpret_cast<uint32_t*>(host), nullptr,
+                   false};
   RLIC_HIP_TRY(hipEventCreateWithFlags(&check.packed, hipEventDisableTiming),
                "creating the check's event");
   const int rc = convolve_entry<T>(tex, tsy, tsx, u, usy, usx, v, vsy, vsx, ny, nx, kernel, klen,
@@ -1206,8 +1231,7 @@ int convolve_checked_entry(const T* tex, int64_t tsy, int64_t tsx, const T* u, i
   hipError_t e = hipSuccess;
   if (check.recorded) {  // the flags are written until then
     e = rc == RLIC_OK ? hipEventSynchronize(check.packed) : hipStreamSynchronize(stream);
-    const volatile uint32_t* flags = reinterpret_cast<uint32_t*>(host);
-    *what = (flags[0] ? 1 : 0) | (flags[1] ? 2 : 0);
+    *what = (check.flags[0] ? 1 : 0) | (check.flags[1] ? 2 : 0);
   }
   (void)hipEventDestroy(check.packed);
   if (rc == RLIC_OK) RLIC_HIP_TRY(e, "checking values");
