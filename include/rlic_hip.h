@@ -350,10 +350,12 @@ int rlic_trace_stats_read(int64_t* live_lane_steps, int64_t* executed_lane_steps
 
 /* Replay autotuner.  No counterpart in the reference (one CPU loop).  The
  * first rlic_convolve_* call with at least 3 passes on at least 2^18 pixels
- * for a new (dtype, shape, kernel length, profile) times its second pass
- * under each candidate plan — LDS-staged replay with every tile whose box
- * (tile + kernel-half-length halo) fits the LDS, and L2-gather replay with
- * two tile strip heights — and later calls with that key use the fastest.
+ * for a new (dtype, shape, kernel length, profile, boxes) times its second
+ * pass under each candidate plan — boxes cut to the lines where there are
+ * enough passes to replay for them (boxes), LDS-staged replay with every tile
+ * whose box (tile + kernel-half-length halo) fits the LDS, and L2-gather
+ * replay with two tile strip heights — and later calls with that key use the
+ * fastest.
  * Every plan gives the same bits.  RLIC_AUTOTUNE=0 disables tuning;
  * RLIC_AUTOTUNE_CACHE=<file> loads the table from and appends it to a text
  * file.  rlic_autotune_read writes the table as a JSON list (same buffer

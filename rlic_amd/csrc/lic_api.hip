@@ -283,15 +283,18 @@ ReplayPlan default_plan(int32_t klen, const rlic::FieldGeom& g, const Record& re
 }
 
 // Replay autotuner.  The first call with at least 3 passes on a field of at
-// least 2^18 pixels for a new (dtype, shape, kernel length, profile) times
-// its pass 2 under every candidate plan — each LDS tile whose box fits
-// (64x64, 32x64, 32x32), the hybrid when it applies, and L2 gathers with
-// two strip heights — on the
-// caller's stream with HIP events (all candidates write the same bits), and
-// keeps the fastest for that key.  RLIC_AUTOTUNE=0 disables it;
-// RLIC_AUTOTUNE_CACHE=<file> loads and appends the table as text.
+// least 2^18 pixels for a new (dtype, shape, kernel length, profile, boxes)
+// times its pass 2 under every candidate plan — boxes cut to the lines where
+// box_allowed (`boxes`, which depends on the number of passes: a plan measured
+// without that candidate says nothing to a call that has it), each LDS tile
+// whose box fits (64x64, 32x64, 32x32), the hybrid when it applies, and L2
+// gathers with two strip heights — on the caller's stream with HIP events (all
+// candidates write the same bits), and keeps the fastest for that key.
+// RLIC_AUTOTUNE=0 disables it; RLIC_AUTOTUNE_CACHE=<file> loads and appends the
+// table as text, a line each: the key without `boxes`, the plan, its time, and
+// "boxes 0" or "boxes 1" (a line without it: 1 for the box plan).
 struct TuneKey {
-  int32_t dtype_size, ny, nx, klen, profile;
+  int32_t dtype_size, ny, nx, klen, profile, boxes;
   bool operator<(const TuneKey& o) const { return std::memcmp(this, &o, sizeof(*this)) < 0; }
 };
 struct TuneEntry {
@@ -316,6 +319,7 @@ int64_t tuner_read_file_locked(const char* path) {
   while (std::fscanf(f, " rlic-replay-plan %d %d %d %d %d %d %d %d %d %d %f", &k.dtype_size,
                      &k.ny, &k.nx, &k.klen, &k.profile, &e.plan.lds, &e.plan.th, &e.plan.tw,
                      &e.plan.band, &e.plan.wave_w_log2, &e.ms) == 11) {
+    if (std::fscanf(f, " boxes %d", &k.boxes) != 1) k.boxes = is_box_plan(e.plan) ? 1 : 0;
     g_tuner.table[k] = e;
     ++count;
   }
@@ -352,9 +356,9 @@ void tuner_store_locked(const TuneKey& k, const TuneEntry& e) {
   const char* path = std::getenv("RLIC_AUTOTUNE_CACHE");
   if (!path || !*path) return;
   if (FILE* f = std::fopen(path, "a")) {
-    std::fprintf(f, "rlic-replay-plan %d %d %d %d %d %d %d %d %d %d %.6f\n", k.dtype_size, k.ny,
-                 k.nx, k.klen, k.profile, e.plan.lds, e.plan.th, e.plan.tw, e.plan.band,
-                 e.plan.wave_w_log2, e.ms);
+    std::fprintf(f, "rlic-replay-plan %d %d %d %d %d %d %d %d %d %d %.6f boxes %d\n", k.dtype_size,
+                 k.ny, k.nx, k.klen, k.profile, e.plan.lds, e.plan.th, e.plan.tw, e.plan.band,
+                 e.plan.wave_w_log2, e.ms, k.boxes);
     std::fclose(f);
   }
 }
@@ -730,7 +734,8 @@ int run_on_device(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
     if (env_int("RLIC_AUTOTUNE", 1) != 0 && iterations >= 3 && n >= (int64_t{1} << 18)) {
       // an allocation-free call uses a tuned plan when the table has one,
       // and never tunes (the timing events are HIP objects)
-      const TuneKey key{static_cast<int32_t>(sizeof(T)), ny, nx, klen, profile};
+      const TuneKey key{static_cast<int32_t>(sizeof(T)), ny, nx, klen, profile,
+                        record.bounds != nullptr ? 1 : 0};
       std::lock_guard<std::mutex> lock(g_tuner.mu);
       tuner_load_locked();
       auto hit = g_tuner.table.find(key);
@@ -1823,11 +1828,10 @@ int64_t rlic_autotune_read(char* buf, int64_t len) {
     snprintf(item, sizeof(item),
              "%s{\"dtype_size\": %d, \"ny\": %d, \"nx\": %d, \"kernel_len\": %d, \"profile\": %d, "
              "\"replay\": \"%s\", \"tile\": [%d, %d], \"band\": %d, \"wave_w_log2\": %d, "
-             "\"pass_ms\": %.6f}",
+             "\"pass_ms\": %.6f, \"boxes\": %s}",
              first ? "" : ", ", k.dtype_size, k.ny, k.nx, k.klen, k.profile,
              e.plan.lds == 2 ? "lds_hybrid" : (e.plan.lds ? "lds" : "l2"), e.plan.th, e.plan.tw,
-             e.plan.band, e.plan.wave_w_log2,
-             e.ms);
+             e.plan.band, e.plan.wave_w_log2, e.ms, k.boxes ? "true" : "false");
     json += item;
     first = false;
   }
