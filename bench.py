@@ -83,6 +83,20 @@ def valu_from_profiles(kernel: str, workload: str) -> dict | None:
         return None
 
 
+def by_kernel(prof: dict) -> dict:
+    """A launch profile with the replays from boxes cut to the lines
+    (lic_replay_box) apart from the other ones from LDS."""
+    prof = dict(prof)
+    lds = prof.get("lic_replay_lds", {})
+    if lds.get("box_count"):
+        prof["lic_replay_box"] = {"count": lds["box_count"], "total_ms": lds["box_ms"]}
+        rest = {"count": lds["count"] - lds["box_count"], "total_ms": lds["total_ms"] - lds["box_ms"]}
+        del prof["lic_replay_lds"]
+        if rest["count"]:
+            prof["lic_replay_lds"] = rest
+    return prof
+
+
 def measure_copy_gbs(dev, repeats: int = 10) -> float:
     """Measured HBM bandwidth of a plain device copy (STREAM copy): PyTorch's
     copy of 2^28 float32 (1 GiB read, 1 GiB written), timed with events on
@@ -185,7 +199,7 @@ def batch_measure(dev, steps: int, warmup: int, small: bool = False) -> dict:
     _native.profiler_read()
     batched()
     torch.cuda.synchronize()
-    prof = _native.profiler_read()
+    prof = by_kernel(_native.profiler_read())
     _native.profiler_enable(False)
     del fields
     torch.cuda.empty_cache()
@@ -397,7 +411,7 @@ def single_call_measure(wl, dev, steps: int, warmup: int) -> dict:
     _native.profiler_read()
     step()
     torch.cuda.synchronize()
-    prof = _native.profiler_read()
+    prof = by_kernel(_native.profiler_read())
     _native.profiler_enable(False)
     ny, nx = wl.shape
     return {"workload": wl.name, "shape": [ny, nx], "kernel_len": wl.kernel_len,
@@ -568,7 +582,7 @@ def main() -> int:
         step()
     torch.cuda.synchronize()
     elapsed = time.perf_counter() - t0
-    prof = _native.profiler_read()
+    prof = by_kernel(_native.profiler_read())
     _native.profiler_enable(False)
     log(f"bench: kernel times {json.dumps(prof)}")
 

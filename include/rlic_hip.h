@@ -331,8 +331,9 @@ const char* rlic_last_error(void);
  * rlic_profiler_enable(1): every later kernel launch of the library is
  * bracketed by two hipEvents recorded on the stream it runs on.
  * rlic_profiler_read: resolves the recorded events (waits for them),
- * writes a JSON object {"<kernel>": {"count": n, "total_ms": t}, ...} into
- * buf (NUL-terminated) and clears the record when len is large enough,
+ * writes a JSON object {"<kernel>": {"count": n, "total_ms": t}, ...}
+ * ("lic_replay_lds", the replays from LDS, also with "box_count" and "box_ms",
+ * those of them that are lic_replay_box launches) into buf (NUL-terminated) and clears the record when len is large enough,
  * keeps the record otherwise (e.g. buf == NULL to size the buffer), and
  * returns the number of bytes needed including the NUL. */
 int rlic_profiler_enable(int on);
@@ -345,7 +346,9 @@ int64_t rlic_profiler_read(char* buf, int64_t len);
  * streamline was alive and the steps its wave executed (a wave runs until
  * all its lanes' lines have ended).  rlic_trace_stats_read returns the two
  * sums accumulated since the last read and resets them; their ratio is the
- * lane efficiency lost to uneven streamline termination. */
+ * lane efficiency lost to uneven streamline termination.  (Steps that a wave
+ * did twice, by the trace's short path and then by its full rule, count
+ * once.) */
 int rlic_trace_stats_read(int64_t* live_lane_steps, int64_t* executed_lane_steps);
 
 /* Replay autotuner.  No counterpart in the reference (one CPU loop).  The

@@ -199,7 +199,14 @@ hipError_t launch_plan(const ReplayPlan& p, const T* src, T* dst, const T* kerne
   return rlic::launch_replay<T>(src, kernel, klen, g, m, profile, dst, codes, stream);
 }
 
-const char* plan_kernel_name(const ReplayPlan& p) { return p.lds ? "lic_replay_lds" : "lic_replay"; }
+constexpr char kBoxKernel[] = "lic_replay_box";
+const char* plan_kernel_name(const ReplayPlan& p) {
+  return is_box_plan(p) ? kBoxKernel : p.lds ? "lic_replay_lds" : "lic_replay";
+}
+// The plan's name in the autotuner's table.
+const char* plan_name(const ReplayPlan& p) {
+  return is_box_plan(p) ? "lds_box" : p.lds == 2 ? "lds_hybrid" : p.lds ? "lds" : "l2";
+}
 
 // LDS plans stage a box per tile (192 x 192 for a 64 x 64 float tile at
 // kmid 64) whatever the image size.  Below 2^18 pixels (512 x 512) the
@@ -1763,14 +1770,30 @@ int64_t rlic_profiler_read(char* buf, int64_t len) {
     (void)hipEventDestroy(t.stop);
   }
   g_prof_pending.clear();
+  // box launches are told apart within the replays from LDS
+  std::map<std::string, std::pair<int64_t, double>> all = g_prof_done;
+  std::pair<int64_t, double> boxes{0, 0.0};
+  if (auto box = all.find(kBoxKernel); box != all.end()) {
+    boxes = box->second;
+    all.erase(box);
+    auto& lds = all["lic_replay_lds"];
+    lds.first += boxes.first;
+    lds.second += boxes.second;
+  }
   std::string json = "{";
   bool first = true;
-  for (const auto& kv : g_prof_done) {
-    char item[256];
-    snprintf(item, sizeof(item), "%s\"%s\": {\"count\": %lld, \"total_ms\": %.6f}",
+  for (const auto& kv : all) {
+    char item[320];
+    snprintf(item, sizeof(item), "%s\"%s\": {\"count\": %lld, \"total_ms\": %.6f",
              first ? "" : ", ", kv.first.c_str(), static_cast<long long>(kv.second.first),
              kv.second.second);
     json += item;
+    if (kv.first == "lic_replay_lds") {
+      snprintf(item, sizeof(item), ", \"box_count\": %lld, \"box_ms\": %.6f",
+               static_cast<long long>(boxes.first), boxes.second);
+      json += item;
+    }
+    json += "}";
     first = false;
   }
   json += "}";
@@ -1830,8 +1853,8 @@ int64_t rlic_autotune_read(char* buf, int64_t len) {
              "\"replay\": \"%s\", \"tile\": [%d, %d], \"band\": %d, \"wave_w_log2\": %d, "
              "\"pass_ms\": %.6f, \"boxes\": %s}",
              first ? "" : ", ", k.dtype_size, k.ny, k.nx, k.klen, k.profile,
-             e.plan.lds == 2 ? "lds_hybrid" : (e.plan.lds ? "lds" : "l2"), e.plan.th, e.plan.tw,
-             e.plan.band, e.plan.wave_w_log2, e.ms, k.boxes ? "true" : "false");
+             plan_name(e.plan), e.plan.th, e.plan.tw, e.plan.band, e.plan.wave_w_log2, e.ms,
+             k.boxes ? "true" : "false");
     json += item;
     first = false;
   }

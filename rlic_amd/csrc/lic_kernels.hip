@@ -209,8 +209,9 @@ __global__ __launch_bounds__(64) void lic_trace_pair(
 // group with its position frozen.  Per wave and direction this kernel finds
 // each lane's first stop code (the step where its line ended), and adds
 // the lanes' live steps to stats[0] and the steps the wave executed, times
-// the lanes that hold a pixel, to stats[1].  Same block and lane mapping as
-// lic_trace.
+// the lanes that hold a pixel, to stats[1].  A wave holds the pixels of one of
+// lic_trace's.  What the record does not tell is left out: groups of the short
+// path that were done again by the full rule.
 __global__ __launch_bounds__(256) void lic_record_stats(const uint4* __restrict__ codes,
                                                         int32_t klen, FieldGeom g, TileMap m,
                                                         unsigned long long* __restrict__ stats) {

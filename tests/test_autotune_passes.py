@@ -71,3 +71,34 @@ def test_tables_with_and_without_the_mark(tmp_path):
     got = {(e["nx"], e["boxes"]): e["pass_ms"] for e in _native.autotune_table()}
     assert got == {(600, False): 0.5, (600, True): 0.25, (700, True): 0.25, (700, False): 0.75}
     _native.autotune_clear()
+
+
+@pytest.mark.gpu
+def test_box_replays_are_told_apart(monkeypatch, tmp_path):
+    import torch
+
+    monkeypatch.setenv("RLIC_REPLAY_LDS", "1")
+    monkeypatch.setenv("RLIC_REPLAY_BOX", "2")
+    monkeypatch.setenv("RLIC_AUTOTUNE", "0")
+    rng = np.random.default_rng(8)
+    t = lambda *s: torch.from_numpy(rng.random(s).astype(np.float32)).to("cuda:0")  # noqa: E731
+    _native.profiler_enable(True)
+    _native.profiler_read()
+    try:
+        rlic_amd.convolve(t(90, 70), t(90, 70), t(90, 70), kernel=t(33), iterations=4)
+        ran = _native.profiler_read()
+    finally:
+        _native.profiler_enable(False)
+    assert {k for k in ran if "replay" in k} == {"lic_replay_lds"}
+    replays = ran["lic_replay_lds"]
+    assert replays["count"] == replays["box_count"] == 3
+    assert replays["box_ms"] == replays["total_ms"] > 0
+
+
+def test_the_box_plan_has_a_name(tmp_path):
+    path = tmp_path / "plans.txt"
+    path.write_text("rlic-replay-plan 4 512 600 129 3 2 32 32 0 0 0.25\n")
+    _native.autotune_clear()
+    assert _native.autotune_load(path) == 1
+    assert [e["replay"] for e in _native.autotune_table()] == ["lds_box"]
+    _native.autotune_clear()
