@@ -376,6 +376,17 @@ int rlic_autotune_clear(void);
  * counterpart in the reference; for tests. */
 int rlic_div_check_f32(const float* a, const float* b, float* q, int64_t n, void* stream);
 
+/* The same for the shorter quotient that the trace takes where velocities and
+ * numerators are in its range (float: a 0 or 2^-60..2, b 2^-60..2^40; double: a
+ * 0 or 2^-300..2, b 2^-300..2^150): it equals a[i] / b[i] there.
+ * rlic_quotient_sweep_f32: every pair of a numerator mantissa in
+ * [first, first + count) (of 2^23) and a divisor mantissa; the number of
+ * quotients that are not correctly rounded is added to *wrong (device memory).
+ * Synchronous; for tests. */
+int rlic_quotient_check_f32(const float* a, const float* b, float* q, int64_t n, void* stream);
+int rlic_quotient_check_f64(const double* a, const double* b, double* q, int64_t n, void* stream);
+int rlic_quotient_sweep_f32(int64_t first, int64_t count, uint64_t* wrong, void* stream);
+
 /* Scratch memory.  A call's device scratch (packed cells, move record,
  * ping-pong buffer, queue descriptors) is one block; blocks up to 256 MiB
  * are cached per (device, stream) and reused by later calls on that stream.

@@ -1199,6 +1199,17 @@ int64_t server_field_bytes(int64_t ny, int64_t nx, int64_t klen, int keep, int64
       rlic::Server::field_bytes<T>(ny, nx, klen, keep != 0 || iterations > 1));
 }
 
+template <typename T>
+int quotient_check(const T* a, const T* b, T* q, int64_t n, void* stream) {
+  t_last_error.clear();
+  if (n < 0 || (n > 0 && (!a || !b || !q)))
+    return set_error(RLIC_ERR_INVALID_ARGUMENT, "invalid argument");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  RLIC_HIP_TRY(rlic::launch_quotient_check<T>(a, b, q, n, s), "quotient check");
+  RLIC_HIP_TRY(hipStreamSynchronize(s), "quotient check");
+  return RLIC_OK;
+}
+
 // Allocation-free convolve: the same checks and computation as
 // convolve_entry with device arrays, its scratch in the fixed device array
 // (see rlic_convolve_noalloc_* below).
@@ -1812,6 +1823,29 @@ int rlic_div_check_f32(const float* a, const float* b, float* q, int64_t n, void
   hipStream_t s = static_cast<hipStream_t>(stream);
   RLIC_HIP_TRY(rlic::launch_div_check(a, b, q, n, s), "division check");
   RLIC_HIP_TRY(hipStreamSynchronize(s), "division check");
+  return RLIC_OK;
+}
+
+int rlic_quotient_check_f32(const float* a, const float* b, float* q, int64_t n, void* stream) {
+  return quotient_check<float>(a, b, q, n, stream);
+}
+
+int rlic_quotient_check_f64(const double* a, const double* b, double* q, int64_t n, void* stream) {
+  return quotient_check<double>(a, b, q, n, stream);
+}
+
+int rlic_quotient_sweep_f32(int64_t first, int64_t count, uint64_t* wrong, void* stream) {
+  t_last_error.clear();
+  if (first < 0 || count < 0 || count > int64_t{1} << 23 || first > (int64_t{1} << 23) - count ||
+      !wrong)
+    return set_error(RLIC_ERR_INVALID_ARGUMENT, "invalid argument");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  static_assert(sizeof(uint64_t) == sizeof(unsigned long long));
+  RLIC_HIP_TRY(rlic::launch_quotient_sweep(static_cast<uint32_t>(first),
+                                           static_cast<uint32_t>(count),
+                                           reinterpret_cast<unsigned long long*>(wrong), s),
+               "quotient sweep");
+  RLIC_HIP_TRY(hipStreamSynchronize(s), "quotient sweep");
   return RLIC_OK;
 }
 

@@ -386,7 +386,8 @@ __device__ __forceinline__ double copy_sign_of(double x, double s) {
 // exact remainder, correction: Markstein 1990) without its scaling and
 // special cases.  In float one Newton step and one correction do: every pair
 // of 23-bit mantissas was tried on gfx950 against the remainder test (2^46
-// pairs, none wrong); scaling by powers of two is exact in between.  In
+// pairs, none wrong: tests/test_quotient.py); scaling by powers of two is exact
+// in between.  In
 // double these are the steps of hipcc's own division.
 __device__ __forceinline__ float quotient_rn(float n, float d) {
   const float y0 = __builtin_amdgcn_rcpf(d);

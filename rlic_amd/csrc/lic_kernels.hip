@@ -835,6 +835,48 @@ hipError_t launch_div_check(const float* a, const float* b, float* q, int64_t n,
   return hipGetLastError();
 }
 
+template <typename T>
+__global__ __launch_bounds__(256) void lic_quotient_check(const T* __restrict__ a,
+                                                          const T* __restrict__ b,
+                                                          T* __restrict__ q, int64_t n) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i < n) q[i] = quotient_rn(a[i], b[i]);
+}
+
+template <typename T>
+hipError_t launch_quotient_check(const T* a, const T* b, T* q, int64_t n, hipStream_t stream) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(lic_quotient_check<T>, dim3(static_cast<unsigned>((n + 255) / 256)),
+                     dim3(256), 0, stream, a, b, q, n);
+  return hipGetLastError();
+}
+
+// A thread per divisor mantissa, `count` numerator mantissas from `first` on:
+// the quotient is the correctly rounded one if it is off by less than half a unit
+// in its last place, as the exact remainder tells (no quotient lies half way).
+__global__ __launch_bounds__(256) void lic_quotient_sweep(uint32_t first, uint32_t count,
+                                                          unsigned long long* wrong) {
+  const uint32_t mantissa = blockIdx.x * 256 + threadIdx.x;  // below 2^23
+  const float d = __builtin_bit_cast(float, 0x3F800000u | mantissa);
+  uint32_t bad = 0;
+  for (uint32_t k = 0; k < count; ++k) {
+    const float n = __builtin_bit_cast(float, 0x3F800000u | (first + k));
+    const float q = quotient_rn(n, d);
+    const float r = fma_t(-q, d, n);
+    const bool below_1 = q < 1.0f || (q == 1.0f && r < 0.0f);
+    bad += abs_t(r) < d * (below_1 ? 0x1p-25f : 0x1p-24f) ? 0u : 1u;
+  }
+  if (bad != 0) atomicAdd(wrong, static_cast<unsigned long long>(bad));
+}
+
+hipError_t launch_quotient_sweep(uint32_t first, uint32_t count, unsigned long long* wrong,
+                                 hipStream_t stream) {
+  if (count == 0) return hipSuccess;
+  hipLaunchKernelGGL(lic_quotient_sweep, dim3((1u << 23) / 256), dim3(256), 0, stream, first,
+                     count, wrong);
+  return hipGetLastError();
+}
+
 hipError_t launch_record_stats(const uint4* codes, int32_t klen, const FieldGeom& g,
                                const TileMap& m, unsigned long long* stats, hipStream_t stream) {
   hipLaunchKernelGGL(lic_record_stats, dim3(m.n_tiles), dim3(kBlock), 0, stream, codes, klen, g,
@@ -996,6 +1038,7 @@ hipError_t launch_replay_lds_hybrid(const T* x, const T* kernel, int32_t klen, c
   template hipError_t launch_replay<T>(const T*, const T*, int32_t, const FieldGeom&,          \
                                        const TileMap&, int, T*, const uint4*, hipStream_t);    \
   template void choose_row_order<T>(FieldGeom&);                                               \
+  template hipError_t launch_quotient_check<T>(const T*, const T*, T*, int64_t, hipStream_t);  \
   template bool lds_replay_fits<T>(int32_t);                                                   \
   template bool trace_pair_fits<T>(int32_t, const FieldGeom&);                                 \
   template hipError_t launch_trace_pair<T>(const Cell<T>*, const T*, int32_t, const FieldGeom&, \

@@ -95,6 +95,13 @@ hipError_t launch_fill_modes(T* out, int32_t ny, int32_t nx, const ModeSet& mode
 // q[i] = a[i] / b[i] with the streamline kernels' float division (a check).
 hipError_t launch_div_check(const float* a, const float* b, float* q, int64_t n,
                             hipStream_t stream);
+// The same with quotient_rn; and for numerator mantissas [first, first + count)
+// and every divisor mantissa, the number of float quotients that are not
+// correctly rounded, added to *wrong.
+template <typename T>
+hipError_t launch_quotient_check(const T* a, const T* b, T* q, int64_t n, hipStream_t stream);
+hipError_t launch_quotient_sweep(uint32_t first, uint32_t count, unsigned long long* wrong,
+                                 hipStream_t stream);
 
 // Adds the live lane-steps (stats[0]) and executed lane-steps (stats[1]) of
 // a tracing pass with tile map m, read from its move record.
