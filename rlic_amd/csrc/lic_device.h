@@ -325,7 +325,8 @@ __device__ __forceinline__ bool velocity_wide(T w) {
 // cell (0, 0), which no step reaches.  Each packing of a field has its own
 // `epoch`; a packing thread that sees a wide component stores the epoch
 // there, so the word needs no clearing before (a stale word that happens to
-// equal the epoch only costs the short path).
+// equal the epoch only costs the short path), but in a captured graph
+// (launch_clear_mark).
 template <typename T>
 __device__ __forceinline__ bool wide_mark(const Cell<T>* cells, uint32_t epoch) {
   return *reinterpret_cast<const uint32_t*>(cells) == epoch;

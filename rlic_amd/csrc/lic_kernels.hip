@@ -694,7 +694,19 @@ void choose_row_order(FieldGeom& g) {
 
 uint32_t next_epoch() {
   static std::atomic<uint32_t> epoch{0};
-  return epoch.fetch_add(1, std::memory_order_relaxed) + 1;
+  for (;;) {
+    const uint32_t e = epoch.fetch_add(1, std::memory_order_relaxed) + 1;
+    if (e != 0) return e;
+  }
+}
+
+__global__ void lic_clear_mark(uint32_t* mark) { *mark = 0u; }
+
+template <typename T>
+hipError_t launch_clear_mark(Cell<T>* cells, hipStream_t stream) {
+  hipLaunchKernelGGL(lic_clear_mark, dim3(1), dim3(1), 0, stream,
+                     reinterpret_cast<uint32_t*>(cells));
+  return hipGetLastError();
 }
 
 template <typename T>
@@ -1028,6 +1040,7 @@ hipError_t launch_replay_lds_hybrid(const T* x, const T* kernel, int32_t klen, c
   template hipError_t launch_pack<T>(const T*, int64_t, int64_t, const T*, int64_t, int64_t,   \
                                      const T*, int64_t, int64_t, const FieldGeom&, Cell<T>*,   \
                                      uint32_t, hipStream_t, const T*, int32_t, T*, uint32_t*);  \
+  template hipError_t launch_clear_mark<T>(Cell<T>*, hipStream_t);                             \
   template hipError_t launch_repack_texture<T>(const T*, const FieldGeom&, Cell<T>*,           \
                                                hipStream_t);                                    \
   template hipError_t launch_copy2d<T>(const T*, int64_t, int64_t, int32_t, int32_t, T*,       \
