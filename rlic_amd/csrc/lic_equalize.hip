@@ -14,15 +14,17 @@
 //     when vmax == vmin every finite pixel is in bin 0;
 //   * out = cdf[bin] / N in double, rounded once to the image type.
 //
-// Five stream-ordered launches, no host round trip: the finite range (one
+// Four stream-ordered launches, no host round trip: the finite range (one
 // read of the image; a partial result per block on order-preserving integer
-// keys), their reduction (which also clears the counters), the histogram (a
-// second read; per-block LDS histograms merged with global atomics), an
-// inclusive scan of the counts (one block), and the map (a third read and
-// the write).  All of it is integer and HBM traffic: 3 reads and 1 write of
-// the image.  4096^2 floats, 256 bins: range 16, histogram 20, map 28 us, 70 us
-// a call (87, 74, 44 and 213 with an atomic per block on the range, 8 blocks
-// per CU on the counters and a division per pixel).
+// keys; it also clears the counters), the histogram (a second read; every block
+// reduces the partial ranges, and its LDS histograms are merged with global
+// atomics), an inclusive scan of the counts (one block), and the map (a third
+// read and the write).  All of it is integer and HBM traffic: 3 reads and 1
+// write of the image; below about 512^2 pixels the launches (256^2, 256 bins:
+// 20.5 us a call, 23.6 with a launch for the reduction).  4096^2 floats, 256
+// bins: range 16, histogram 20, map 28 us, 65 us a call (87, 74, 44 and 207 with
+// an atomic per block on the range, 8 blocks per CU on the counters and a
+// division per pixel).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -116,16 +118,16 @@ __device__ __forceinline__ int32_t eq_bin(double x, const EqRange& r, int32_t nb
 // The range and scale of the binning, from the reduced keys (every thread
 // computes the same values).
 template <typename T>
-__device__ __forceinline__ EqRange read_range(const EqState<T>* st, int32_t nbins) {
+__device__ __forceinline__ EqRange read_range(const EqState<T>& st, int32_t nbins) {
   EqRange r;
-  r.count = st->count;
+  r.count = st.count;
   r.constant = true;
   r.halves = false;
   r.lo = 0.0;
   r.scale = 0.0;
   if (r.count == 0) return r;
-  const double vmin = static_cast<double>(from_key(st->min_key));
-  const double vmax = static_cast<double>(from_key(st->max_key));
+  const double vmin = static_cast<double>(from_key(st.min_key));
+  const double vmax = static_cast<double>(from_key(st.max_key));
   if (!(vmax > vmin)) return r;
   r.constant = false;
   const double d = vmax - vmin;
@@ -140,11 +142,12 @@ __device__ __forceinline__ EqRange read_range(const EqState<T>* st, int32_t nbin
   return r;
 }
 
-// The block's smallest and largest key and count, in thread 0's arguments.
+// The block's smallest and largest key and count, from its threads', in every
+// thread.  `waves` holds one state for each of the block's waves.
 template <typename T>
-__device__ __forceinline__ void reduce_range(typename KeyOf<T>::type& lo,
-                                             typename KeyOf<T>::type& hi,
-                                             unsigned long long& cnt) {
+__device__ __forceinline__ EqState<T> reduce_range(typename KeyOf<T>::type lo,
+                                                   typename KeyOf<T>::type hi,
+                                                   unsigned long long cnt, EqState<T>* waves) {
   typedef typename KeyOf<T>::type Key;
   for (int off = 32; off > 0; off >>= 1) {
     const Key olo = __shfl_xor(lo, off), ohi = __shfl_xor(hi, off);
@@ -152,52 +155,49 @@ __device__ __forceinline__ void reduce_range(typename KeyOf<T>::type& lo,
     hi = ohi > hi ? ohi : hi;
     cnt += __shfl_xor(cnt, off);
   }
-  __shared__ Key s_lo[kThreads / 64], s_hi[kThreads / 64];
-  __shared__ unsigned long long s_cnt[kThreads / 64];
-  const int32_t w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    s_lo[w] = lo;
-    s_hi[w] = hi;
-    s_cnt[w] = cnt;
-  }
+  if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = EqState<T>{lo, hi, cnt};
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int k = 1; k < kThreads / 64; ++k) {
-      lo = s_lo[k] < lo ? s_lo[k] : lo;
-      hi = s_hi[k] > hi ? s_hi[k] : hi;
-      cnt += s_cnt[k];
-    }
+  EqState<T> all = waves[0];
+  for (int32_t k = 1; k < static_cast<int32_t>(blockDim.x >> 6); ++k) {
+    all.min_key = waves[k].min_key < all.min_key ? waves[k].min_key : all.min_key;
+    all.max_key = waves[k].max_key > all.max_key ? waves[k].max_key : all.max_key;
+    all.count += waves[k].count;
   }
+  return all;
 }
 
-// The blocks' ranges to the image's (block 0), and the counters to zero.
-// (One atomic per block on the range's three words cost 60 us of a 4096^2
-// image's 80: 2048 blocks on one cache line.)
+// The image's range from its blocks' (st[1] on), in every thread; for the
+// launches that follow, in st[0].  Every block reduces them for itself: a
+// launch for it is 3 us more, and one atomic per block on the range's three
+// words cost 60 us of a 4096^2 image's 80 (2048 blocks on one cache line).
 template <typename T>
-__global__ __launch_bounds__(kThreads) void lic_eq_init(const EqState<T>* part, int32_t parts,
-                                                       EqState<T>* st, uint32_t* hist,
-                                                       int32_t nbins) {
+__device__ __forceinline__ EqState<T> image_range(EqState<T>* st, int32_t parts,
+                                                  EqState<T>* waves) {
   typedef typename KeyOf<T>::type Key;
-  for (int32_t b = blockIdx.x * kThreads + threadIdx.x; b < nbins; b += gridDim.x * kThreads)
-    hist[b] = 0u;
-  if (blockIdx.x != 0) return;
   Key lo = KeyOf<T>::kMax, hi = 0;
   unsigned long long cnt = 0;
-  for (int32_t k = threadIdx.x; k < parts; k += kThreads) {
-    lo = part[k].min_key < lo ? part[k].min_key : lo;
-    hi = part[k].max_key > hi ? part[k].max_key : hi;
-    cnt += part[k].count;
+  for (int32_t k = threadIdx.x; k < parts; k += blockDim.x) {
+    const EqState<T> part = st[1 + k];
+    lo = part.min_key < lo ? part.min_key : lo;
+    hi = part.max_key > hi ? part.max_key : hi;
+    cnt += part.count;
   }
-  reduce_range<T>(lo, hi, cnt);
-  if (threadIdx.x == 0) *st = EqState<T>{lo, hi, cnt};
+  const EqState<T> all = reduce_range<T>(lo, hi, cnt, waves);
+  if (blockIdx.x == 0 && threadIdx.x == 0) st[0] = all;
+  return all;
 }
 
-// Smallest and largest finite value and the count of finite pixels, per block.
+// Smallest and largest finite value and the count of finite pixels, per block,
+// and the counters to zero.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void lic_eq_range(const T* __restrict__ img, int64_t n,
                                                         int32_t nx, int64_t sy, int64_t sx,
-                                                        EqState<T>* part) {
+                                                        EqState<T>* part, uint32_t* hist,
+                                                        int32_t nbins) {
   typedef typename KeyOf<T>::type Key;
+  __shared__ EqState<T> waves[kThreads / 64];
+  for (int32_t b = blockIdx.x * kThreads + threadIdx.x; b < nbins; b += gridDim.x * kThreads)
+    hist[b] = 0u;
   Key lo = KeyOf<T>::kMax, hi = 0;
   unsigned long long cnt = 0;
   each_pixel(img, n, nx, sy, sx, [&](T x, int64_t) {
@@ -208,8 +208,8 @@ __global__ __launch_bounds__(kThreads) void lic_eq_range(const T* __restrict__ i
       ++cnt;
     }
   });
-  reduce_range<T>(lo, hi, cnt);
-  if (threadIdx.x == 0) part[blockIdx.x] = EqState<T>{lo, hi, cnt};
+  const EqState<T> all = reduce_range<T>(lo, hi, cnt, waves);
+  if (threadIdx.x == 0) part[blockIdx.x] = all;
 }
 
 // Histogram of the finite pixels' bins: LDS histograms of a block (nbins up to
@@ -220,11 +220,14 @@ __global__ __launch_bounds__(kThreads) void lic_eq_range(const T* __restrict__ i
 template <typename T, bool LDS>
 __global__ __launch_bounds__(kHistThreads) void lic_eq_hist(const T* __restrict__ img, int64_t n,
                                                        int32_t nx, int64_t sy, int64_t sx,
-                                                       int32_t nbins, const EqState<T>* st,
+                                                       int32_t nbins, EqState<T>* st,
+                                                       int32_t parts,
                                                        uint32_t* __restrict__ hist,
                                                        int32_t copies) {
-  extern __shared__ uint32_t local[];  // copies * nbins counters
-  const EqRange r = read_range(st, nbins);
+  // the waves' ranges, then copies * nbins counters
+  extern __shared__ __align__(16) uint32_t local[];
+  const EqRange r = read_range(image_range(st, parts, reinterpret_cast<EqState<T>*>(local)), nbins);
+  __syncthreads();
   uint32_t* mine = LDS ? local + ((threadIdx.x >> 6) & (copies - 1)) * nbins : hist;
   if (LDS) {
     for (int32_t b = threadIdx.x; b < copies * nbins; b += kHistThreads) local[b] = 0u;
@@ -282,7 +285,7 @@ __global__ __launch_bounds__(kThreads) void lic_eq_map(const T* __restrict__ img
                                                       const uint32_t* __restrict__ cdf,
                                                       T* __restrict__ out) {
   __shared__ T table[TABLE ? kTableBins : 1];
-  const EqRange r = read_range(st, nbins);
+  const EqRange r = read_range(*st, nbins);
   auto value = [&](int32_t b) {
     return static_cast<T>(static_cast<double>(cdf[b]) / static_cast<double>(r.count));
   };
@@ -310,9 +313,11 @@ __global__ __launch_bounds__(kThreads) void lic_eq_map(const T* __restrict__ img
 template <typename T>
 __global__ __launch_bounds__(kThreads) void lic_eq_bins(const T* __restrict__ img, int64_t n,
                                                        int32_t nx, int64_t sy, int64_t sx,
-                                                       int32_t nbins, const EqState<T>* st,
+                                                       int32_t nbins, EqState<T>* st,
+                                                       int32_t parts,
                                                        int32_t* __restrict__ bins) {
-  const EqRange r = read_range(st, nbins);
+  __shared__ EqState<T> waves[kThreads / 64];
+  const EqRange r = read_range(image_range(st, parts, waves), nbins);
   each_pixel(img, n, nx, sy, sx, [&](T x, int64_t p) {
     bins[p] = __builtin_isfinite(x) ? (r.constant ? 0 : eq_bin(static_cast<double>(x), r, nbins))
                                     : -1;
@@ -397,7 +402,7 @@ __global__ __launch_bounds__(kThreads) void lic_eq_tile_hist(
     const T* __restrict__ img, int32_t ny, int32_t nx, int64_t sy, int64_t sx, int32_t nbins,
     const EqState<T>* st, TileGrid tg, uint32_t* __restrict__ hist_all) {
   __shared__ uint32_t local[LDS ? kLdsBins : 1];
-  const EqRange r = read_range(st, nbins);
+  const EqRange r = read_range(*st, nbins);
   const int32_t t = blockIdx.x;
   const int32_t ty = t / tg.tiles_x, tx = t - ty * tg.tiles_x;
   uint32_t* hist = hist_all + static_cast<int64_t>(t) * nbins;
@@ -468,7 +473,7 @@ __global__ __launch_bounds__(kThreads) void lic_eq_tile_map(
     const T* __restrict__ img, int32_t ny, int32_t nx, int64_t sy, int64_t sx, int32_t nbins,
     const EqState<T>* st, const uint32_t* __restrict__ gcdf, const uint32_t* __restrict__ tcdf,
     TileGrid tg, T* __restrict__ out) {
-  const EqRange r = read_range(st, nbins);
+  const EqRange r = read_range(*st, nbins);
   const int64_t n = static_cast<int64_t>(ny) * nx;
   for (int64_t p = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; p < n;
        p += static_cast<int64_t>(gridDim.x) * kThreads) {
@@ -520,32 +525,35 @@ size_t equalize_scratch_bytes(int32_t nbins) {
   return counters_offset<T>() + sizeof(uint32_t) * static_cast<size_t>(nbins);
 }
 
-// The image's finite range into st[0], and its nbins counters cleared.
+// The image's partial ranges into st[1] on, and its nbins counters cleared; the
+// number of parts.
 template <typename T>
-static void launch_range(const T* img, int64_t n, int32_t nx, int64_t sy, int64_t sx,
-                         int32_t nbins, EqState<T>* st, uint32_t* hist, hipStream_t stream) {
-  const int g = std::min(grid_for(n, 8), kRangeBlocks);
+static int32_t launch_range(const T* img, int64_t n, int32_t nx, int64_t sy, int64_t sx,
+                            int32_t nbins, EqState<T>* st, uint32_t* hist, hipStream_t stream) {
+  // enough blocks to clear many counters of a small image
+  const int32_t clear = std::min((nbins + 4 * kThreads - 1) / (4 * kThreads), 256);
+  const int32_t g = std::min(std::max(grid_for(n, 8), clear), kRangeBlocks);
   hipLaunchKernelGGL(lic_eq_range<T>, dim3(g), dim3(kThreads), 0, stream, img, n, nx, sy, sx,
-                     st + 1);
-  const int blocks = std::min(1024, (nbins + kThreads - 1) / kThreads);
-  hipLaunchKernelGGL(lic_eq_init<T>, dim3(blocks < 1 ? 1 : blocks), dim3(kThreads), 0, stream,
-                     st + 1, g, st, hist, nbins);
+                     st + 1, hist, nbins);
+  return g;
 }
 
-// The global histogram of the image, into cleared counters.
+// The image's range into st[0], and its global histogram into cleared counters.
 template <typename T>
 static void launch_hist(const T* img, int64_t n, int32_t nx, int64_t sy, int64_t sx, int32_t nbins,
-                        const EqState<T>* st, uint32_t* hist, hipStream_t stream) {
+                        EqState<T>* st, int32_t parts, uint32_t* hist, hipStream_t stream) {
   const int gh = (grid_for(n, 8) + 3) / 4;  // two blocks of 16 waves per CU at most
+  const size_t waves = sizeof(EqState<T>) * (kHistThreads / 64);
   if (nbins <= kLdsBins) {
     const int32_t copies = nbins <= kTableBins ? 4 : 1;
     const size_t lds = sizeof(uint32_t) * static_cast<size_t>(copies) * nbins;  // at most 64 KB
     hipLaunchKernelGGL((lic_eq_hist<T, true>), dim3(gh), dim3(kHistThreads),
-                       static_cast<unsigned>(lds), stream, img, n, nx, sy, sx, nbins, st, hist,
-                       copies);
-  } else {
-    hipLaunchKernelGGL((lic_eq_hist<T, false>), dim3(gh), dim3(kHistThreads), 0, stream, img, n,
-                       nx, sy, sx, nbins, st, hist, 1);
+                       static_cast<unsigned>(std::max(lds, waves)), stream, img, n, nx, sy, sx,
+                       nbins, st, parts, hist, copies);
+  } else {  // nothing to merge: spread over the CUs (256^2: 18.7 us on 8, 8.5 on 32)
+    hipLaunchKernelGGL((lic_eq_hist<T, false>), dim3(grid_for(n, 2)), dim3(kHistThreads),
+                       static_cast<unsigned>(waves), stream, img, n, nx, sy, sx, nbins, st, parts,
+                       hist, 1);
   }
 }
 
@@ -555,9 +563,9 @@ hipError_t launch_equalize(const T* img, int64_t sy, int64_t sx, int32_t ny, int
   const int64_t n = static_cast<int64_t>(ny) * nx;
   auto* st = static_cast<EqState<T>*>(scratch);
   auto* hist = reinterpret_cast<uint32_t*>(static_cast<char*>(scratch) + counters_offset<T>());
-  launch_range<T>(img, n, nx, sy, sx, nbins, st, hist, stream);
+  const int32_t parts = launch_range<T>(img, n, nx, sy, sx, nbins, st, hist, stream);
   const int g = grid_for(n, 8);
-  launch_hist<T>(img, n, nx, sy, sx, nbins, st, hist, stream);
+  launch_hist<T>(img, n, nx, sy, sx, nbins, st, parts, hist, stream);
   hipLaunchKernelGGL(lic_eq_scan, dim3(1), dim3(kScanThreads), 0, stream, hist, nbins);
   if (nbins <= kTableBins) {
     hipLaunchKernelGGL((lic_eq_map<T, true>), dim3(g), dim3(kThreads), 0, stream, img, n, nx, sy,
@@ -591,7 +599,7 @@ hipError_t launch_equalize_tiles(int method, const T* img, int64_t sy, int64_t s
   auto* hist = reinterpret_cast<uint32_t*>(static_cast<char*>(scratch) + counters_offset<T>());
   char* extra = static_cast<char*>(scratch) +
                 ((equalize_scratch_bytes<T>(nbins) + 255) & ~size_t{255});
-  launch_range<T>(img, n, nx, sy, sx, nbins, st, hist, stream);
+  const int32_t parts = launch_range<T>(img, n, nx, sy, sx, nbins, st, hist, stream);
   const int g = grid_for(n, 8);
   if (method == kEqSlidingTile) {
     // a window taller than 2 ny - 1 rows covers the image from every pixel,
@@ -600,7 +608,7 @@ hipError_t launch_equalize_tiles(int method, const T* img, int64_t sy, int64_t s
     tw = static_cast<int32_t>(std::min<int64_t>(tw, 2 * int64_t{nx} - 1));
     auto* bins = reinterpret_cast<int32_t*>(extra);
     hipLaunchKernelGGL(lic_eq_bins<T>, dim3(g), dim3(kThreads), 0, stream, img, n, nx, sy, sx,
-                       nbins, st, bins);
+                       nbins, st, parts, bins);
     const dim3 grid(static_cast<unsigned>((nx + kSlide - 1) / kSlide),
                     static_cast<unsigned>((ny + kSlide - 1) / kSlide));
     const int64_t box = (int64_t{kSlide} + th - 1) * (int64_t{kSlide} + tw - 1) *
@@ -624,7 +632,7 @@ hipError_t launch_equalize_tiles(int method, const T* img, int64_t sy, int64_t s
                     tiles_along(nx, std::min(tw, nx))};
   const int32_t tiles = tg.tiles_y * tg.tiles_x;
   auto* tcdf = reinterpret_cast<uint32_t*>(extra);
-  launch_hist<T>(img, n, nx, sy, sx, nbins, st, hist, stream);
+  launch_hist<T>(img, n, nx, sy, sx, nbins, st, parts, hist, stream);
   if (nbins <= kLdsBins) {
     hipLaunchKernelGGL((lic_eq_tile_hist<T, true>), dim3(tiles), dim3(kThreads), 0, stream, img,
                        ny, nx, sy, sx, nbins, st, tg, tcdf);
