@@ -255,6 +255,13 @@ static const void* persistent_fn(int profile, bool buf) {
 }
 
 // Blocks of a persistent grid that fill the device: CUs x resident blocks per CU.
+// At most kBlocksPerCu of them: the float kernel's registers would leave room
+// for a seventh, and its waves then only share the issue slots and the L1 that
+// six already fill. 64 float fields of sides 300..500, 3 passes: 3.34 ms with
+// seven, 3.11 with six; 8 such fields, 5 passes: 0.95 and 0.88; 200 of sides
+// 200..400, 2 passes: 5.32 and 5.15; many uneven or tiny fields alike (0 to 3%).
+constexpr int kBlocksPerCu = 6;
+
 static int persistent_grid(const void* fn) {
   int dev = 0, cus = 0, per_cu = 0;
   if (hipGetDevice(&dev) != hipSuccess) return 1024;
@@ -265,7 +272,7 @@ static int persistent_grid(const void* fn) {
     (void)hipGetLastError();
     per_cu = 4;
   }
-  return cus * per_cu;
+  return cus * std::min(per_cu, kBlocksPerCu);
 }
 
 static size_t align_up(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
