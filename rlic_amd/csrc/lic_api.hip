@@ -675,13 +675,8 @@ int run_on_device(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
       code_ptr,
       bounds ? reinterpret_cast<rlic::ReplayBounds*>(base + off_codes + code_bytes) : nullptr,
       false};
-  const uint32_t epoch = rlic::next_epoch();
-  if (fixed) {  // the calls made for capture
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
-    if (capture != hipStreamCaptureStatusNone)
-      RLIC_HIP_TRY(rlic::launch_clear_mark<T>(c, stream), "clearing the field's mark");
-  }
+  // the calls made for capture count the epoch on the device
+  const uint32_t epoch = fixed ? rlic::captured_epoch() : rlic::next_epoch();
   if (check) check->recorded = true;  // also if a launch fails: the caller waits for the stream
   {
     // the cells and the padded weight copy in one launch

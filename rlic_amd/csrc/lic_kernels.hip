@@ -96,7 +96,9 @@ template <typename T, bool FMA, bool BRANCHLESS, bool POL, bool REC, bool BUF>
 __global__ __launch_bounds__(256) void lic_trace(const Cell<T>* __restrict__ cells,
                                                  const T* __restrict__ kernel, int32_t klen,
                                                  FieldGeom g, TileMap m, T* __restrict__ out,
-                                                 uint4* __restrict__ codes, uint32_t epoch) {
+                                                 uint4* __restrict__ codes, uint32_t epoch,
+                                                 uint32_t* corner) {
+  count_epoch(corner);
   int32_t ty, tx, py, px;
   tile_of_block(blockIdx.x, m, ty, tx);
   if constexpr (BUF) pixel_of_quads(threadIdx.x, m, py, px);
@@ -151,8 +153,10 @@ __global__ __launch_bounds__(256) void lic_trace(const Cell<T>* __restrict__ cel
 template <typename T, bool FMA, bool BRANCHLESS, bool POL, bool REC>
 __global__ __launch_bounds__(64) void lic_trace_pair(
     const Cell<T>* __restrict__ cells, const T* __restrict__ kernel, int32_t klen, FieldGeom g,
-    TileMap m, T* __restrict__ out, uint4* __restrict__ codes, uint32_t epoch) {
+    TileMap m, T* __restrict__ out, uint4* __restrict__ codes, uint32_t epoch,
+    uint32_t* corner) {
   extern __shared__ __align__(16) unsigned char smem[];
+  count_epoch(corner);
   const int32_t lane = threadIdx.x;
   const bool fwd = lane < 32;
   const int32_t k = lane & 31;
@@ -696,17 +700,17 @@ uint32_t next_epoch() {
   static std::atomic<uint32_t> epoch{0};
   for (;;) {
     const uint32_t e = epoch.fetch_add(1, std::memory_order_relaxed) + 1;
-    if (e != 0) return e;
+    if (e != kCountedEpoch) return e;
   }
 }
 
-__global__ void lic_clear_mark(uint32_t* mark) { *mark = 0u; }
+uint32_t captured_epoch() { return kCountedEpoch; }
 
+// The corner cell that a trace counts its epoch in (count_epoch).
 template <typename T>
-hipError_t launch_clear_mark(Cell<T>* cells, hipStream_t stream) {
-  hipLaunchKernelGGL(lic_clear_mark, dim3(1), dim3(1), 0, stream,
-                     reinterpret_cast<uint32_t*>(cells));
-  return hipGetLastError();
+static uint32_t* counted_corner(const Cell<T>* cells, uint32_t epoch) {
+  if (epoch != kCountedEpoch) return nullptr;
+  return reinterpret_cast<uint32_t*>(const_cast<Cell<T>*>(cells));
 }
 
 template <typename T>
@@ -733,10 +737,12 @@ static hipError_t trace_one(const Cell<T>* cells, const T* kernel, int32_t klen,
                             hipStream_t stream) {
   if (fits_buffer(cell_slots(g) * static_cast<int64_t>(sizeof(Cell<T>)))) {
     hipLaunchKernelGGL((lic_trace<T, FMA, BL, POL, REC, true>), dim3(m.n_tiles), dim3(kBlock),
-                       0, stream, cells, kernel, klen, g, m, out, codes, epoch);
+                       0, stream, cells, kernel, klen, g, m, out, codes, epoch,
+                       counted_corner(cells, epoch));
   } else {
     hipLaunchKernelGGL((lic_trace<T, FMA, BL, POL, REC, false>), dim3(m.n_tiles), dim3(kBlock),
-                       0, stream, cells, kernel, klen, g, m, out, codes, epoch);
+                       0, stream, cells, kernel, klen, g, m, out, codes, epoch,
+                       counted_corner(cells, epoch));
   }
   return hipGetLastError();
 }
@@ -785,7 +791,7 @@ static hipError_t trace_pair_one(const Cell<T>* cells, const T* kernel, int32_t 
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
   hipLaunchKernelGGL(fn, dim3(m.n_tiles * 8), dim3(64), lds, stream, cells, kernel, klen, g, m,
-                     out, codes, epoch);
+                     out, codes, epoch, counted_corner(cells, epoch));
   return hipGetLastError();
 }
 
@@ -1040,7 +1046,6 @@ hipError_t launch_replay_lds_hybrid(const T* x, const T* kernel, int32_t klen, c
   template hipError_t launch_pack<T>(const T*, int64_t, int64_t, const T*, int64_t, int64_t,   \
                                      const T*, int64_t, int64_t, const FieldGeom&, Cell<T>*,   \
                                      uint32_t, hipStream_t, const T*, int32_t, T*, uint32_t*);  \
-  template hipError_t launch_clear_mark<T>(Cell<T>*, hipStream_t);                             \
   template hipError_t launch_repack_texture<T>(const T*, const FieldGeom&, Cell<T>*,           \
                                                hipStream_t);                                    \
   template hipError_t launch_copy2d<T>(const T*, int64_t, int64_t, int32_t, int32_t, T*,       \

@@ -36,14 +36,11 @@ hipError_t launch_pack(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64
                        const T* kernel = nullptr, int32_t klen = 0, T* kpad = nullptr,
                        uint32_t* flags = nullptr);
 
-// A value for one packing of a field's cells (wide_mark), never 0: the packing
-// and the traces of its cells are given the same.
+// A value for one packing of a field's cells (wide_mark): the packing and the
+// traces of its cells are given the same.  captured_epoch, for launches that are
+// recorded into a graph, stands for another value at every replay.
 uint32_t next_epoch();
-
-// Takes the mark of a wide field off, before a packing that is recorded into a
-// graph: its epoch is the same at every replay.
-template <typename T>
-hipError_t launch_clear_mark(Cell<T>* cells, hipStream_t stream);
+uint32_t captured_epoch();
 
 // Zeros on each side of the padded kernel-weight copy the streamline
 // kernels read (they load taps in groups of 8 without bounds checks).
