@@ -422,7 +422,8 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
   const int32_t nchunks = chunks_of(nsteps);
   // Short path: whole groups of a chunk by fast_group; when a moving lane is
   // reported, the chunk is done again by the full rule (one saved state per
-  // chunk: saving it for every group cost 2 VALU instructions per step).  What
+  // chunk: saving it for every group cost 2 VALU instructions per step; the
+  // paired trace in float is apart, below).  What
   // is thrown away costs a group at least, so the path is left for the rest of
   // the line and for its other direction where more reports are likely: after
   // one of many lanes, one in a chunk's first two groups, or a second one; in
@@ -446,6 +447,83 @@ __device__ __forceinline__ T trace_direction(T acc, T pu, T pv, uint32_t row,
   int32_t misses = 0;
   bool live_now = false, moves_now = false;  // set before a chunk of the short path
   bool status_known = false;
+  if constexpr (LANE_DIR && sizeof(T) == 4) {
+    // So few waves that the longest one sets the launch's time, and in float one
+    // of them nearly always has a report: so only the reported group is done
+    // again.  A launch before the short path existed, with whole chunks done
+    // again (and 8 times the reports: near_tie), now: 256^2 L = 65 17.9, 22.3,
+    // 16.7 us, L = 33 11.9, 13.8, 12.0, 362^2 L = 65 23.9, 25.5, 20.4; without
+    // any report 64^2 L = 65 13.6, 11.1, 11.6.  In double, where reports are
+    // rare, whole chunks are 1 to 3% faster.
+    StepGeom sm = sl;
+    uint64_t m_moves = 0;
+    bool all_move = false;
+    for (int32_t ch = 0; ch < nchunks; ++ch) {
+      uint32_t words[4] = {kWordStay, kWordStay, kWordStay, kWordStay};
+      bool any_alive = true;
+#pragma unroll 1
+      for (int g = 0; g < 4; ++g) {
+        const int32_t s0 = ch * kChunkSteps + 8 * g;
+        if (s0 >= nsteps || !any_alive) break;  // uniform
+        uint32_t word = 0;
+        if (NARROW && fast && s0 + 8 <= nsteps && !status_known) {  // uniform
+          live_now = !__builtin_isunordered(pu, pv);
+          moves_now = live_now && (pu != T(0) || pv != T(0));
+          sm = {moves_now ? sl.step_x : 0u, moves_now ? sl.near_y : 0u,
+                moves_now ? sl.far_y : 0u, sl.all_far};
+          m_moves = __builtin_amdgcn_ballot_w64(moves_now);
+          all_move = m_moves == __builtin_amdgcn_ballot_w64(true);
+          status_known = __builtin_amdgcn_ballot_w64(
+                             moves_now && !(fraction_usable(fx) && fraction_usable(fy))) == 0;
+        }
+        if (NARROW && fast && s0 + 8 <= nsteps && status_known) {  // uniform
+          const uint32_t row_0 = row;
+          saved.put(acc, fx, fy, last_u, last_v);
+          T kw[8];
+#pragma unroll
+          for (int q = 0; q < 8; ++q)
+            kw[q] = kernel[FORWARD ? kmid + 1 + s0 + q : kmid - 1 - s0 - q];
+          const uint64_t reported =
+              fast_group<T, FMA, POL, FORWARD, REC, BUF, PAIRS, LANE_DIR>(
+                  acc, fx, fy, pu, pv, last_u, last_v, row, word, kw, cell, sm, lane_sign, s0,
+                  sink) &
+              m_moves;
+          if (reported == 0) {  // uniform
+            if (all_move) {  // uniform
+              if (live_steps) *live_steps = s0 + 8;
+            } else {
+              if (!live_now) acc = saved.acc();
+              const uint32_t still = live_now ? kWordStay : 0x11111111u * kMoveStop;
+              word = moves_now ? word : still;
+              if (live_steps) *live_steps = live_now ? s0 + 8 : *live_steps;
+              any_alive = __builtin_amdgcn_ballot_w64(live_now) != 0;
+            }
+            words[g] = word;
+            continue;
+          }
+          fast = ++misses < 3 && __popcll(reported) < 8;
+          saved.get(acc, fx, fy, last_u, last_v);
+          row = row_0;
+          const CellVal<T> cv = cell(row);
+          pu = cv.u;
+          pv = cv.v;
+          word = 0;
+        }
+        status_known = false;
+        uint64_t m_live = 0;
+        full_group<T, FMA, BRANCHLESS, POL, FORWARD, REC, BUF, PAIRS, LANE_DIR,
+                   NARROW && sizeof(T) == 4>(
+            acc, fx, fy, pu, pv, last_u, last_v, row, m_live, word,
+            kernel + (FORWARD ? kmid + 1 + s0 : kmid - 1 - s0), cell, sl, lane_sign, s0,
+            min(8, nsteps - s0), sink, live_steps);
+        words[g] = word;
+        any_alive = m_live != 0;
+      }
+      if (rec) codes[(c0 + ch) * np + p] = make_uint4(words[0], words[1], words[2], words[3]);
+      if (!any_alive) break;
+    }
+    return acc;
+  }
   for (int32_t ch = 0; ch < nchunks; ++ch) {
     uint32_t words[4] = {kWordStay, kWordStay, kWordStay, kWordStay};
     bool any_alive = true;
