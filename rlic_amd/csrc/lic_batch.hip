@@ -104,7 +104,7 @@ __device__ __forceinline__ void batch_trace_pixel(const BatchField<T>& f,
         acc, c0.u, c0.v, row0, cell, kernel, kmid, n_bwd, sg, f.codes, np, p, chunks_of(n_fwd),
         short_path, saved);
   };
-  const bool wide = !BRANCHLESS || wide_mark(f.cells, f.epoch);  // uniform
+  const bool wide = !BRANCHLESS || kmid < 8 || wide_mark(f.cells, f.epoch);  // uniform
   if (wide) line(std::false_type{});
   else line(std::bool_constant<BRANCHLESS>{});
   dst[p] = acc;
