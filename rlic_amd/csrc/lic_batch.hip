@@ -78,7 +78,7 @@ __global__ __launch_bounds__(256) void lic_pack_batch(const BatchField<T>* field
   store_guarded_cell(
       f.cells, gi, gj, f.g,
       guarded_cell(f.tex, f.tsy, f.tsx, f.u, f.usy, f.usx, f.v, f.vsy, f.vsx, f.g, gi, gj),
-      f.epoch);
+      f.epoch, f.klen);
 }
 
 template <typename T, bool FMA, bool BRANCHLESS, int POL, int REC, bool BUF>
@@ -104,7 +104,7 @@ __device__ __forceinline__ void batch_trace_pixel(const BatchField<T>& f,
         acc, c0.u, c0.v, row0, cell, kernel, kmid, n_bwd, sg, f.codes, np, p, chunks_of(n_fwd),
         short_path, saved);
   };
-  const bool wide = !BRANCHLESS || kmid < 8 || wide_mark(f.cells, f.epoch);  // uniform
+  const bool wide = !BRANCHLESS || wide_mark(f.cells, f.epoch);  // uniform
   if (wide) line(std::false_type{});
   else line(std::bool_constant<BRANCHLESS>{});
   dst[p] = acc;

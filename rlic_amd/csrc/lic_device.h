@@ -525,15 +525,28 @@ __device__ __forceinline__ void pack_cell_of_thread(int32_t tid, int32_t& di, in
   dj = (tid >> 1) & 63;
 }
 
-// Stores guarded cell (gi, gj) and marks a wide field (wide_mark); corner
-// (0, 0) itself, the mark's place, is not written but for a counted epoch.
+// Kernels below this have no whole group of 8 steps in either direction and so
+// no use for the short path, whose preparation takes a third of so short a trace:
+// their fields are marked too.  2048^2 float, L = 3 and 9, us a launch before the
+// short path existed, with it, marked: 33, 47, 36 and 54, 65, 59 (L = 17: 86,
+// 73); double 38, 58, 43 and 75, 94, 84.  (A test of the length in the trace cost
+// a 4096^2 one of L = 129 2.5%.)
+constexpr int32_t kShortPathMinLen = 16;
+
+// Stores guarded cell (gi, gj); marks a wide field (wide_mark) and one traced
+// with fewer than kShortPathMinLen weights in corner (0, 0), its place.
 template <typename T>
 __device__ __forceinline__ void store_guarded_cell(Cell<T>* __restrict__ cells, int32_t gi,
                                                    int32_t gj, const FieldGeom& g,
-                                                   const Cell<T>& c, uint32_t epoch) {
+                                                   const Cell<T>& c, uint32_t epoch,
+                                                   int32_t klen) {
   uint32_t* corner = reinterpret_cast<uint32_t*>(cells);
-  if (gi != 0 || gj != 0) cells[cell_slot(g, gi, gj)] = c;
-  else if (epoch == kCountedEpoch) corner[2] = packing_epoch(corner, epoch);
+  if (gi != 0 || gj != 0) {
+    cells[cell_slot(g, gi, gj)] = c;
+  } else {
+    if (epoch == kCountedEpoch) corner[2] = packing_epoch(corner, epoch);
+    if (klen < kShortPathMinLen) corner[0] = packing_epoch(corner, epoch);
+  }
   if (velocity_wide(c.u) || velocity_wide(c.v)) corner[0] = packing_epoch(corner, epoch);
 }
 

@@ -60,7 +60,7 @@ __global__ __launch_bounds__(256) void lic_pack(const T* __restrict__ tex, int64
   gj += blockIdx.x * 64;
   if (gi >= g.ny + 2 || gj >= g.nx + 2) return;
   const Cell<T> c = guarded_cell(tex, tsy, tsx, u, usy, usx, v, vsy, vsx, g, gi, gj);
-  store_guarded_cell(cells, gi, gj, g, c, epoch);
+  store_guarded_cell(cells, gi, gj, g, c, epoch, klen);
   if (flags && c.x < T(0)) flags[0] = 1u;  // a guard cell holds an image cell's value
 }
 
@@ -130,11 +130,7 @@ __global__ __launch_bounds__(256) void lic_trace(const Cell<T>* __restrict__ cel
         acc, c0.u, c0.v, row0, cell, kernel, kmid, n_bwd, sg, codes, np, p,
         chunks_of(n_fwd), short_path, saved);
   };
-  // A kernel without a whole group of 8 steps has no use for the short path,
-  // whose preparation takes a third of so short a trace: 2048^2 float, L = 3, 9,
-  // us before the short path existed, with it, with this rule: 33, 47, 36 and 54,
-  // 65, 59 (L = 17, with its whole group: 86, 73); double 38, 58, 43 and 75, 94, 84.
-  const bool wide = !BRANCHLESS || kmid < 8 || wide_mark(cells, epoch);  // uniform
+  const bool wide = !BRANCHLESS || wide_mark(cells, epoch);  // uniform
   if (wide) line(std::false_type{});
   else line(std::bool_constant<BRANCHLESS>{});
   out[static_cast<int64_t>(i0) * g.nx + j0] = acc;
@@ -196,7 +192,7 @@ __global__ __launch_bounds__(64) void lic_trace_pair(
           acc, c0.u, c0.v, row0, cell, kernel, kmid, kmid, sg, codes, np, p,
           fwd ? 0 : chunks_of(kmid), short_path, saved, fwd, keep, &live_steps);
     };
-    const bool wide = !BRANCHLESS || kmid < 8 || wide_mark(cells, epoch);  // uniform
+    const bool wide = !BRANCHLESS || wide_mark(cells, epoch);  // uniform
     if (wide) line(std::false_type{});
     else line(std::bool_constant<BRANCHLESS>{});
   }

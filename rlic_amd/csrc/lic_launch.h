@@ -26,14 +26,15 @@ void choose_row_order(FieldGeom& g);
 // The field's guarded cell array (cell_slots(g) cells) from its strided
 // texture, u and v; with `kpad`, in the same launch, the padded
 // weight copy of `kernel`: kpad (klen + 2 * kernel_pad() elements) =
-// [zeros][kernel][zeros].
+// [zeros][kernel][zeros].  klen, the weights that the cells will be traced with,
+// also without kpad: it decides about the trace's loop (kShortPathMinLen).
 // flags (2 words, not null only with kpad): set to 1 where a texture element
 // is below 0, a weight not finite.
 template <typename T>
 hipError_t launch_pack(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t usy,
                        int64_t usx, const T* v, int64_t vsy, int64_t vsx, const FieldGeom& g,
                        Cell<T>* cells, uint32_t epoch, hipStream_t stream,
-                       const T* kernel = nullptr, int32_t klen = 0, T* kpad = nullptr,
+                       const T* kernel, int32_t klen, T* kpad = nullptr,
                        uint32_t* flags = nullptr);
 
 // A value for one packing of a field's cells (wide_mark): the packing and the

@@ -156,7 +156,7 @@ int Server::admit(const T* tex, int64_t tsy, int64_t tsx, const T* u, int64_t us
                        hipMemcpyDefault, stream_);
   if (e == hipSuccess && n > 0)
     e = launch_pack<T>(tex, tsy, tsx, u, usy, usx, v, vsy, vsx, r.g, r.cells, r.epoch,
-                       stream_);
+                       stream_, nullptr, klen);
   if (e != hipSuccess) {
     (void)hipFreeAsync(r.block, stream_);  // not cached: the failed copy may have left it in use
     err = std::string("admitting field: ") + hipGetErrorString(e);
