@@ -243,21 +243,24 @@ int32_t hybrid_halo(int32_t klen, int64_t n) {
 
 // Boxes cut to the lines (launch_replay_box), for a call that replays
 // `replays` passes.  A pass takes less, but the first also finds the boxes.
-// First and later passes, us, against the plans below:
-//   f32  4096^2     L=65   486, 236 vs 346, 264    L=97   676, 297 vs 572, 373
-//                   L=129  774, 342 vs 646, 470    L=151 1032, 438 vs 1187, 817
-//                   L=201 1468, 700 vs 2180, 1616  L=401 4871, 3107 vs 6083, 4840
-//        2048^2     L=65   124, 62 vs 89, 69       L=113  220, 88 vs 173, 109
-//                   L=145  297, 126 vs 254, 161    L=151  347, 129 vs 312, 211
-//        1400x1300  L=97   77, 40 vs 64, 52        L=145  109, 56 vs 99, 79
-//        1024^2     L=129  56, 31 vs 45, 36        L=201  124, 65 vs 129, 103
-//        520x600    L=65   22, 11 vs 22, 19        L=145  42, 19 vs 49, 40
-//   f64  2048^2     L=49   161, 64 vs 107, 60      L=67   253, 91 vs 209, 117
-//                   L=97   281, 111 vs 253, 169    L=151  478, 234 vs 572, 434
-//        1400x1300  L=67   95, 48 vs 79, 59        L=113  131, 69 vs 135, 116
-//        520x600    L=67   32, 18 vs 36, 31        L=129  52, 37 vs 77, 70
+// First and later passes against the plans below, us a launch (events around
+// each; what the trace takes to write the record is the same for both):
+//   f32  4096^2     L=65   368, 245 vs 290, 265    L=97   516, 318 vs 385, 383
+//                   L=129  579, 360 vs 484, 486    L=151  754, 460 vs 863, 816
+//                   L=201 1062, 684 vs 1680, 1596  L=401 3355, 2714 vs 4913, 4765
+//        2048^2     L=65    92, 64 vs 74, 72       L=113  143, 88 vs 115, 114
+//                   L=145  203, 122 vs 171, 163    L=151  206, 134 vs 218, 218
+//        1400x1300  L=97    63, 42 vs 55, 55       L=145   86, 56 vs 82, 82
+//        1024^2     L=129   44, 30 vs 36, 36       L=201   88, 61 vs 107, 107
+//        520x600    L=65    16, 14 vs 21, 21       L=145   28, 21 vs 41, 42
+//   f64  2048^2     L=49    98, 67 vs 65, 63       L=67   148, 94 vs 124, 122
+//                   L=97   179, 111 vs 178, 177    L=151  303, 218 vs 426, 427
+//        1400x1300  L=67    72, 50 vs 62, 62       L=113  105, 65 vs 124, 117
+//        520x600    L=67    28, 20 vs 33, 33       L=129   45, 33 vs 73, 73
 // so the fewer passes there are to pay for the first, the longer the kernel
-// must be.  RLIC_REPLAY_BOX = 0: never, 2: wherever they fit (tests).
+// must be.  The two are even after, at worst over the sizes: float 4.9 replays
+// at L = 65, 3.0 at 97, 1.8 at 145, 0.9 at 151; double 1.9 at 67, 1.0 at 97, 0.7
+// at 113: the lines below lie on the safe side of these.  RLIC_REPLAY_BOX = 0: never, 2: wherever they fit (tests).
 template <typename T>
 bool box_allowed(int32_t klen, const rlic::FieldGeom& g, int64_t replays) {
   const int box = env_int("RLIC_REPLAY_BOX", 1);

@@ -19,18 +19,19 @@
 // 151), the box of as many waves as fit is staged and the others gather from
 // the image beside them: a wave's 64 lines part far less than the tile's.
 // Against a tile gathering from the image as a whole: 4096^2 L = 201 969 ->
-// 700 us, L = 401 4610 -> 3107; 2048^2 double L = 151 323 -> 234.
+// 684 us, L = 401 4610 -> 2714; 2048^2 double L = 151 323 -> 218.
 //
-// What bounds it: at 4096^2, L = 129, 342 us a later pass (whole boxes in
-// lic_replay_lds: 470), of which reading the record alone takes 228 (64 bytes
+// What bounds it: at 4096^2, L = 129, 360 us a later pass (whole boxes in
+// lic_replay_lds: 486), of which reading the record alone takes 228 (64 bytes
 // a pixel); VALU and scalar issue are each about 60% busy, LDS 45%.  The first
-// pass takes 280 us more, the moves' dot products and a second chain of loads.
-// Tried: two lines per lane in three blocks of 50 KB (528 us; fewer boxes
-// fit), bounds per chunk of 32 steps with runs of chunks that fit (registers
-// spilled), bounds kept by the tracing pass (12% longer there), up to four
-// boxes one after the other for the waves left (L = 257 1076 -> 897 us, but
-// 32 spilled registers: L = 129 342 -> 392), the first pass's record held in
-// registers (no faster: the second read comes from the caches).
+// pass takes 220 us more, the moves' dot products and a second chain of loads.
+// Tried (against the 342 us a later pass took in those runs): two lines per
+// lane in three blocks of 50 KB (528 us; fewer boxes fit), bounds per chunk of
+// 32 steps with runs of chunks that fit (registers spilled), bounds kept by the
+// tracing pass (12% longer there), up to four boxes one after the other for the
+// waves left (L = 257 1076 -> 897 us, but 32 spilled registers: L = 129 342 ->
+// 392), the first pass's record held in registers (no faster: the second read
+// comes from the caches).
 #include <algorithm>
 #include <type_traits>
 

@@ -76,9 +76,9 @@ __device__ __forceinline__ bool jump_stays(uint32_t jump, const StepGeom& sg) {
 // the field lies within VelocityRange (velocity_wide), so the products
 // neither overflow nor lose bits to underflow.  With |e| > near_tie n_y |u|
 // the two exact quotients differ by more than near_tie / 2 relatively, so
-// their roundings compare as the exact ones do; otherwise (an exact or a near tie, both components zero, a NaN component:
-// every one of them fails the comparison) the lane is reported.  The
-// quotient is quotient_rn's, which needs a numerator that is zero or not tiny
+// their roundings compare as the exact ones do; otherwise (an exact or a near
+// tie, both components zero, a NaN component: every one of them fails the
+// comparison) the lane is reported.  The quotient is quotient_rn's, which needs a numerator that is zero or not tiny
 // (numerator_key_min): smaller ones are reported too.  A time of zero (n = 0)
 // compares below the other one only if that does not underflow to zero: in
 // float, lanes with |e| below kProductMin are reported (0.7% of a trace); in
@@ -100,14 +100,19 @@ __device__ __forceinline__ bool jump_stays(uint32_t jump, const StepGeom& sg) {
 // 16 for v_rcp_f64 (measured with streams of one instruction).  So choices are
 // made with lane masks in VGPRs (sign words and v_bitop3) rather than with
 // compares and v_cndmask.  A step is about 36 VALU instructions, 90 issue
-// cycles per wave (the full rule's 57 took about 170); with that the L1 gather
-// path is as busy (TD 97%, 29-34 cycles per wave gather on the CU's one
-// path).  Trace launches, full rule in plain rows -> with this alone -> and
+// cycles per wave (the full rule's 57 took about 170).  The texture data unit's
+// busy counter reads 94 to 97% beside it, but it does so in every variant, at
+// 48 and at 63 cycles a gather of equal accesses, so it counts waiting and shows
+// no bound.  Trace launches, full rule in plain rows -> with this alone -> and
 // row pairs (cell_slot): 4096^2 float L=129 with the record 2.47 -> 1.92 ->
 // 1.86 ms, 2111x1500 float with holes L=201 775 -> 684 -> 603 us, 1021x1537
 // double L=151 499 -> 447 -> 430 us, 16384^2 float polarization L=257 (plain
 // rows) 72.2 -> 55.0 -> 54.5 ms, 8192^2 double polarization 30.1 -> 26.4 ->
-// 26.4 ms, 256^2 double L=65 (paired lanes) 22.6 -> 19.3 -> 19.9 us.
+// 26.4 ms, 256^2 double L=65 (paired lanes) 22.6 -> 19.3 -> 19.9 us.  With the
+// full rule as it is now beside it, the first and the last of these in one run:
+// 2.50 and 1.87 ms, 789 and 627 us, 501 and 418 us; paired 21.5 and 19.2 us.  Row
+// pairs alone cost the paired lanes 3% and are kept there because a field has
+// one layout for every kernel.
 template <typename T, bool FMA, int POL, bool FORWARD, int REC, bool BUF, bool PAIRS,
           bool LANE_DIR, typename Sink>
 __device__ __forceinline__ uint64_t fast_group(
